@@ -12,9 +12,13 @@
 //   list2(P)   children of colleagues of parent(P) that are not colleagues of P
 //   list3(B)   first sep3 boxes below colleagues of B
 //   list4(P)   source leaves S bigger than P: sep(S,P) and !sep(S,parent(P))
-// Lists are sorted by box number.  Each list is built by one thread: a count
-// pass, an exclusive scan, a fill pass and an in-place insertion sort.
+// Lists are sorted by box number.  Each box's lists are built by one
+// wavefront: a count pass, an exclusive scan, a fill pass, and a sort by a
+// block per list.
 #include "qbx_internal.h"
+
+#include <algorithm>
+#include <climits>
 
 namespace qbx {
 
@@ -91,143 +95,229 @@ struct ListOut {
     int fill;          // 0 count, 1 fill
 };
 
-__device__ inline void emit(ListOut &o, int item, int &k, int v)
+// appends v of the lanes with `want` to the item's list (k: the entries so
+// far, the same in every lane)
+__device__ inline void emit(const ListOut &o, int item, int &k, bool want, int v)
 {
-    if (o.fill) o.lists[o.starts[item] + k] = v;
-    ++k;
+    const unsigned long long m = __ballot(want);
+    if (want && o.fill)
+        o.lists[o.starts[item] + k + __popcll(m & ((1ULL << (threadIdx.x & 63)) - 1))] = v;
+    k += __popcll(m);
 }
 
-constexpr int STACK = 192;
-
-__global__ void k_list13(TV t, int n, int e, int minsrc, int ntb, const int *target_boxes,
-                         ListOut o1, ListOut o3, int *err)
+// ancestors of b, b first; every lane returns their number
+__device__ inline int tv_ancestors(const TV &t, int b, int *anc)
 {
-    int it = blockIdx.x * blockDim.x + threadIdx.x;
-    if (it >= ntb) return;
-    int B = target_boxes[it];
+    int na = 0;
+    for (int a = b; a >= 0 && na < MAX_LEVELS; a = t.parent[a]) {
+        if (threadIdx.x == 0) anc[na] = a;
+        ++na;
+    }
+    __syncthreads();
+    return na;
+}
+
+// Lists 1 and 3, one wavefront per target box.  The searches under the box's
+// colleagues run over a stack in LDS, 64 boxes a round: a coarse target box
+// (centers with extent stop there) walks most of the tree, which as one
+// thread per box took 40 ms a launch of serial steps on a surface of 737280
+// sources (now 0.31 ms, every box's walk spread over 64 lanes).  Bit 31 of a
+// stack entry marks the boxes below a sep3 box of too few sources, whose
+// leaves all go to list 1.
+//
+// The stack holds nlevels * 64 * 2^dim entries: a round pops the top 64 and
+// pushes the children of the top one last, so depths never fall towards the
+// top, and boxes of a depth are pushed only when no box of that depth is left.
+__global__ void __launch_bounds__(64) k_list13(TV t, int n, int e, int minsrc, int ntb,
+                                               const int *target_boxes, ListOut o1, ListOut o3)
+{
+    extern __shared__ int stack[];
+    __shared__ int anc[MAX_LEVELS];
+    constexpr unsigned SUB = 0x80000000u;
+    const int lane = threadIdx.x, nchild = 1 << t.dim;
+    const int it = blockIdx.x;
+    const int B = target_boxes[it];
     int k1 = 0, k3 = 0;
     int ncol = 1;
     for (int d = 0; d < t.dim; ++d) ncol *= (2 * n + 1);
     // (a) leaves not smaller than B: colleagues of each ancestor-or-self
-    int anc[MAX_LEVELS];
-    int na = 0;
-    for (int a = B; a >= 0 && na < MAX_LEVELS; a = t.parent[a]) anc[na++] = a;
-    for (int j = na - 1; j >= 0; --j) {
-        for (int kc = 0; kc < ncol; ++kc) {
-            int C = tv_colleague(t, anc[j], n, kc);
-            if (C < 0 || !tv_leaf(t, C) || t.src_nonchild[C] == 0) continue;
-            if (tv_gap(t, C, B, 0) < n) emit(o1, it, k1, C);
+    const int na = tv_ancestors(t, B, anc);
+    for (int i0 = 0; i0 < na * ncol; i0 += 64) {
+        const int i = i0 + lane;
+        int C = -1;
+        if (i < na * ncol) {
+            C = tv_colleague(t, anc[i / ncol], n, i % ncol);
+            if (C >= 0 && !(t.src_nonchild[C] > 0 && tv_leaf(t, C) && tv_gap(t, C, B, 0) < n))
+                C = -1;
         }
+        emit(o1, it, k1, C >= 0, C);
     }
     // (b) below same-level colleagues
-    int stack[STACK];
-    for (int kc = 0; kc < ncol; ++kc) {
-        int C = tv_colleague(t, B, n, kc);
-        if (C < 0 || tv_leaf(t, C)) continue;
+    for (int kc = 0; kc < ncol; kc += 64) {
         int sp = 0;
-        for (int ch = (1 << t.dim) - 1; ch >= 0; --ch) {
-            int x = t.child[(size_t)ch * t.nboxes + C];
-            if (x >= 0) stack[sp++] = x;
-        }
-        while (sp > 0) {
-            int D = stack[--sp];
-            if (t.src_cumul[D] == 0) continue;
-            bool leaf = tv_leaf(t, D);
-            if (tv_gap(t, D, B, e) >= n) {
-                if (t.src_cumul[D] < minsrc) {
-                    // all source leaves below D go to list 1
-                    int sub[STACK];
-                    int sq = 0;
-                    sub[sq++] = D;
-                    while (sq > 0) {
-                        int X = sub[--sq];
-                        if (t.src_cumul[X] == 0) continue;
-                        if (tv_leaf(t, X)) {
-                            if (t.src_nonchild[X] > 0) emit(o1, it, k1, X);
-                            continue;
-                        }
-                        for (int ch = (1 << t.dim) - 1; ch >= 0; --ch) {
-                            int x = t.child[(size_t)ch * t.nboxes + X];
-                            if (x < 0) continue;
-                            if (sq >= STACK) { atomicOr(err, 1); return; }
-                            sub[sq++] = x;
-                        }
-                    }
-                } else {
-                    emit(o3, it, k3, D);
-                }
-            } else if (leaf) {
-                if (t.src_nonchild[D] > 0) emit(o1, it, k1, D);
-            } else {
-                for (int ch = (1 << t.dim) - 1; ch >= 0; --ch) {
-                    int x = t.child[(size_t)ch * t.nboxes + D];
-                    if (x < 0) continue;
-                    if (sp >= STACK) { atomicOr(err, 1); return; }
-                    stack[sp++] = x;
+        int D = kc + lane < ncol ? tv_colleague(t, B, n, kc + lane) : -1;
+        bool sub = false, expand = D >= 0;
+        for (;;) {
+            // push the children of the lanes' boxes, lane 0's on top
+            int cnt = 0;
+            if (expand)
+                for (int ch = 0; ch < nchild; ++ch)
+                    cnt += t.child[(size_t)ch * t.nboxes + D] >= 0;
+            int after = cnt;   // this lane's and the higher lanes' children
+            for (int o = 1; o < 64; o <<= 1) {
+                const int x = __shfl_down(after, o);
+                if (lane + o < 64) after += x;
+            }
+            const int total = __shfl(after, 0);
+            if (cnt > 0) {
+                int at = sp + after - cnt;
+                for (int ch = 0; ch < nchild; ++ch) {
+                    const int x = t.child[(size_t)ch * t.nboxes + D];
+                    if (x >= 0) stack[at++] = (int)((unsigned)x | (sub ? SUB : 0u));
                 }
             }
+            __syncthreads();
+            sp += total;
+            if (sp == 0) break;
+            const int m = sp < 64 ? sp : 64;
+            const unsigned v = lane < m ? (unsigned)stack[sp - 1 - lane] : 0u;
+            __syncthreads();
+            sp -= m;
+            D = (int)(v & ~SUB);
+            sub = (v & SUB) != 0;
+            bool one = false, three = false;
+            expand = false;
+            if (lane < m && t.src_cumul[D] > 0) {
+                const bool leaf = tv_leaf(t, D);
+                const bool sep = !sub && tv_gap(t, D, B, e) >= n;
+                three = sep && t.src_cumul[D] >= minsrc;
+                sub = sub || sep;
+                one = !three && leaf && t.src_nonchild[D] > 0;
+                expand = !three && !leaf;
+            }
+            emit(o1, it, k1, one, D);
+            emit(o3, it, k3, three, D);
         }
     }
-    if (!o1.fill) o1.cnt[it] = k1;
-    if (!o3.fill) o3.cnt[it] = k3;
+    if (lane == 0 && !o1.fill) o1.cnt[it] = k1;
+    if (lane == 0 && !o3.fill) o3.cnt[it] = k3;
 }
 
-__global__ void k_list24(TV t, int n, int nttp, const int *ttp_boxes, ListOut o2, ListOut o4)
+// Lists 2 and 4, one wavefront per box, the candidates dealt to the lanes
+__global__ void __launch_bounds__(64) k_list24(TV t, int n, int nttp, const int *ttp_boxes,
+                                               ListOut o2, ListOut o4)
 {
-    int it = blockIdx.x * blockDim.x + threadIdx.x;
-    if (it >= nttp) return;
-    int P = ttp_boxes[it];
+    __shared__ int anc[MAX_LEVELS];
+    const int lane = threadIdx.x, nchild = 1 << t.dim;
+    const int it = blockIdx.x;
+    const int P = ttp_boxes[it];
     int k2 = 0, k4 = 0;
     int lp = t.level[P];
     if (lp > 0) {
         int ncol = 1;
         for (int d = 0; d < t.dim; ++d) ncol *= (2 * n + 1);
         int Q = t.parent[P];
-        for (int kc = 0; kc < ncol; ++kc) {
-            int C = tv_colleague(t, Q, n, kc);
-            if (C < 0) continue;
-            for (int ch = 0; ch < (1 << t.dim); ++ch) {
-                int A = t.child[(size_t)ch * t.nboxes + C];
-                if (A < 0 || t.src_cumul[A] == 0) continue;
+        for (int i0 = 0; i0 < ncol; i0 += 64) {
+            const int C = i0 + lane < ncol ? tv_colleague(t, Q, n, i0 + lane) : -1;
+            for (int ch = 0; ch < nchild; ++ch) {
+                const int A = C >= 0 ? t.child[(size_t)ch * t.nboxes + C] : -1;
                 long long g = 0;
-                for (int d = 0; d < t.dim; ++d) {
-                    long long dd = (long long)t.coords[(size_t)d * t.nboxes + A] -
-                                   t.coords[(size_t)d * t.nboxes + P];
-                    if (dd < 0) dd = -dd;
-                    if (dd > g) g = dd;
-                }
-                if (g > n) emit(o2, it, k2, A);
+                if (A >= 0 && t.src_cumul[A] > 0)
+                    for (int d = 0; d < t.dim; ++d) {
+                        long long dd = (long long)t.coords[(size_t)d * t.nboxes + A] -
+                                       t.coords[(size_t)d * t.nboxes + P];
+                        if (dd < 0) dd = -dd;
+                        if (dd > g) g = dd;
+                    }
+                emit(o2, it, k2, g > n, A);
             }
         }
-        int anc[MAX_LEVELS];
-        int na = 0;
-        for (int a = Q; a >= 0 && na < MAX_LEVELS; a = t.parent[a]) anc[na++] = a;
-        for (int j = na - 1; j >= 0; --j) {
-            for (int kc = 0; kc < ncol; ++kc) {
-                int Sb = tv_colleague(t, anc[j], n, kc);
-                if (Sb < 0 || !tv_leaf(t, Sb) || t.src_nonchild[Sb] == 0) continue;
-                if (tv_gap(t, Sb, P, 0) >= n && tv_gap(t, Sb, Q, 0) < n) emit(o4, it, k4, Sb);
+        const int na = tv_ancestors(t, Q, anc);
+        for (int i0 = 0; i0 < na * ncol; i0 += 64) {
+            const int i = i0 + lane;
+            bool four = false;
+            int Sb = -1;
+            if (i < na * ncol) {
+                Sb = tv_colleague(t, anc[i / ncol], n, i % ncol);
+                four = Sb >= 0 && t.src_nonchild[Sb] > 0 && tv_leaf(t, Sb) &&
+                       tv_gap(t, Sb, P, 0) >= n && tv_gap(t, Sb, Q, 0) < n;
             }
+            emit(o4, it, k4, four, Sb);
         }
     }
-    if (!o2.fill) o2.cnt[it] = k2;
-    if (!o4.fill) o4.cnt[it] = k4;
+    if (lane == 0 && !o2.fill) o2.cnt[it] = k2;
+    if (lane == 0 && !o4.fill) o4.cnt[it] = k4;
 }
 
-__global__ void k_sort_lists(int nitems, const int *starts, int *lists)
+// Sorts each list (distinct box numbers) from `in` to `out`, a block per
+// list.  Up to SORT_RANK entries: every entry's rank by comparison with the
+// others in LDS.  More: a bitmap of the box numbers in LDS, `words` of it at
+// a time, read back in order (one thread's insertion sort of the longest
+// list, 12 thousand boxes, took 240 ms; a launch now takes under 45 us).
+constexpr int SORT_RANK = 256, SORT_WORDS = 8192;
+
+__global__ void __launch_bounds__(256) k_sort_lists(const int *starts, const int *in, int *out,
+                                                    int nboxes, int words)
 {
-    int it = blockIdx.x * blockDim.x + threadIdx.x;
-    if (it >= nitems) return;
-    int a = starts[it], b = starts[it + 1];
-    for (int i = a + 1; i < b; ++i) {
-        int v = lists[i];
-        int j = i - 1;
-        while (j >= a && lists[j] > v) {
-            lists[j + 1] = lists[j];
-            --j;
+    extern __shared__ unsigned bits[];
+    __shared__ int wsum[4];
+    const int tid = threadIdx.x;
+    const int a = starts[blockIdx.x], n = starts[blockIdx.x + 1] - a;
+    if (n <= SORT_RANK) {
+        int v = 0;
+        if (tid < n) {
+            v = in[a + tid];
+            bits[tid] = (unsigned)v;
         }
-        lists[j + 1] = v;
+        __syncthreads();
+        if (tid < n) {
+            int r = 0;
+            for (int j = 0; j < n; ++j) r += (int)bits[j] < v;
+            out[a + r] = v;
+        }
+        return;
     }
+    int base = a;
+    for (long lo = 0; lo < nboxes; lo += 32L * words) {
+        for (int w = tid; w < words; w += 256) bits[w] = 0;
+        __syncthreads();
+        for (int i = tid; i < n; i += 256) {
+            const long b = in[a + i] - lo;
+            if (b >= 0 && b < 32L * words) atomicOr(&bits[b >> 5], 1u << (b & 31));
+        }
+        __syncthreads();
+        for (int w0 = 0; w0 < words; w0 += 256) {
+            const int w = w0 + tid;
+            unsigned x = w < words ? bits[w] : 0u;
+            const int c = __popc(x);
+            int s = c;
+            for (int o = 1; o < 64; o <<= 1) {
+                const int y = __shfl_up(s, o);
+                if ((tid & 63) >= o) s += y;
+            }
+            if ((tid & 63) == 63) wsum[tid >> 6] = s;
+            __syncthreads();
+            int at = base + s - c, all = 0;
+            for (int k = 0; k < 4; ++k) {
+                if (k < (tid >> 6)) at += wsum[k];
+                all += wsum[k];
+            }
+            while (x) {
+                out[at++] = (int)(lo + 32L * w + __ffs(x) - 1);
+                x &= x - 1;
+            }
+            base += all;
+            __syncthreads();
+        }
+    }
+}
+
+static void sort_lists(hipStream_t st, int nitems, int nboxes, const dbuf<int> &starts,
+                       const dbuf<int> &in, dbuf<int> &out)
+{
+    const int words = std::max(SORT_RANK, std::min(cdiv(nboxes, 32), SORT_WORDS));
+    hipLaunchKernelGGL(k_sort_lists, dim3(nitems), dim3(256), words * sizeof(unsigned), st,
+                       starts.p, in.p, out.p, nboxes, words);
 }
 
 __global__ void k_box_flags(TV t, const int *tgt_nonchild, int *f_src, int *f_srcpar,
@@ -306,11 +396,13 @@ static int level_starts(hipStream_t st, const qbx_tree *T, const dbuf<int> &boxe
     return QBX_OK;
 }
 
+// starts, and room for the lists as they are found (raw) and sorted
 static int build_lists(qbx_ctx *ctx, hipStream_t st, int nitems, dbuf<int> &starts,
-                       dbuf<int> &lists, int *total, dbuf<int> &cnt)
+                       dbuf<int> &raw, dbuf<int> &lists, int *total, dbuf<int> &cnt)
 {
     QBX_TRY(starts.alloc(nitems + 1));
     QBX_TRY(exclusive_scan(ctx, st, cnt.p, starts.p, nitems, total));
+    QBX_TRY(raw.alloc(std::max(*total, 1)));
     QBX_TRY(lists.alloc(std::max(*total, 1)));
     lists.n = *total;
     return QBX_OK;
@@ -370,75 +462,70 @@ static int traverse(qbx_ctx *ctx, hipStream_t st, const qbx_tree *T, int n, int 
                            R->ntarget_boxes, R->target_boxes.p, R->box_to_target_box.p);
     QBX_HIP(hipGetLastError());
 
-    // err[0]: stack overflow flag; err[1], err[2]: the coarsest levels of
-    // qbx_trav::mpole_min_level and local_min_level
-    dbuf<int> err;
-    QBX_TRY(err.alloc(3));
-    const int err_init[3] = {0, T->nlevels, T->nlevels};
-    QBX_HIP(hipMemcpyAsync(err.p, err_init, sizeof(err_init), hipMemcpyHostToDevice, st));
     // lists 1 and 3
     {
         int ntb = R->ntarget_boxes;
-        dbuf<int> c1, c3;
+        const size_t stack = sizeof(int) * 64 * (size_t)T->nlevels << T->dim;
+        dbuf<int> c1, c3, r1, r3;
         QBX_TRY(c1.alloc(std::max(ntb, 1)));
         QBX_TRY(c3.alloc(std::max(ntb, 1)));
         ListOut o1{c1.p, nullptr, nullptr, 0}, o3{c3.p, nullptr, nullptr, 0};
         if (ntb)
-            hipLaunchKernelGGL(k_list13, dim3(cdiv(ntb, 64)), dim3(64), 0, st, t, n, ext, minsrc,
-                               ntb, R->target_boxes.p, o1, o3, err.p);
+            hipLaunchKernelGGL(k_list13, dim3(ntb), dim3(64), stack, st, t, n, ext, minsrc, ntb,
+                               R->target_boxes.p, o1, o3);
         QBX_HIP(hipGetLastError());
-        QBX_TRY(build_lists(ctx, st, ntb, R->l1_starts, R->l1_lists, &R->n1, c1));
-        QBX_TRY(build_lists(ctx, st, ntb, R->l3_starts, R->l3_lists, &R->n3, c3));
-        o1 = ListOut{nullptr, R->l1_starts.p, R->l1_lists.p, 1};
-        o3 = ListOut{nullptr, R->l3_starts.p, R->l3_lists.p, 1};
+        QBX_TRY(build_lists(ctx, st, ntb, R->l1_starts, r1, R->l1_lists, &R->n1, c1));
+        QBX_TRY(build_lists(ctx, st, ntb, R->l3_starts, r3, R->l3_lists, &R->n3, c3));
+        o1 = ListOut{nullptr, R->l1_starts.p, r1.p, 1};
+        o3 = ListOut{nullptr, R->l3_starts.p, r3.p, 1};
         if (ntb) {
-            hipLaunchKernelGGL(k_list13, dim3(cdiv(ntb, 64)), dim3(64), 0, st, t, n, ext, minsrc,
-                               ntb, R->target_boxes.p, o1, o3, err.p);
-            hipLaunchKernelGGL(k_sort_lists, dim3(cdiv(ntb, 64)), dim3(64), 0, st, ntb,
-                               R->l1_starts.p, R->l1_lists.p);
-            hipLaunchKernelGGL(k_sort_lists, dim3(cdiv(ntb, 64)), dim3(64), 0, st, ntb,
-                               R->l3_starts.p, R->l3_lists.p);
+            hipLaunchKernelGGL(k_list13, dim3(ntb), dim3(64), stack, st, t, n, ext, minsrc, ntb,
+                               R->target_boxes.p, o1, o3);
+            sort_lists(st, ntb, nb, R->l1_starts, r1, R->l1_lists);
+            sort_lists(st, ntb, nb, R->l3_starts, r3, R->l3_lists);
         }
         QBX_HIP(hipGetLastError());
     }
     // lists 2 and 4
     {
         int nt = R->nttp_boxes;
-        dbuf<int> c2, c4;
+        dbuf<int> c2, c4, r2, r4;
         QBX_TRY(c2.alloc(std::max(nt, 1)));
         QBX_TRY(c4.alloc(std::max(nt, 1)));
         ListOut o2{c2.p, nullptr, nullptr, 0}, o4{c4.p, nullptr, nullptr, 0};
         if (nt)
-            hipLaunchKernelGGL(k_list24, dim3(cdiv(nt, 64)), dim3(64), 0, st, t, n, nt,
-                               R->ttp_boxes.p, o2, o4);
+            hipLaunchKernelGGL(k_list24, dim3(nt), dim3(64), 0, st, t, n, nt, R->ttp_boxes.p, o2,
+                               o4);
         QBX_HIP(hipGetLastError());
-        QBX_TRY(build_lists(ctx, st, nt, R->l2_starts, R->l2_lists, &R->n2, c2));
-        QBX_TRY(build_lists(ctx, st, nt, R->l4_starts, R->l4_lists, &R->n4, c4));
-        o2 = ListOut{nullptr, R->l2_starts.p, R->l2_lists.p, 1};
-        o4 = ListOut{nullptr, R->l4_starts.p, R->l4_lists.p, 1};
+        QBX_TRY(build_lists(ctx, st, nt, R->l2_starts, r2, R->l2_lists, &R->n2, c2));
+        QBX_TRY(build_lists(ctx, st, nt, R->l4_starts, r4, R->l4_lists, &R->n4, c4));
+        o2 = ListOut{nullptr, R->l2_starts.p, r2.p, 1};
+        o4 = ListOut{nullptr, R->l4_starts.p, r4.p, 1};
         if (nt) {
-            hipLaunchKernelGGL(k_list24, dim3(cdiv(nt, 64)), dim3(64), 0, st, t, n, nt,
-                               R->ttp_boxes.p, o2, o4);
-            hipLaunchKernelGGL(k_sort_lists, dim3(cdiv(nt, 64)), dim3(64), 0, st, nt,
-                               R->l2_starts.p, R->l2_lists.p);
-            hipLaunchKernelGGL(k_sort_lists, dim3(cdiv(nt, 64)), dim3(64), 0, st, nt,
-                               R->l4_starts.p, R->l4_lists.p);
+            hipLaunchKernelGGL(k_list24, dim3(nt), dim3(64), 0, st, t, n, nt, R->ttp_boxes.p, o2,
+                               o4);
+            sort_lists(st, nt, nb, R->l2_starts, r2, R->l2_lists);
+            sort_lists(st, nt, nb, R->l4_starts, r4, R->l4_lists);
         }
         QBX_HIP(hipGetLastError());
     }
-    min_level(st, R->n2, R->l2_lists.p, nullptr, nullptr, T->box_levels.p, err.p + 1);
-    min_level(st, R->n3, R->l3_lists.p, nullptr, nullptr, T->box_levels.p, err.p + 1);
+    // the coarsest levels: qbx_trav::mpole_min_level and local_min_level
+    dbuf<int> coarsest;
+    QBX_TRY(coarsest.alloc(2));
+    const int none[2] = {T->nlevels, T->nlevels};
+    QBX_HIP(hipMemcpyAsync(coarsest.p, none, sizeof(none), hipMemcpyHostToDevice, st));
+    min_level(st, R->n2, R->l2_lists.p, nullptr, nullptr, T->box_levels.p, coarsest.p);
+    min_level(st, R->n3, R->l3_lists.p, nullptr, nullptr, T->box_levels.p, coarsest.p);
     min_level(st, R->nttp_boxes, nullptr, R->l2_starts.p, R->ttp_boxes.p, T->box_levels.p,
-              err.p + 2);
+              coarsest.p + 1);
     min_level(st, R->nttp_boxes, nullptr, R->l4_starts.p, R->ttp_boxes.p, T->box_levels.p,
-              err.p + 2);
+              coarsest.p + 1);
     QBX_HIP(hipGetLastError());
-    int herr[3] = {0, 0, 0};
-    QBX_HIP(hipMemcpyAsync(herr, err.p, sizeof(herr), hipMemcpyDeviceToHost, st));
+    int hc[2] = {0, 0};
+    QBX_HIP(hipMemcpyAsync(hc, coarsest.p, sizeof(hc), hipMemcpyDeviceToHost, st));
     QBX_HIP(hipStreamSynchronize(st));
-    QBX_CHECK(herr[0] == 0, "qbx_traverse: traversal stack overflow");
-    R->mpole_min_level = herr[1];
-    R->local_min_level = herr[2];
+    R->mpole_min_level = hc[0];
+    R->local_min_level = hc[1];
     return QBX_OK;
 }
 
