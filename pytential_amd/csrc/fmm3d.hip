@@ -274,7 +274,7 @@ __device__ __forceinline__ double p2p_value(const KD &kd, v3 s, v3 nu, v3 t)
     const v3 d = sub(t, s);
     const double r2 = d.x * d.x + d.y * d.y + d.z * d.z;
     if (r2 == 0.0) return 0.0;
-    const double ir = 1.0 / sqrt(r2);
+    const double ir = qbx_rsqrt(r2);
     if (!kd.dip) return INV4PI * ir;
     return INV4PI * ir * ir * ir * (nu.x * d.x + nu.y * d.y + nu.z * d.z);
 }
@@ -1337,7 +1337,9 @@ k3_trans_real(KD kd, TD t, int lv, int i0, const int *boxes, const int *starts,
     }
 }
 
-// P2P (MODE 0, list 1), M2P (1, list 3), L2P (2) for non-QBX targets
+// P2P (MODE 0, list 1), M2P (1, list 3), L2P (2) for non-QBX targets, a
+// wavefront per target box: L2P, and the others where the geometry's work
+// units are those of another traversal
 template <int MODE, int NRC>
 __global__ void __launch_bounds__(64) k3_eval_targets(KD kd, TD t, int ntb, const int *tboxes,
                                                       const int *starts, const int *lists,
@@ -1414,6 +1416,68 @@ __global__ void __launch_bounds__(64) k3_eval_targets(KD kd, TD t, int ntb, cons
             }
         if (active && sub_ == 0) store_add<NRC>(kd, pot + 2 * (size_t)ti * kd.nr, acc);
     }
+}
+
+// P2P (MODE 0, list 1) and M2P (1, list 3) over the geometry's work units
+// (unit_plan): G lanes per target, each walking every G-th source of a list-1
+// box or every G-th list-3 box, reduced by shuffles.  A target in a coarse
+// box against all of a surface's sources is a long walk: with a wavefront per
+// target box the 3001 loose points around 46080 sources kept a few
+// wavefronts busy for 32 ms (P2P) and 2.1 ms (M2P); over units 0.61 and
+// 0.18 ms, one target's walk on 64 lanes.
+template <int MODE, int NRC>
+__global__ void __launch_bounds__(64) k3_eval_units(KD kd, TD t, const int *ubox, const int *ut0,
+                                                    const int *box_g, const int *tboxes,
+                                                    const int *starts, const int *lists,
+                                                    const int *fstart, const int *fcount,
+                                                    const int *unfilt, const double *tgt, int nt,
+                                                    const double *src, int ns,
+                                                    const double *str, const double *nrm,
+                                                    const double *expn, double *pot)
+{
+    const int u = blockIdx.x;
+    const int it = ubox[u];
+    const int B = tboxes[it];
+    const int G = box_g[it];
+    const int lane = threadIdx.x;
+    const int tsub = lane / G, sub_ = lane & (G - 1);
+    const int tl = ut0[u] + tsub;
+    const bool active = tl < fcount[B];
+    const int ti = active ? unfilt[fstart[B] + tl] : 0;
+    const v3 tp = active ? ld3(tgt, nt, ti) : v3{0, 0, 0};
+    cplx acc[NRC];
+#pragma unroll
+    for (int q = 0; q < NRC; ++q) acc[q] = {0, 0};
+    const int e0 = starts[it], e1 = starts[it + 1];
+    if (active && MODE == 0) {
+        for (int e = e0; e < e1; ++e) {
+            const int Sb = lists[e];
+            const int s0 = t.sstart[Sb], s1 = s0 + t.scount[Sb];
+            for (int s = s0 + sub_; s < s1; s += G) {
+                const v3 nu = kd.dip ? ld3(nrm, ns, s) : v3{0, 0, 0};
+                const double g = p2p_value(kd, ld3(src, ns, s), nu, tp);
+#pragma unroll
+                for (int q = 0; q < NRC; ++q)
+                    if (q < kd.rc) acc[q] += g * ldq(kd, str, s, kd.r0 + q);
+            }
+        }
+    } else if (active) {
+        for (int e = e0 + sub_; e < e1; e += G) {
+            const int D = lists[e];
+            const int lv = t.level[D];
+            sum_irregular_n<NRC>(kd, expn + ecoef_off(kd, D, lv), kd.order[lv],
+                                 sub(tp, boxc(t, D)), acc);
+        }
+#pragma unroll
+        for (int q = 0; q < NRC; ++q) acc[q] = INV4PI * acc[q];
+    }
+#pragma unroll
+    for (int q = 0; q < NRC; ++q)
+        for (int m = G >> 1; m >= 1; m >>= 1) {
+            acc[q].x += __shfl_xor(acc[q].x, m);
+            acc[q].y += __shfl_xor(acc[q].y, m);
+        }
+    if (active && sub_ == 0) store_add<NRC>(kd, pot + 2 * (size_t)ti * kd.nr, acc);
 }
 
 // ---- QBX stages
@@ -2600,6 +2664,26 @@ int f3_eval_targets(qbx_ctx *ctx, void *stream, const qbx_tree *T, const qbx_tra
     const TD td = make_td(T);
     const int *starts = mode == 1 ? R->l3_starts.p : R->l1_starts.p;
     const int *lists = mode == 1 ? R->l3_lists.p : R->l1_lists.p;
+    if (mode != 2 && G->trav == R) {
+        const unit_plan &U = mode == 0 ? G->p2p_plan : G->m2p_plan;
+        if (U.nunits == 0) return QBX_OK;
+#define EVAL3_UNITS(M, N)                                                                  \
+    hipLaunchKernelGGL((k3_eval_units<M, N>), dim3(U.nunits), dim3(64), 0, st, kd, td,     \
+                       U.unit_box.p, U.unit_t0.p, U.box_g.p, R->target_boxes.p, starts,   \
+                       lists, G->nqbtl_box_target_starts.p,                               \
+                       G->nqbtl_box_target_counts_nonchild.p, G->nqbtl_unfiltered.p,      \
+                       T->targets.p, T->ntargets, T->sources.p, T->nsources, str, nrm, expn, \
+                       pot)
+#define EV3U0(N) EVAL3_UNITS(0, N)
+#define EV3U1(N) EVAL3_UNITS(1, N)
+        if (mode == 0) FOR_RHS_CHUNKS3(kd, NRC_S, EV3U0);
+        else FOR_RHS_CHUNKS3(kd, NRC_S, EV3U1);
+#undef EV3U0
+#undef EV3U1
+#undef EVAL3_UNITS
+        QBX_HIP(hipGetLastError());
+        return QBX_OK;
+    }
 #define EVAL3_LAUNCH(M, N)                                                                 \
     hipLaunchKernelGGL((k3_eval_targets<M, N>), dim3(ntb), dim3(64), 0, st, kd, td, ntb,   \
                        R->target_boxes.p, starts, lists, G->nqbtl_box_target_starts.p,    \
