@@ -8,14 +8,25 @@
 //   dpot_dk[t] = sum_s dG_k/dk q_s = sum_s i e^{ik|t-s|} / (4 pi) q_s
 //   v[s]      = sum_t conj(G_k(t, s)) u_t     (the adjoint, G^H u)
 //
-// Forward: few targets (thousands) against many sources (10^5-10^6), so the
-// sources are split into chunks across blocks: block (target tile, source
-// chunk) sums its chunk for 256 targets through LDS tiles of sources and
-// writes a partial; a second kernel adds the partials of each target in chunk
-// order (deterministic, no atomics).  Adjoint: one thread per source, the
-// targets staged through LDS.  Coincident points contribute zero.
+// Both directions are a point per thread against the other set, staged
+// through LDS in tiles.  Forward: few targets (thousands) against many
+// sources, so the sources are split into chunks across blocks until they
+// fill the chip: block (tile of 256 targets, chunk) sums its chunk and writes
+// a partial, and a second kernel adds the partials of each target in chunk
+// order.  Adjoint: a source takes 1, 4 or 16 threads of a block, whichever
+// first gives blocks to fill the chip, added in LDS in order (no scratch
+// memory: calls on several streams share nothing).  Deterministic, no
+// atomics.  Coincident points contribute zero.
+//
+// FP64 VALU bound: a pair is 59 (forward with the k-derivative) or 57
+// instructions.  4096 targets and 737280 sources, 3.0e9 pairs: forward
+// 8.1 -> 5.4 ms, adjoint 8.0 -> 5.2 ms against two Newton steps, nine-term
+// Taylor series and a branch per pair for coincidence and for the range of
+// the sine.
 #include "qbx_internal.h"
 #include "qbx_math.h"
+
+#include <algorithm>
 
 namespace qbx {
 
@@ -23,58 +34,100 @@ constexpr int H3_THREADS = 256;   // targets (forward) / sources (adjoint) per b
 constexpr int H3_TILE = 256;      // staged points per LDS tile
 constexpr double INV4PI = 0.07957747154594766788;
 
-__global__ void __launch_bounds__(H3_THREADS)
-k_h3_p2p_partial(int ns, const double *src, const double *q, int nt, const double *tgt,
-                 double k, int chunk, double *part_pot, double *part_dk)
-{
-    __shared__ double sx[H3_TILE], sy[H3_TILE], sz[H3_TILE], sqr[H3_TILE], sqi[H3_TILE];
-    const int t = blockIdx.x * H3_THREADS + threadIdx.x;
-    const int c = blockIdx.y;
-    const int s0 = c * chunk, s1 = min(ns, s0 + chunk);
-    const bool act = t < nt;
-    const double tx = act ? tgt[t] : 0.0, ty = act ? tgt[(size_t)nt + t] : 0.0,
-                 tz = act ? tgt[2 * (size_t)nt + t] : 0.0;
+struct H3Sums {
     double pr = 0, pi = 0, dr = 0, di = 0;
-    for (int b = s0; b < s1; b += H3_TILE) {
-        const int nb = min(H3_TILE, s1 - b);
+};
+
+// e^{+-ikr} q / r (and i e^{ikr} q) of one pair, added.  FAST leaves out the
+// test for coincident points and large k r and reports either (a coincident
+// pair's k r is a NaN) for the tile to be summed again without FAST.
+template <bool FAST, bool ADJ>
+__device__ __forceinline__ bool h3_pair(double dx, double dy, double dz, double k, double qr,
+                                        double qi, H3Sums &a)
+{
+    const double r2 = dx * dx + dy * dy + dz * dz;
+    if (!FAST && r2 == 0.0) return false;
+    const double ir = qbx_rsqrt(r2);
+    const double x = k * (r2 * ir);
+    double sn, cs;
+    if (FAST)
+        qbx_sincos_core(x, &sn, &cs);
+    else
+        qbx_sincos(x, &sn, &cs);
+    const double si = ADJ ? -sn : sn;
+    const double er = cs * qr - si * qi;
+    const double ei = cs * qi + si * qr;
+    a.pr += er * ir;
+    a.pi += ei * ir;
+    if (!ADJ) {
+        a.dr -= ei;
+        a.di += er;
+    }
+    return FAST && !(__builtin_fabs(x) <= QBX_SINCOS_MAX);
+}
+
+// part[chunk][point] = the sum over the chunk's points b (values q) at point
+// a of set A, SPL threads to a point; ADJ false: part_dk likewise
+template <bool ADJ, int SPL>
+__global__ void __launch_bounds__(H3_THREADS)
+k_h3_p2p(int nb, const double *ptb, const double *q, int na, const double *pta, double k,
+         int chunk, double scale, double *part, double *part_dk)
+{
+    __shared__ double2 bxy[H3_TILE], bq[H3_TILE];
+    __shared__ double bz[H3_TILE];
+    constexpr int PP = H3_THREADS / SPL;
+    const int sub = threadIdx.x / PP;
+    const int t = blockIdx.x * PP + threadIdx.x % PP;
+    const int c = blockIdx.y;
+    const int b0 = c * chunk, b1 = min(nb, b0 + chunk);
+    const bool act = t < na;
+    const double ax = act ? pta[t] : 0.0, ay = act ? pta[(size_t)na + t] : 0.0,
+                 az = act ? pta[2 * (size_t)na + t] : 0.0;
+    H3Sums tot;
+    for (int b = b0; b < b1; b += H3_TILE) {
+        const int n = min(H3_TILE, b1 - b);
         __syncthreads();
-        for (int j = threadIdx.x; j < nb; j += H3_THREADS) {
-            const int s = b + j;
-            sx[j] = src[s];
-            sy[j] = src[(size_t)ns + s];
-            sz[j] = src[2 * (size_t)ns + s];
-            sqr[j] = q[2 * (size_t)s];
-            sqi[j] = q[2 * (size_t)s + 1];
+        for (int j = threadIdx.x; j < n; j += H3_THREADS) {
+            const size_t s = b + j;
+            bxy[j] = {ptb[s], ptb[(size_t)nb + s]};
+            bz[j] = ptb[2 * (size_t)nb + s];
+            bq[j] = {q[2 * s], q[2 * s + 1]};
         }
         __syncthreads();
-        if (act)
-            for (int j = 0; j < nb; ++j) {
-                const double dx = tx - sx[j], dy = ty - sy[j], dz = tz - sz[j];
-                const double r2 = dx * dx + dy * dy + dz * dz;
-                if (r2 == 0.0) continue;
-                // 1/r and r from the refined hardware estimate; sin and cos
-                // by qbx_sincos (a few ulp, no library call)
-                const double ir = qbx_rsqrt(r2);
-                const double r = r2 * ir;
-                double sn, cs;
-                qbx_sincos(k * r, &sn, &cs);
-                // e^{ikr} q
-                const double er = cs * sqr[j] - sn * sqi[j];
-                const double ei = cs * sqi[j] + sn * sqr[j];
-                pr += er * ir;
-                pi += ei * ir;
-                // i e^{ikr} q
-                dr -= ei;
-                di += er;
-            }
+        H3Sums a;
+        bool again = false;
+#pragma unroll 2
+        for (int j = sub; j < n; j += SPL)
+            again |= h3_pair<true, ADJ>(ax - bxy[j].x, ay - bxy[j].y, az - bz[j], k, bq[j].x,
+                                        bq[j].y, a);
+        if (again && act) {
+            a = H3Sums();
+            for (int j = sub; j < n; j += SPL)
+                h3_pair<false, ADJ>(ax - bxy[j].x, ay - bxy[j].y, az - bz[j], k, bq[j].x,
+                                    bq[j].y, a);
+        }
+        tot.pr += a.pr;
+        tot.pi += a.pi;
+        tot.dr += a.dr;
+        tot.di += a.di;
+    }
+    if (SPL > 1) {
+        __syncthreads();
+        bq[threadIdx.x] = {tot.pr, tot.pi};
+        __syncthreads();
+        if (sub > 0) return;
+        for (int w = 1; w < SPL; ++w) {
+            tot.pr += bq[w * PP + t % PP].x;
+            tot.pi += bq[w * PP + t % PP].y;
+        }
     }
     if (act) {
-        const size_t o = (size_t)c * nt + t;
-        part_pot[2 * o] = pr;
-        part_pot[2 * o + 1] = pi;
-        if (part_dk) {
-            part_dk[2 * o] = dr;
-            part_dk[2 * o + 1] = di;
+        const size_t o = (size_t)c * na + t;
+        part[2 * o] = tot.pr * scale;
+        part[2 * o + 1] = tot.pi * scale;
+        if (!ADJ && part_dk) {
+            part_dk[2 * o] = tot.dr * scale;
+            part_dk[2 * o + 1] = tot.di * scale;
         }
     }
 }
@@ -90,48 +143,6 @@ __global__ void k_h3_reduce(int nchunks, int nt, const double *part, double *out
     }
     out[2 * (size_t)t] = re * INV4PI;
     out[2 * (size_t)t + 1] = im * INV4PI;
-}
-
-__global__ void __launch_bounds__(H3_THREADS)
-k_h3_p2p_adjoint(int ns, const double *src, int nt, const double *tgt, double k,
-                 const double *u, double *v)
-{
-    __shared__ double tx_[H3_TILE], ty_[H3_TILE], tz_[H3_TILE], ur[H3_TILE], ui[H3_TILE];
-    const int s = blockIdx.x * H3_THREADS + threadIdx.x;
-    const bool act = s < ns;
-    const double sx = act ? src[s] : 0.0, sy = act ? src[(size_t)ns + s] : 0.0,
-                 sz = act ? src[2 * (size_t)ns + s] : 0.0;
-    double vr = 0, vi = 0;
-    for (int b = 0; b < nt; b += H3_TILE) {
-        const int nb = min(H3_TILE, nt - b);
-        __syncthreads();
-        for (int j = threadIdx.x; j < nb; j += H3_THREADS) {
-            const int t = b + j;
-            tx_[j] = tgt[t];
-            ty_[j] = tgt[(size_t)nt + t];
-            tz_[j] = tgt[2 * (size_t)nt + t];
-            ur[j] = u[2 * (size_t)t];
-            ui[j] = u[2 * (size_t)t + 1];
-        }
-        __syncthreads();
-        if (act)
-            for (int j = 0; j < nb; ++j) {
-                const double dx = tx_[j] - sx, dy = ty_[j] - sy, dz = tz_[j] - sz;
-                const double r2 = dx * dx + dy * dy + dz * dz;
-                if (r2 == 0.0) continue;
-                const double ir = qbx_rsqrt(r2);
-                const double r = r2 * ir;
-                double sn, cs;
-                qbx_sincos(k * r, &sn, &cs);
-                // e^{-ikr} u / r
-                vr += (cs * ur[j] + sn * ui[j]) * ir;
-                vi += (cs * ui[j] - sn * ur[j]) * ir;
-            }
-    }
-    if (act) {
-        v[2 * (size_t)s] = vr * INV4PI;
-        v[2 * (size_t)s + 1] = vi * INV4PI;
-    }
 }
 
 // out[e, j, r] = sum_i mat[i, j] in[e, i, r]  (the transpose of qbx_upsample)
@@ -176,7 +187,7 @@ int qbx_helmholtz3d_p2p(qbx_ctx *ctx, void *stream, int nsources, const double *
         return QBX_OK;
     }
     const int tiles = cdiv(ntargets, H3_THREADS);
-    // enough blocks to fill the chip (>= 8 per CU on 256 CUs), chunks of at
+    // enough blocks to fill the chip (8 per CU on 256 CUs), chunks of at
     // least one LDS tile
     int nchunks = std::max(1, 2048 / tiles);
     nchunks = std::min(nchunks, cdiv(nsources, H3_TILE));
@@ -187,8 +198,8 @@ int qbx_helmholtz3d_p2p(qbx_ctx *ctx, void *stream, int nsources, const double *
     QBX_TRY(scratch_reserve(ctx, st, dpot_dk ? 2 * pb : pb, &scr));
     double *ppot = (double *)scr;
     double *pdk = dpot_dk ? ppot + 2 * (size_t)nchunks * ntargets : nullptr;
-    hipLaunchKernelGGL(k_h3_p2p_partial, dim3(tiles, nchunks), dim3(H3_THREADS), 0, st, nsources,
-                       sources, strengths, ntargets, targets, k, chunk, ppot, pdk);
+    hipLaunchKernelGGL((k_h3_p2p<false, 1>), dim3(tiles, nchunks), dim3(H3_THREADS), 0, st,
+                       nsources, sources, strengths, ntargets, targets, k, chunk, 1.0, ppot, pdk);
     hipLaunchKernelGGL(k_h3_reduce, dim3(cdiv(ntargets, 256)), dim3(256), 0, st, nchunks,
                        ntargets, ppot, pot);
     if (dpot_dk)
@@ -208,8 +219,18 @@ int qbx_helmholtz3d_p2p_adjoint(qbx_ctx *ctx, void *stream, int nsources, const 
     QBX_CHECK(ntargets == 0 || (targets && u), "qbx_helmholtz3d_p2p_adjoint: null targets");
     if (nsources == 0) return QBX_OK;
     hipStream_t st = S(stream);
-    hipLaunchKernelGGL(k_h3_p2p_adjoint, dim3(cdiv(nsources, H3_THREADS)), dim3(H3_THREADS), 0,
-                       st, nsources, sources, ntargets, targets, k, u, v);
+#define H3_ADJ(SPL)                                                                       \
+    hipLaunchKernelGGL((k_h3_p2p<true, SPL>), dim3(cdiv(nsources, H3_THREADS / (SPL))),    \
+                       dim3(H3_THREADS), 0, st, ntargets, targets, u, nsources, sources, k, \
+                       ntargets, INV4PI, v, nullptr)
+    // 1024 blocks (four per CU) at 1 and 4 threads a source, else 16
+    if (nsources >= 1024 * H3_THREADS)
+        H3_ADJ(1);
+    else if (nsources >= 256 * H3_THREADS)
+        H3_ADJ(4);
+    else
+        H3_ADJ(16);
+#undef H3_ADJ
     QBX_HIP(hipGetLastError());
     return QBX_OK;
 }

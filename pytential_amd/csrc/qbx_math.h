@@ -19,73 +19,75 @@ namespace qbx {
 // division are correctly rounded or nearly so and cost 30..90 instructions
 // each; the pair loops only need a few ulp.
 
-// 1 / sqrt(x) for positive normal x: the hardware estimate refined by two
-// Newton steps (each squares the relative error)
+// 1 / sqrt(x) for positive normal x: the hardware estimate y (relative error
+// below 2^-22) refined by one step of third order, y (1 + e/2 + 3 e^2/8) with
+// e = 1 - x y^2 (the dropped term is 5 e^3/16); two instructions fewer than
+// two Newton steps and the same last rounding
 __device__ __forceinline__ double qbx_rsqrt(double x)
 {
-    double y = __builtin_amdgcn_rsq(x);
-    const double h = 0.5 * x;
-    double e = __builtin_fma(-h * y, y, 0.5);
-    y = __builtin_fma(y, e, y);
-    e = __builtin_fma(-h * y, y, 0.5);
-    return __builtin_fma(y, e, y);
+    const double y = __builtin_amdgcn_rsq(x);
+    const double e = __builtin_fma(-x * y, y, 1.0);
+    return __builtin_fma(y * e, __builtin_fma(0.375, e, 0.5), y);
 }
 
-// 1 / x for normal x: the hardware estimate refined by two Newton steps
+// 1 / x for normal x: the hardware estimate y refined by y (1 + e + e^2),
+// e = 1 - x y
 __device__ __forceinline__ double qbx_rcp(double x)
 {
-    double y = __builtin_amdgcn_rcp(x);
-    double e = __builtin_fma(-x, y, 1.0);
-    y = __builtin_fma(y, e, y);
-    e = __builtin_fma(-x, y, 1.0);
-    return __builtin_fma(y, e, y);
+    const double y = __builtin_amdgcn_rcp(x);
+    const double e = __builtin_fma(-x, y, 1.0);
+    return __builtin_fma(y, __builtin_fma(e, e, e), y);
 }
 
-// sin and cos of one argument, within 2 ulp of 1 for |x| <= 1.6e6 (checked
-// against the host library over [0, 1.6e6]): Cody and Waite's reduction
-// (W. J. Cody and W. Waite, Software Manual for the Elementary Functions,
-// 1980) by q = rint(x 2/pi) with pi/2 split into three doubles, the first
-// two of 33 significant bits so that q P1 and q P2 are exact for |q| < 2^20,
-// then the Taylor series of sin and cos on |r| <= pi/4 (through r^17 and
-// r^16: truncation below 1e-17); the quadrant from q mod 4.  Larger
-// arguments take the device library.
-__device__ __forceinline__ void qbx_sincos(double x, double *sn, double *cs)
+constexpr double QBX_SINCOS_MAX = 1.6e6;
+
+// sin and cos of one argument |x| <= QBX_SINCOS_MAX, within 2 ulp of 1
+// (checked against the host library over that range): reduction by the
+// nearest multiple q of pi/2 (W. J. Cody and W. Waite, Software Manual for
+// the Elementary Functions, 1980; q from adding and subtracting 1.5 2^52, so
+// that its last bits are the sum's), pi/2 in two doubles (the first product
+// is exact inside its fused multiply-add), then polynomials in r^2 that
+// interpolate (sin r - r)/r^3 and (cos r - 1 + r^2/2)/r^4 at the Chebyshev
+// points of |r| <= pi/4 (six coefficients each: 2e-17 and 9e-19 of 1),
+// the quadrant from q mod 4.
+__device__ __forceinline__ void qbx_sincos_core(double x, double *sn, double *cs)
 {
-    if (!(__builtin_fabs(x) <= 1.6e6)) {
-        sincos(x, sn, cs);
-        return;
-    }
-    constexpr double TWO_OVER_PI = 0.6366197723675814;
-    constexpr double P1 = 1.5707963267341256, P2 = 6.077100506303966e-11,
-                     P3 = 2.0222662487959506e-21;
-    const double q = __builtin_rint(x * TWO_OVER_PI);
-    const double r = __builtin_fma(-q, P3, __builtin_fma(-q, P2, __builtin_fma(-q, P1, x)));
+    constexpr double TWO_OVER_PI = 0.6366197723675814, MAGIC = 6755399441055744.0;
+    constexpr double P1 = 1.5707963267948966, P2 = 6.123233995736766e-17;
+    const double t = __builtin_fma(x, TWO_OVER_PI, MAGIC);
+    const double q = t - MAGIC;
+    const int quad = __double2loint(t);
+    const double r = __builtin_fma(-q, P2, __builtin_fma(-q, P1, x));
     const double z = r * r;
-    // 1/n! with alternating signs
-    double ps = -8.22063524662433e-18;
-    ps = __builtin_fma(ps, z, 2.8114572543455206e-15);
-    ps = __builtin_fma(ps, z, -7.647163731819816e-13);
-    ps = __builtin_fma(ps, z, 1.6059043836821613e-10);
-    ps = __builtin_fma(ps, z, -2.505210838544172e-08);
-    ps = __builtin_fma(ps, z, 2.7557319223985893e-06);
-    ps = __builtin_fma(ps, z, -0.0001984126984126984);
-    ps = __builtin_fma(ps, z, 0.008333333333333333);
+    double ps = 1.5918129027234826e-10;
+    ps = __builtin_fma(ps, z, -2.505113184128889e-08);
+    ps = __builtin_fma(ps, z, 2.7557316102534617e-06);
+    ps = __builtin_fma(ps, z, -0.0001984126983675854);
+    ps = __builtin_fma(ps, z, 0.008333333333330948);
     ps = __builtin_fma(ps, z, -0.16666666666666666);
-    double pc = -1.5619206968586225e-16;
-    pc = __builtin_fma(pc, z, 4.779477332387385e-14);
-    pc = __builtin_fma(pc, z, -1.1470745597729725e-11);
-    pc = __builtin_fma(pc, z, 2.08767569878681e-09);
-    pc = __builtin_fma(pc, z, -2.755731922398589e-07);
-    pc = __builtin_fma(pc, z, 2.48015873015873e-05);
-    pc = __builtin_fma(pc, z, -0.001388888888888889);
+    double pc = -1.1382632258093615e-11;
+    pc = __builtin_fma(pc, z, 2.087614626607931e-09);
+    pc = __builtin_fma(pc, z, -2.7557317271718644e-07);
+    pc = __builtin_fma(pc, z, 2.4801587298765665e-05);
+    pc = __builtin_fma(pc, z, -0.0013888888888887398);
     pc = __builtin_fma(pc, z, 0.041666666666666664);
     pc = __builtin_fma(pc, z, -0.5);
     const double sr = __builtin_fma(r * z, ps, r);
     const double cr = __builtin_fma(z, pc, 1.0);
-    const int quad = (int)(long long)q & 3;
     const double a = (quad & 1) ? cr : sr, b = (quad & 1) ? sr : cr;
-    *sn = (quad & 2) ? -a : a;
-    *cs = ((quad + 1) & 2) ? -b : b;
+    *sn = __hiloint2double(__double2hiint(a) ^ ((quad << 30) & 0x80000000), __double2loint(a));
+    *cs = __hiloint2double(__double2hiint(b) ^ (((quad + 1) << 30) & 0x80000000),
+                           __double2loint(b));
+}
+
+// the same for any argument: beyond the range the device library
+__device__ __forceinline__ void qbx_sincos(double x, double *sn, double *cs)
+{
+    if (!(__builtin_fabs(x) <= QBX_SINCOS_MAX)) {
+        sincos(x, sn, cs);
+        return;
+    }
+    qbx_sincos_core(x, sn, cs);
 }
 
 // natural logarithm of a positive normal x, within a few ulp: x = m 2^e with

@@ -26,7 +26,7 @@ def test_loose_points_match_oracle(oracle_lib, kind, npoints, nrhs):
     src = QBXLayerPotentialSource(d, fine_order=4, qbx_order=2, fmm_order=6)
     pot, = src.exec_compute_potential("laplace", torch.as_tensor(dens, device="cuda"),
                                       [(pts, 0)], source_kind=kind)
-    pot = pot.cpu().numpy()
+    pot = pot.cpu().numpy().reshape(npoints, nrhs)
     g = oracle.GeometryData(d, pts, np.zeros(npoints, np.int32), max_leaf_refine_weight=512,
                             from_sep_smaller_min_nsources_cumul=30)
     for r in range(nrhs):
