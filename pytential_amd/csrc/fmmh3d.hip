@@ -514,7 +514,9 @@ __global__ void __launch_bounds__(512) kh_p2e(HD hd, TD t, int nitems, const int
 // recurrence (as radial_seq: stable for the dominant y_n, the small j_n of
 // x < n accurate to the rounding of |h_n|), Y by the column recurrences, all
 // unrolled.
-template <int PF>
+// CORE: k r is known to be within the reduced range of qbx_sincos (the device
+// library's sine for larger arguments, never reached, took 50 registers).
+template <int PF, bool CORE = false>
 __device__ __forceinline__ void s_waves_reg(double k, v3 d, cplx *F)
 {
     const double r2 = d.x * d.x + d.y * d.y + d.z * d.z;
@@ -522,7 +524,10 @@ __device__ __forceinline__ void s_waves_reg(double k, v3 d, cplx *F)
     const double r = r2 * ir;
     const double x = k * r, ix = qbx_rcp(x);
     double sn, cs;
-    qbx_sincos(x, &sn, &cs);
+    if (CORE)
+        qbx_sincos_core(x, &sn, &cs);
+    else
+        qbx_sincos(x, &sn, &cs);
     double yv[PF + 2], jv[PF + 2];
     yv[0] = -cs * ix;
     yv[1] = (-cs * ix - sn) * ix;
@@ -570,58 +575,236 @@ __device__ __forceinline__ void s_waves_reg(double k, v3 d, cplx *F)
     }
 }
 
-// P2QBXL for one density with the QBX expansion in registers (orders <= 5):
-// a wavefront per global QBX center, the center's list-1 sources dealt to
-// the lanes round-robin across the boxes.  Each lane forms a source's S
-// waves -- y_n by the forward recurrence, j_n by Miller's backward
-// recurrence from N = max(PF, x) + 10 + 4 sqrt(max(PF, x)) normalised by j_0
-// or j_1, Y by the column recurrences, all unrolled -- and adds
-// q (-1)^m S_n^{-m}(s - c) (or its nu-gradient) into its registers; the
-// lanes' sums are reduced by shuffles and lane 0 adds ik times them.
+// The sums over sources behind one center's QBX expansion, S waves only:
+// with g_n = q h_n(k r) and A_n^m = Q_n^m(z) (x + i y)^m (Q_n^m the Legendre
+// recurrence scaled to leading coefficient 1, the point on the unit sphere),
+// Y_n^m = c_n^m A_n^m and
+//   sum q h_n conj(Y_n^m) = c (xx + yy, yx - xy),
+//   sum q h_n Y_n^m       = c (xx - yy, yx + xy)
+// from the four real sums xx = sum Re g Re A, ..., yx = sum Im g Re A: two
+// multiply-adds per coefficient, and the constants c once per center.
+template <int PQ>
+struct SWaveSums {
+    cplx s0[PQ + 1];                      // m = 0: sum g_n Q_n^0
+    double t[PQ * (PQ + 1) / 2 + 1][4];   // m > 0: xx, yy, yx, xy
+    __device__ static constexpr int at(int n, int m) { return n * (n - 1) / 2 + m - 1; }
+
+    __device__ void zero()
+    {
+#pragma unroll
+        for (int n = 0; n <= PQ; ++n) s0[n] = {0.0, 0.0};
+#pragma unroll
+        for (int i = 0; i < PQ * (PQ + 1) / 2; ++i)
+#pragma unroll
+            for (int j = 0; j < 4; ++j) t[i][j] = 0.0;
+    }
+
+    __device__ __forceinline__ void add(double k, double ik, v3 d, cplx q)
+    {
+        const double r2 = d.x * d.x + d.y * d.y + d.z * d.z;
+        const double ir = qbx_rsqrt(r2);
+        const double ix = ir * ik;
+        double sn, cs;
+        qbx_sincos_core(k * (r2 * ir), &sn, &cs);
+        cplx g[PQ + 2];
+        const cplx h0 = {sn * ix, -cs * ix};
+        const cplx h1 = {(h0.x - cs) * ix, (h0.y - sn) * ix};
+        g[0] = q * h0;
+        g[1] = q * h1;
+#pragma unroll
+        for (int n = 2; n <= PQ; ++n) {
+            const double f = (2.0 * n - 1.0) * ix;
+            g[n] = {f * g[n - 1].x - g[n - 2].x, f * g[n - 1].y - g[n - 2].y};
+        }
+        const double z = d.z * ir;
+        const cplx w = {d.x * ir, d.y * ir};
+        cplx wm = w;
+#pragma unroll
+        for (int m = 0; m <= PQ; ++m) {
+            if (m > 1) wm = wm * w;
+            double a1 = 0.0, a0 = 1.0;
+#pragma unroll
+            for (int n = m; n <= PQ; ++n) {
+                if (n > m) {
+                    // Q_n = z Q_{n-1} - Q_{n-2} ((n-1)^2 - m^2) / (4 (n-1)^2 - 1)
+                    const double c = ((n - 1.0) * (n - 1.0) - (double)m * m) /
+                                     (4.0 * (n - 1.0) * (n - 1.0) - 1.0);
+                    const double a = n == m + 1 ? z : z * a0 - c * a1;
+                    a1 = a0;
+                    a0 = a;
+                }
+                if (m == 0) {
+                    if (n == 0) {
+                        s0[0] += g[0];
+                    } else {
+                        s0[n].x += g[n].x * a0;
+                        s0[n].y += g[n].y * a0;
+                    }
+                } else {
+                    const cplx A = n == m ? wm : a0 * wm;
+                    double *u = t[at(n, m)];
+                    u[0] += g[n].x * A.x;
+                    u[1] += g[n].y * A.y;
+                    u[2] += g[n].y * A.x;
+                    u[3] += g[n].x * A.y;
+                }
+            }
+        }
+    }
+
+    // (n, m), every m, into v[IDX(n, m)]
+    __device__ __forceinline__ void expansion(cplx *v) const
+    {
+        double cmm = 0.28209479177387814347;  // 1 / sqrt(4 pi)
+#pragma unroll
+        for (int m = 0; m <= PQ; ++m) {
+            if (m > 0) cmm *= -sqrt((2.0 * m + 1.0) / (2.0 * m));
+            double c = cmm;
+#pragma unroll
+            for (int n = m; n <= PQ; ++n) {
+                if (n > m) c *= sqrt((4.0 * n * n - 1.0) / ((double)n * n - (double)m * m));
+                if (m == 0) {
+                    v[IDX(n, 0)] = c * s0[n];
+                } else {
+                    const double *u = t[at(n, m)];
+                    const double sg = (m & 1) ? -c : c;
+                    v[IDX(n, m)] = {c * (u[0] + u[1]), c * (u[2] - u[3])};
+                    v[IDX(n, -m)] = {sg * (u[0] - u[1]), sg * (u[2] + u[3])};
+                }
+            }
+        }
+    }
+};
+
+// P2QBXL for one density with the QBX expansion in registers (orders <= 5, and
+// a tree whose diagonal times k is within the reduced range of the sine).
+// A block takes a group of up to GC_GROUP centers of one target box, a wave
+// per center (two or four where the group holds two or one).  The box's
+// list-1 sources pass through LDS P2Q_CH at a time, dealt to the 64 lanes of
+// every center's wave without regard to box borders: the list's source
+// counts are summed P2Q_CH entries at a time and each staged source finds its
+// box by bisection; the next chunk's loads are in flight while one is summed.
+// The lanes' sums are added by shuffles, the waves' in LDS.
+//
+// FP64 VALU bound, about 130 instructions per (center, source) pair at order
+// 3.  1.19e9 pairs (737280 sources, 163972 centers): 16.9 -> 6.6 ms.  With a
+// wave per center walking box by box, a box of 80 sources left lanes idle,
+// and 16 complex products of the waves took half of 560 instruction slots.
+constexpr int P2Q_CH = 256;
+
 template <int PQ, int DIP>
-__global__ void __launch_bounds__(64) kh_p2qbxl_reg(HD hd, TD t, int ng, const int *gcent,
-                                                    const int *c2tb, const int *starts,
-                                                    const int *lists, const double *ctrs,
-                                                    int nctr, const double *src, int ns,
-                                                    const double *str, const double *nrm,
-                                                    double *qexp)
+__global__ void __launch_bounds__(256) kh_p2qbxl_reg(HD hd, TD t, const int *ubox,
+                                                     const int *uc0, const int *gcs,
+                                                     const int *gcl, const int *starts,
+                                                     const int *lists, const double *ctrs,
+                                                     int nctr, const double *src, int ns,
+                                                     const double *str, const double *nrm,
+                                                     double *qexp)
 {
     constexpr int PF = PQ + DIP;
     constexpr int NC = (PQ + 1) * (PQ + 1);
     constexpr int NF = (PF + 1) * (PF + 1);
-    const int g = blockIdx.x;
-    if (g >= ng) return;
-    const int ci = gcent[g];
-    const int tb = c2tb[ci];
-    const v3 c = ld3(ctrs, nctr, ci);
-    const int lane = threadIdx.x;
-    const double k = hd.k;
+    __shared__ double2 sxy[P2Q_CH], szq[P2Q_CH];      // x, y; z, Re q
+    __shared__ double sqi[P2Q_CH];
+    __shared__ double snu[DIP ? 3 * P2Q_CH : 1];
+    __shared__ int pre[P2Q_CH + 1], first[P2Q_CH], wsum[4];
+    __shared__ double red[4 * 2 * NC];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int it = ubox[blockIdx.x];
+    const int c0 = gcs[it] + uc0[blockIdx.x];
+    const int ncen = min(GC_GROUP, gcs[it + 1] - c0);
+    // waves per center; wave -> center and share
+    const int wpc = ncen == 1 ? 4 : ncen == 2 ? 2 : 1;
+    const int cw = wave / wpc, share = wave % wpc;
+    const bool act = cw < ncen;
+    const int ci = act ? gcl[c0 + cw] : 0;
+    const v3 c = act ? ld3(ctrs, nctr, ci) : v3{0, 0, 0};
+    const double k = hd.k, ik = 1.0 / k;
+    SWaveSums<PQ> A;
     cplx acc[NC];
+    if (DIP) {
 #pragma unroll
-    for (int i = 0; i < NC; ++i) acc[i] = {0.0, 0.0};
-    int base = 0;
-    for (int e = starts[tb]; e < starts[tb + 1]; ++e) {
-        const int Sb = lists[e];
-        const int s0 = t.sstart[Sb], cnt = t.scount[Sb];
-        for (int j = (lane - (base & 63) + 64) & 63; j < cnt; j += 64) {
-            const int si = s0 + j;
-            const v3 d = sub(ld3(src, ns, si), c);
-            cplx F[NF];
-            s_waves_reg<PF>(k, d, F);
-            const cplx qs = ldc(str + 2 * ((size_t)si * hd.nr + hd.r0));
-            v3 nu = {0.0, 0.0, 0.0};
-            if (DIP) nu = ld3(nrm, ns, si);
-#pragma unroll
-            for (int n = 0; n <= PQ; ++n)
-#pragma unroll
-                for (int m = -n; m <= n; ++m) {
-                    cplx fv = DIP ? nu_grad(F, PF, k, n, -m, nu) : F[IDX(n, -m)];
-                    if (m & 1) fv = -fv;
-                    acc[IDX(n, m)] += qs * fv;
-                }
-        }
-        base += cnt;
+        for (int i = 0; i < NC; ++i) acc[i] = {0.0, 0.0};
+    } else {
+        A.zero();
     }
+    const int e1 = starts[it + 1];
+    for (int e0 = starts[it]; e0 < e1; e0 += P2Q_CH) {
+        // the entries' first sources and running counts
+        const int e = e0 + tid;
+        int cnt = 0;
+        if (e < e1) {
+            const int Sb = lists[e];
+            cnt = t.scount[Sb];
+            first[tid] = t.sstart[Sb];
+        }
+        int run = cnt;
+        for (int o = 1; o < 64; o <<= 1) {
+            const int y = __shfl_up(run, o);
+            if (lane >= o) run += y;
+        }
+        if (lane == 63) wsum[wave] = run;
+        __syncthreads();
+        for (int w = 0; w < wave; ++w) run += wsum[w];
+        pre[tid + 1] = run;
+        if (tid == 0) pre[0] = 0;
+        __syncthreads();
+        const int total = pre[P2Q_CH];
+        double2 rxy = {0, 0}, rzq = {0, 0};
+        double rqi = 0;
+        v3 rnu = {0, 0, 0};
+        auto fetch = [&](int v) {
+            if (v >= total) return;
+            int lo = 0, hi = P2Q_CH;   // pre[lo] <= v < pre[hi]
+            while (hi - lo > 1) {
+                const int mid = (lo + hi) >> 1;
+                if (pre[mid] <= v) lo = mid; else hi = mid;
+            }
+            const int si = first[lo] + v - pre[lo];
+            const double *q = str + 2 * ((size_t)si * hd.nr + hd.r0);
+            rxy = {src[si], src[(size_t)ns + si]};
+            rzq = {src[2 * (size_t)ns + si], q[0]};
+            rqi = q[1];
+            if (DIP) rnu = ld3(nrm, ns, si);
+        };
+        fetch(tid);
+        for (int v0 = 0; v0 < total; v0 += P2Q_CH) {
+            sxy[tid] = rxy;
+            szq[tid] = rzq;
+            sqi[tid] = rqi;
+            if (DIP) {
+                snu[tid] = rnu.x;
+                snu[P2Q_CH + tid] = rnu.y;
+                snu[2 * P2Q_CH + tid] = rnu.z;
+            }
+            __syncthreads();
+            fetch(v0 + P2Q_CH + tid);
+            const int n = min(P2Q_CH, total - v0);
+            if (act)
+                for (int j = share * 64 + lane; j < n; j += 64 * wpc) {
+                    const double2 xy = sxy[j], zq = szq[j];
+                    const v3 d = {xy.x - c.x, xy.y - c.y, zq.x - c.z};
+                    const cplx qs = {zq.y, sqi[j]};
+                    if (DIP) {
+                        cplx F[NF];
+                        s_waves_reg<PF, true>(k, d, F);
+                        const v3 nu = {snu[j], snu[P2Q_CH + j], snu[2 * P2Q_CH + j]};
+#pragma unroll
+                        for (int nn = 0; nn <= PQ; ++nn)
+#pragma unroll
+                            for (int m = -nn; m <= nn; ++m) {
+                                cplx fv = nu_grad(F, PF, k, nn, -m, nu);
+                                if (m & 1) fv = -fv;
+                                acc[IDX(nn, m)] += qs * fv;
+                            }
+                    } else {
+                        A.add(k, ik, d, qs);
+                    }
+                }
+            __syncthreads();
+        }
+    }
+    if (!DIP) A.expansion(acc);
 #pragma unroll
     for (int i = 0; i < NC; ++i)
 #pragma unroll
@@ -629,15 +812,22 @@ __global__ void __launch_bounds__(64) kh_p2qbxl_reg(HD hd, TD t, int ng, const i
             acc[i].x += __shfl_xor(acc[i].x, off);
             acc[i].y += __shfl_xor(acc[i].y, off);
         }
-    if (lane == 0) {
-        const cplx ik = {0.0, k};
+    if (lane == 0)
 #pragma unroll
         for (int i = 0; i < NC; ++i) {
-            double *dst = qexp + 2 * (((size_t)ci * NC + i) * hd.nr + hd.r0);
-            const cplx v = ik * acc[i];
-            dst[0] += v.x;
-            dst[1] += v.y;
+            red[2 * (wave * NC + i)] = acc[i].x;
+            red[2 * (wave * NC + i) + 1] = acc[i].y;
         }
+    __syncthreads();
+    if (act && share == 0 && lane < NC) {
+        cplx v = {0.0, 0.0};
+        for (int w = wave; w < wave + wpc; ++w)
+            v += cplx{red[2 * (w * NC + lane)], red[2 * (w * NC + lane) + 1]};
+        const cplx ikv = {0.0, k};
+        v = ikv * v;
+        double *dst = qexp + 2 * (((size_t)ci * NC + lane) * hd.nr + hd.r0);
+        dst[0] += v.x;
+        dst[1] += v.y;
     }
 }
 
@@ -2667,17 +2857,18 @@ int h3_form_global_qbx_locals(qbx_ctx *ctx, void *stream, const qbx_tree *T,
     if (G->nglobal == 0) return QBX_OK;
     QBX_CHECK(G->trav == R, "P2QBXL: geometry was built for another traversal");
     const TD td = make_td(T);
-    if (hd.pq <= 5) {
+    // no source is farther from a center than the root box's diagonal
+    if (hd.pq <= 5 && std::fabs(hd.k) * 1.75 * hd.h[0] <= QBX_SINCOS_MAX) {
         // the expansion in registers, one density per launch
-        const int ng = G->nglobal;
+        const unit_plan &U = G->gc_group_plan;
         for (int r0 = 0; r0 < hd.nr; ++r0) {
             hd.r0 = r0;
             hd.rc = 1;
 #define H3_PQR(PQV, DV)                                                                    \
-    hipLaunchKernelGGL((kh_p2qbxl_reg<PQV, DV>), dim3(ng), dim3(64), 0, st, hd, td, ng,    \
-                       G->global_qbx_centers.p, G->center_to_target_box.p, R->l1_starts.p, \
-                       R->l1_lists.p, G->centers.p, G->ncenters, T->sources.p, T->nsources, \
-                       str, nrm, qexp)
+    hipLaunchKernelGGL((kh_p2qbxl_reg<PQV, DV>), dim3(U.nunits), dim3(256), 0, st, hd, td, \
+                       U.unit_box.p, U.unit_t0.p, G->gc_by_tbox_starts.p, G->gc_by_tbox.p, \
+                       R->l1_starts.p, R->l1_lists.p, G->centers.p, G->ncenters,           \
+                       T->sources.p, T->nsources, str, nrm, qexp)
 #define H3_PQD(PQV)          \
     if (hd.dip)              \
         H3_PQR(PQV, 1);      \
