@@ -145,43 +145,6 @@ __device__ __forceinline__ cplx neg_m(cplx v, int am)  // (-1)^m conj(v)
     return (am & 1) ? cplx{-v.x, v.y} : cplx{v.x, -v.y};
 }
 
-// single Y_n^m(d), O(n)
-__device__ cplx ups_nm(int n, int m, v3 d)
-{
-    const int am = m < 0 ? -m : m;
-    if (am > n || n < 0) return {0, 0};
-    const double r2 = d.x * d.x + d.y * d.y + d.z * d.z;
-    const cplx hw = {-0.5 * d.x, -0.5 * d.y};
-    cplx b = {1, 0}, a = {0, 0};
-    for (int i = 1; i <= am; ++i) b = (1.0 / i) * (b * hw);
-    for (int k = am + 1; k <= n; ++k) {
-        const cplx c =
-            (1.0 / ((double)(k - am) * (k + am))) * (((2.0 * k - 1.0) * d.z) * b - r2 * a);
-        a = b;
-        b = c;
-    }
-    return m < 0 ? neg_m(b, am) : b;
-}
-
-// single T_n^m(d), O(n)
-__device__ cplx the_nm(int n, int m, v3 d)
-{
-    const int am = m < 0 ? -m : m;
-    if (am > n || n < 0) return {0, 0};
-    const double r2 = d.x * d.x + d.y * d.y + d.z * d.z;
-    const double ir2 = 1.0 / r2;
-    const cplx w = {d.x * ir2, d.y * ir2};
-    cplx b = {sqrt(ir2), 0}, a = {0, 0};
-    for (int i = 1; i <= am; ++i) b = (-(2.0 * i - 1.0)) * (b * w);
-    for (int k = am + 1; k <= n; ++k) {
-        const cplx c = ir2 * (((2.0 * k - 1.0) * d.z) * b -
-                              ((double)(k + am - 1) * (k - am - 1)) * a);
-        a = b;
-        b = c;
-    }
-    return m < 0 ? neg_m(b, am) : b;
-}
-
 // full table T_n^m(d), n <= P, in registers
 template <int P>
 __device__ __forceinline__ void the_table(v3 d, cplx *T)
@@ -279,22 +242,6 @@ __device__ __forceinline__ double p2p_value(const KD &kd, v3 s, v3 nu, v3 t)
     return INV4PI * ir * ir * ir * (nu.x * d.x + nu.y * d.y + nu.z * d.z);
 }
 
-// coefficient (n, m) one unit-strength source contributes to a multipole
-// (local = 0) or local (1)
-__device__ __forceinline__ cplx p2e_basis(const KD &kd, int local, int n, int m, v3 d, v3 nu)
-{
-    if (!kd.dip) return local ? the_nm(n, m, d) : conj(ups_nm(n, m, d));
-    const cplx nm = {nu.x, -nu.y}, np = {nu.x, nu.y};
-    cplx g;
-    if (local)
-        g = (-nu.z) * the_nm(n + 1, m, d) +
-            0.5 * (nm * the_nm(n + 1, m + 1, d) - np * the_nm(n + 1, m - 1, d));
-    else
-        g = nu.z * ups_nm(n - 1, m, d) +
-            0.5 * (nm * ups_nm(n - 1, m + 1, d) - np * ups_nm(n - 1, m - 1, d));
-    return local ? g : conj(g);
-}
-
 template <int NRC>
 __device__ __forceinline__ void store_add(const KD &kd, double *o, const cplx *acc)
 {
@@ -306,253 +253,43 @@ __device__ __forceinline__ void store_add(const KD &kd, double *o, const cplx *a
         }
 }
 
-// P2M over source boxes: thread per (box, coefficient)
-template <int NRC>
-__global__ void k3_p2m(KD kd, TD t, Flat fl, const int *boxes, const double *src, int ns,
-                       const double *str, const double *nrm, double *mpole)
-{
-    const long gid = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    int lv, i, j;
-    if (!flat_locate(fl, gid, lv, i, j)) return;
-    const int b = boxes[i];
-    int n, m;
-    nm_of(j, n, m);
-    const v3 c = boxc(t, b);
-    const int s0 = t.sstart[b], s1 = s0 + t.scount[b];
-    cplx acc[NRC];
-#pragma unroll
-    for (int q = 0; q < NRC; ++q) acc[q] = {0, 0};
-    for (int s = s0; s < s1; ++s) {
-        const v3 nu = kd.dip ? ld3(nrm, ns, s) : v3{0, 0, 0};
-        const cplx bs = p2e_basis(kd, 0, n, m, sub(ld3(src, ns, s), c), nu);
-#pragma unroll
-        for (int q = 0; q < NRC; ++q)
-            if (q < kd.rc) acc[q] += ldq(kd, str, s, kd.r0 + q) * bs;
-    }
-    double *o = mpole + ecoef_off(kd, b, lv) + 2L * j * kd.nr;
-#pragma unroll
-    for (int q = 0; q < NRC; ++q)
-        if (q < kd.rc) stc(o + 2 * (kd.r0 + q), acc[q]);
-}
-
-// P2L over list 4: thread per (ttp box, coefficient), accumulating
-template <int NRC>
-__global__ void k3_p2l(KD kd, TD t, Flat fl, const int *ttp, const int *starts, const int *lists,
-                       const double *src, int ns, const double *str, const double *nrm,
-                       double *local)
-{
-    const long gid = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    int lv, i, j;
-    if (!flat_locate(fl, gid, lv, i, j)) return;
-    const int e0 = starts[i], e1 = starts[i + 1];
-    if (e0 == e1) return;
-    const int b = ttp[i];
-    int n, m;
-    nm_of(j, n, m);
-    const v3 c = boxc(t, b);
-    cplx acc[NRC];
-#pragma unroll
-    for (int q = 0; q < NRC; ++q) acc[q] = {0, 0};
-    for (int e = e0; e < e1; ++e) {
-        const int S = lists[e];
-        const int s0 = t.sstart[S], s1 = s0 + t.scount[S];
-        for (int s = s0; s < s1; ++s) {
-            const v3 nu = kd.dip ? ld3(nrm, ns, s) : v3{0, 0, 0};
-            const cplx bs = p2e_basis(kd, 1, n, m, sub(ld3(src, ns, s), c), nu);
-#pragma unroll
-            for (int q = 0; q < NRC; ++q)
-                if (q < kd.rc) acc[q] += ldq(kd, str, s, kd.r0 + q) * bs;
-        }
-    }
-    store_add<NRC>(kd, local + ecoef_off(kd, b, lv) + 2L * j * kd.nr, acc);
-}
-
-// P2M / P2L through LDS, one block per box, sources S at a time.  Phase A
-// (one lane per source) computes the source's harmonic table once, m >= 0
-// half: Y_n^m(s - c) for n <= p (multipoles) or T_n^m(s - c) for n <= p + 1
-// (locals, the dipole needs n + 1), at ht[s][n(n+1)/2 + m]; phase B (one lane
-// per coefficient (n, m)) sums q_s b_nm(s) over the chunk, with the negative
-// orders from (-1)^m conj and the dipole rules of p2e_basis.  O(p^2) work per
-// source instead of O(p^3) from one harmonic per thread and source.
-struct P2EShape3 {
-    int S;  // sources per chunk
-    int R;  // row stride (complex entries, odd) >= (pt+1)(pt+2)/2
-    __host__ __device__ int doubles(int nrc) const { return 2 * S * R + 2 * S * nrc + 3 * S + S; }
+// P2M and P2L, a block per box, on the FP64 matrix cores for any number of
+// densities.  S sources at a time (the box's own, or those of its list-4
+// boxes, dealt without regard to box borders) the block forms the harmonics
+// of source - center once, real rows H[n^2 + 2m - 1 or + 2m][source] (Re, Im
+// of Y_n^m or T_n^m, m >= 0, n <= pt), and stages real weights: each
+// density's strength (S), or the strength times each component of the source
+// normal (D), real parts in one tile of 16 columns and imaginary parts in
+// another that is skipped while they are all zero (up to 8 weights: both in
+// one tile).  U = H weights, then the coefficients: the negative orders from
+// (-1)^m conj, and for D
+//   P2L: -U_z(n+1,m) + ((U_x - i U_y)(n+1,m+1) - (U_x + i U_y)(n+1,m-1)) / 2
+//   P2M: conj of U_z(n-1,m) + ((U_x - i U_y)(n-1,m+1) - (U_x + i U_y)(n-1,m-1)) / 2.
+// The waves split the row tiles RG ways and the sources 4 / RG ways; their
+// sums meet in LDS.  Bound by the tables' recurrences and the latency of a
+// step's loads at two blocks a CU (216 registers), not by the matrix cores.
+//
+// Row stride S + 2 doubles (even, and odd multiples of 2 mod 32 banks): the
+// harmonics are written along the sources and read down the rows without
+// bank conflicts.
+//
+// The one-lane-per-source tables and the gathered operands of the kernels
+// before kept most lanes waiting: 14.8e6 (box, source) pairs at order 8 with
+// 32 real densities (91 GFLOP here) took 13.9 ms, now 5.0; 1.06e6 pairs,
+// one dipole density at order 10, 4.3 ms, now 0.88.
+struct P2EShape {
+    int S, SS, rows, RT, RG, RTW, NB, pt;
+    size_t bytes;
 };
 
-__device__ __forceinline__ int tri(int n, int m) { return n * (n + 1) / 2 + m; }
-
-// the source's table for k3_p2e: h[tri(n, m)], m >= 0, n <= pt, of d = source -
-// center -- irregular harmonics (LOCAL) or regular ones (multipoles), by the
-// recurrences in m and n
-template <bool LOCAL>
-__device__ __forceinline__ void p2e3_table(v3 d, int pt, double *h)
-{
-    const double r2 = d.x * d.x + d.y * d.y + d.z * d.z;
-    if (LOCAL) {
-        const double ir2 = 1.0 / r2;
-        const cplx w = {d.x * ir2, d.y * ir2};
-        cplx tmm = {sqrt(ir2), 0};
-        for (int mm = 0; mm <= pt; ++mm) {
-            if (mm > 0) tmm = (-(2.0 * mm - 1.0)) * (tmm * w);
-            cplx a = {0, 0}, b = tmm;
-            stc(h + 2 * tri(mm, mm), b);
-            for (int nn = mm + 1; nn <= pt; ++nn) {
-                const cplx cc = ir2 * (((2.0 * nn - 1.0) * d.z) * b -
-                                       ((double)(nn + mm - 1) * (nn - mm - 1)) * a);
-                stc(h + 2 * tri(nn, mm), cc);
-                a = b;
-                b = cc;
-            }
-        }
-    } else {
-        const cplx hw = {-0.5 * d.x, -0.5 * d.y};
-        cplx ymm = {1, 0};
-        for (int mm = 0; mm <= pt; ++mm) {
-            if (mm > 0) ymm = (1.0 / mm) * (ymm * hw);
-            cplx a = {0, 0}, b = ymm;
-            stc(h + 2 * tri(mm, mm), b);
-            for (int nn = mm + 1; nn <= pt; ++nn) {
-                const cplx cc = (1.0 / ((double)(nn - mm) * (nn + mm))) *
-                                (((2.0 * nn - 1.0) * d.z) * b - r2 * a);
-                stc(h + 2 * tri(nn, mm), cc);
-                a = b;
-                b = cc;
-            }
-        }
-    }
-}
-
-template <int NRC, bool LOCAL>
-__global__ void __launch_bounds__(512) k3_p2e(KD kd, TD t, int lv, int i0, P2EShape3 sh,
-                                               const int *boxes, const int *starts,
-                                               const int *lists, const double *src, int ns,
-                                               const double *str, const double *nrm,
-                                               double *expn)
-{
-    extern __shared__ double lds[];
-    const int i = i0 + blockIdx.x;
-    const int Bx = boxes[i];
-    int e0 = 0, e1 = 1;
-    if (LOCAL) {
-        e0 = starts[i];
-        e1 = starts[i + 1];
-        if (e0 == e1) return;
-    }
-    const int p = kd.order[lv];
-    const int pt = LOCAL ? p + 1 : p;
-    const int S = sh.S, R = sh.R;
-    double *Ht = lds, *Qs = Ht + 2 * S * R, *Nu = Qs + 2 * S * NRC;
-    int *idx = (int *)(Nu + 3 * S);
-    const int tid = threadIdx.x, nth = blockDim.x;
-    const bool dip = kd.dip;
-    const int rc = kd.rc, r0 = kd.r0, nr = kd.nr;
-    const v3 c = boxc(t, Bx);
-    const bool act = tid < (p + 1) * (p + 1);
-    int n = 0, m = 0;
-    if (act) nm_of(tid, n, m);
-    cplx acc[NRC];
-#pragma unroll
-    for (int q = 0; q < NRC; ++q) acc[q] = {0, 0};
-
-    // table entry (nn, mm) of staged source sl, any sign of mm, zero outside
-    auto hval = [&](int sl, int nn, int mm) -> cplx {
-        const int am = mm < 0 ? -mm : mm;
-        if (nn < 0 || am > nn) return {0, 0};
-        const cplx v = {Ht[2 * (sl * R + tri(nn, am))], Ht[2 * (sl * R + tri(nn, am)) + 1]};
-        return mm < 0 ? neg_m(v, am) : v;
-    };
-
-    auto flush = [&](int cnt) {
-        __syncthreads();
-        if (tid < cnt) {
-            const int si = idx[tid];
-            p2e3_table<LOCAL>(sub(ld3(src, ns, si), c), pt, Ht + 2 * tid * R);
-#pragma unroll
-            for (int q = 0; q < NRC; ++q)
-                if (q < rc) {
-                    const double *pq = str + 2 * ((size_t)si * nr + r0 + q);
-                    Qs[2 * (tid * NRC + q)] = pq[0];
-                    Qs[2 * (tid * NRC + q) + 1] = pq[1];
-                }
-            if (dip) {
-                Nu[3 * tid] = nrm[si];
-                Nu[3 * tid + 1] = nrm[(size_t)ns + si];
-                Nu[3 * tid + 2] = nrm[2 * (size_t)ns + si];
-            }
-        }
-        __syncthreads();
-        if (act)
-            for (int sl = 0; sl < cnt; ++sl) {
-                cplx b;
-                if (!dip) {
-                    b = LOCAL ? hval(sl, n, m) : conj(hval(sl, n, m));
-                } else {
-                    const double nx = Nu[3 * sl], ny = Nu[3 * sl + 1], nz = Nu[3 * sl + 2];
-                    const cplx nmn = {nx, -ny}, npl = {nx, ny};
-                    if (LOCAL) {
-                        b = (-nz) * hval(sl, n + 1, m) +
-                            0.5 * (nmn * hval(sl, n + 1, m + 1) - npl * hval(sl, n + 1, m - 1));
-                    } else {
-                        b = conj(nz * hval(sl, n - 1, m) +
-                                 0.5 * (nmn * hval(sl, n - 1, m + 1) -
-                                        npl * hval(sl, n - 1, m - 1)));
-                    }
-                }
-#pragma unroll
-                for (int q = 0; q < NRC; ++q)
-                    if (q < rc)
-                        acc[q] += cplx{Qs[2 * (sl * NRC + q)], Qs[2 * (sl * NRC + q) + 1]} * b;
-            }
-    };
-
-    int fill = 0;
-    for (int e = e0; e < e1; ++e) {
-        const int Sb = LOCAL ? lists[e] : Bx;
-        int s = t.sstart[Sb];
-        const int s1 = s + t.scount[Sb];
-        while (s < s1) {
-            const int take = min(s1 - s, S - fill);
-            for (int j = tid; j < take; j += nth) idx[fill + j] = s + j;
-            fill += take;
-            s += take;
-            if (fill == S) {
-                flush(S);
-                fill = 0;
-            }
-        }
-    }
-    if (fill > 0) flush(fill);
-    if (act) {
-        double *o = expn + ecoef_off(kd, Bx, lv) + 2L * tid * nr;
-#pragma unroll
-        for (int q = 0; q < NRC; ++q)
-            if (q < rc) {
-                double *pq = o + 2 * (r0 + q);
-                stc(pq, LOCAL ? ldc(pq) + acc[q] : acc[q]);
-            }
-    }
-}
-
-// P2M / P2L for many right-hand sides on the FP64 matrix cores: the sources
-// of the box (P2M) or of its list-4 boxes (P2L) are staged P2E3M_S at a time
-// with their tables (p2e3_table) and the strengths of up to 16 right-hand
-// sides; out[(n,m)][r] (+)= sum_s b_(n,m)(s) q_s[r] with b as in k3_p2e
-// (single or double layer) is a complex product: rows the coefficients
-// (wave w takes the 16-row tiles w, w + 4, ...), k the staged sources.
-constexpr int P2E3M_S = 32;
-constexpr int P2E3M_RTW = 4;  // (p + 1)^2 <= 256
-
-template <bool LOCAL>
+template <bool LOCAL, bool DIP, int NB, int RTW>
 __global__ void __launch_bounds__(256)
-k3_p2e_mfma(KD kd, TD t, int lv, int i0, int R, const int *boxes, const int *starts,
-            const int *lists, const double *src, int ns, const double *str, const double *nrm,
-            double *expn)
+k3_p2e(KD kd, TD t, int i0, P2EShape sh, const int *boxes, const int *starts,
+       const int *lists, const double *src, int ns, const double *str, const double *nrm,
+       double *expn)
 {
     extern __shared__ double lds[];
-    double *Ht = lds, *Qs = Ht + 2 * P2E3M_S * R, *Nu = Qs + 2 * P2E3M_S * 16;
-    int *idx = (int *)(Nu + 3 * P2E3M_S);
-    __shared__ short nof[256], mof[256];
+    __shared__ int pre[257], first[256], wsum[4], idx[2][32];
     const int i = i0 + blockIdx.x;
     const int Bx = boxes[i];
     int e0 = 0, e1 = 1;
@@ -561,127 +298,244 @@ k3_p2e_mfma(KD kd, TD t, int lv, int i0, int R, const int *boxes, const int *sta
         e1 = starts[i + 1];
         if (e0 == e1) return;
     }
-    const int p = kd.order[lv];
-    const int pt = LOCAL ? p + 1 : p;
-    const int nout = (p + 1) * (p + 1);
-    const int RT = (nout + 15) / 16;
+    const int lv = t.level[Bx], p = kd.order[lv], pt = sh.pt;
+    const int S = sh.S, SS = sh.SS, RT = sh.RT, RG = sh.RG, KG = 4 / RG;
+    double *H = lds, *W = H + RT * 16 * SS;          // W[S][2 NB 16]
+    constexpr int WC = 2 * NB * 16, ND = DIP ? 3 : 1;
     const int tid = threadIdx.x, wv = tid >> 6, lane = tid & 63;
     const int col = lane & 15, kr = lane >> 4;
-    const bool dip = kd.dip;
-    const int rc = kd.rc, r0 = kd.r0, nr = kd.nr;
+    const int rg = wv / KG, kg = wv % KG;
+    const int nr = kd.nr, rc = kd.rc, r0 = kd.r0;
+    const bool pack = NB == 1 && ND * rc <= 8;
     const v3 c = boxc(t, Bx);
-    {
-        int n = (int)sqrt((double)tid);
-        while (n * n > tid) --n;
-        while ((n + 1) * (n + 1) <= tid) ++n;
-        nof[tid] = (short)n;
-        mof[tid] = (short)(tid - n * n - n);
-    }
-    f3_d4 cre[P2E3M_RTW], cim[P2E3M_RTW];
+    f3_d4 acc[RTW][2 * NB];
 #pragma unroll
-    for (int q = 0; q < P2E3M_RTW; ++q) cre[q] = cim[q] = f3_d4{0, 0, 0, 0};
+    for (int a = 0; a < RTW; ++a)
+#pragma unroll
+        for (int b = 0; b < 2 * NB; ++b) acc[a][b] = f3_d4{0, 0, 0, 0};
+    // rows beyond the table stay zero
+    for (int e = sh.rows * SS + tid; e < RT * 16 * SS; e += 256) H[e] = 0.0;
 
-    auto hval = [&](int sl, int nn, int mm) -> cplx {
-        const int am = mm < 0 ? -mm : mm;
-        if (nn < 0 || am > nn) return {0, 0};
-        const cplx v = {Ht[2 * (sl * R + tri(nn, am))], Ht[2 * (sl * R + tri(nn, am)) + 1]};
-        return mm < 0 ? neg_m(v, am) : v;
-    };
-
-    auto flush = [&](int cnt) {
+    for (int eb = e0; eb < e1; eb += 256) {
+        const int e = eb + tid;
+        int cnt = 0;
+        if (e < e1) {
+            const int Sb = LOCAL ? lists[e] : Bx;
+            cnt = t.scount[Sb];
+            first[tid] = t.sstart[Sb];
+        }
+        int run = cnt;
+        for (int o = 1; o < 64; o <<= 1) {
+            const int y = __shfl_up(run, o);
+            if (lane >= o) run += y;
+        }
+        if (lane == 63) wsum[wv] = run;
         __syncthreads();
-        if (tid < cnt) {
-            const int si = idx[tid];
-            p2e3_table<LOCAL>(sub(ld3(src, ns, si), c), pt, Ht + 2 * tid * R);
-            if (dip) {
-                Nu[3 * tid] = nrm[si];
-                Nu[3 * tid + 1] = nrm[(size_t)ns + si];
-                Nu[3 * tid + 2] = nrm[2 * (size_t)ns + si];
+        for (int w = 0; w < wv; ++w) run += wsum[w];
+        pre[tid + 1] = run;
+        if (tid == 0) pre[0] = 0;
+        __syncthreads();
+        const int total = pre[256];
+        // the source of the chunk's place v (the last one again beyond the end)
+        auto source = [&](int v) {
+            v = min(v, total - 1);
+            int lo = 0, hi = 256;
+            while (hi - lo > 1) {
+                const int mid = (lo + hi) >> 1;
+                if (pre[mid] <= v) lo = mid; else hi = mid;
             }
-        }
-        int imag = 0;
-        for (int e = tid; e < P2E3M_S * 16; e += 256) {
-            const int k = e >> 4, r = e & 15;
-            double vr = 0.0, vi = 0.0;
-            if (k < cnt && r < rc) {
-                const double *pq = str + 2 * ((size_t)idx[k] * nr + r0 + r);
-                vr = pq[0];
-                vi = pq[1];
-            }
-            imag |= vi != 0.0;
-            Qs[2 * e] = vr;
-            Qs[2 * e + 1] = vi;
-        }
-        // real strengths (a real density): the products with the zero
-        // imaginary parts are skipped (block-uniform)
-        imag = __syncthreads_or(imag);
-        for (int ks = 0; ks < P2E3M_S / 4; ++ks) {
-            const int sl = ks * 4 + kr;
-            const double bre = Qs[2 * (sl * 16 + col)], bim = Qs[2 * (sl * 16 + col) + 1];
+            return first[lo] + v - pre[lo];
+        };
+        if (total == 0) continue;
+        // a chunk's points and weights pass through registers: the next
+        // chunk's are loaded while this one's are multiplied
+        constexpr int NW = NB * 2;               // weights of a thread (S <= 32)
+        const int s = tid & (S - 1), g = tid / S, ng = 256 / S;
+        v3 x;
+        double wr[NW], wi[NW];
+        auto fetch = [&](int v0, const int *ix) {
+            x = ld3(src, ns, ix[s]);
+            const int n_ = min(S, total - v0);
 #pragma unroll
-            for (int q = 0; q < P2E3M_RTW; ++q) {
-                const int rt = wv + 4 * q;
-                if (rt < RT) {
-                    const int row = rt * 16 + col;
-                    cplx a = {0, 0};
-                    if (row < nout && sl < cnt) {
-                        const int n = nof[row], m = mof[row];
-                        if (!dip) {
-                            a = LOCAL ? hval(sl, n, m) : conj(hval(sl, n, m));
+            for (int u = 0; u < NW; ++u) {
+                const int e2 = tid + 256 * u, k = e2 / (NB * 16), cc = e2 % (NB * 16);
+                // 16 / ND densities to a tile of 16 columns
+                const int in = pack ? cc & 7 : cc & 15, dir = in % ND;
+                const int r = (cc >> 4) * (16 / ND) + in / ND;
+                wr[u] = wi[u] = 0.0;
+                if (k < n_ && r < rc && in / ND < 16 / ND) {
+                    const int si = ix[k];
+                    const double *q = str + 2 * ((size_t)si * nr + r0 + r);
+                    const double f = DIP ? nrm[(size_t)dir * ns + si] : 1.0;
+                    wr[u] = f * q[0];
+                    wi[u] = f * q[1];
+                }
+            }
+        };
+        if (tid < S) {
+            idx[0][tid] = source(tid);
+            idx[1][tid] = source(S + tid);
+        }
+        __syncthreads();
+        fetch(0, idx[0]);
+        for (int v0 = 0, buf = 1; v0 < total; v0 += S, buf ^= 1) {
+            // harmonics: thread (source s, orders m = g, g + 256 / S, ...)
+            {
+                const v3 d = sub(x, c);
+                const double r2 = d.x * d.x + d.y * d.y + d.z * d.z;
+                double ir2 = 0.0;
+                cplx w, mm = {1.0, 0.0};
+                if (LOCAL) {
+                    const double ir = qbx_rsqrt(r2);
+                    ir2 = ir * ir;
+                    w = {d.x * ir2, d.y * ir2};
+                    mm = {ir, 0.0};
+                } else {
+                    w = {-0.5 * d.x, -0.5 * d.y};
+                }
+                const double z2 = 2.0 * d.z;
+                int m = 0;
+                for (int mt = g; mt <= pt; mt += ng) {
+                    while (m < mt) {
+                        ++m;
+                        mm = LOCAL ? (-(2.0 * m - 1.0)) * (mm * w) : qbx_rcp(m) * (mm * w);
+                    }
+                    const double m2 = (double)(m * m);
+                    cplx a = {0, 0}, b = mm;
+                    double z = (2.0 * m - 1.0) * d.z, k1 = m;   // (2n-1) d.z, n
+                    double *h = H + (m * m + (m > 0 ? 2 * m - 1 : 0)) * SS + s;
+                    for (int n = m;;) {
+                        h[0] = b.x;
+                        if (m > 0) h[SS] = b.y;
+                        if (++n > pt) break;
+                        z += z2;
+                        cplx v;
+                        if (LOCAL) {
+                            // (n + m - 1) (n - m - 1) = (n - 1)^2 - m^2
+                            v = ir2 * (z * b - (k1 * k1 - m2) * a);
+                            k1 += 1.0;
                         } else {
-                            const double nx = Nu[3 * sl], ny = Nu[3 * sl + 1], nz = Nu[3 * sl + 2];
-                            const cplx nmn = {nx, -ny}, npl = {nx, ny};
-                            if (LOCAL)
-                                a = (-nz) * hval(sl, n + 1, m) +
-                                    0.5 * (nmn * hval(sl, n + 1, m + 1) -
-                                           npl * hval(sl, n + 1, m - 1));
-                            else
-                                a = conj(nz * hval(sl, n - 1, m) +
-                                         0.5 * (nmn * hval(sl, n - 1, m + 1) -
-                                                npl * hval(sl, n - 1, m - 1)));
+                            k1 += 1.0;
+                            v = qbx_rcp(k1 * k1 - m2) * (z * b - r2 * a);
+                        }
+                        a = b;
+                        b = v;
+                        h += (2 * n - 1) * SS;
+                    }
+                }
+            }
+            int imag = 0;
+#pragma unroll
+            for (int u = 0; u < NW; ++u) {
+                const int e2 = tid + 256 * u, k = e2 / (NB * 16), cc = e2 % (NB * 16);
+                if (k >= S) continue;
+                if (pack) {
+                    W[k * WC + cc] = cc < 8 ? wr[u] : wi[u];
+                } else {
+                    imag |= wi[u] != 0.0;
+                    W[k * WC + cc] = wr[u];
+                    W[k * WC + NB * 16 + cc] = wi[u];
+                }
+            }
+            imag = __syncthreads_or(imag);
+            if (v0 + S < total) fetch(v0 + S, idx[buf]);
+            for (int ks = kg; ks < S / 4; ks += KG) {
+                const int k = ks * 4 + kr;
+                double b[2 * NB];
+#pragma unroll
+                for (int j = 0; j < 2 * NB; ++j) b[j] = W[k * WC + j * 16 + col];
+#pragma unroll
+                for (int a = 0; a < RTW; ++a) {
+                    const int rt = rg * RTW + a;
+                    if (rt < RT) {
+                        const double h = H[(rt * 16 + col) * SS + k];
+#pragma unroll
+                        for (int j = 0; j < NB; ++j) {
+                            acc[a][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(h, b[j], acc[a][j],
+                                                                             0, 0, 0);
+                            if (imag)
+                                acc[a][NB + j] = __builtin_amdgcn_mfma_f64_16x16x4f64(
+                                    h, b[NB + j], acc[a][NB + j], 0, 0, 0);
                         }
                     }
-                    cre[q] = __builtin_amdgcn_mfma_f64_16x16x4f64(a.x, bre, cre[q], 0, 0, 0);
-                    if (imag) {
-                        cre[q] = __builtin_amdgcn_mfma_f64_16x16x4f64(-a.y, bim, cre[q], 0, 0, 0);
-                        cim[q] = __builtin_amdgcn_mfma_f64_16x16x4f64(a.x, bim, cim[q], 0, 0, 0);
+                }
+            }
+            if (tid < S) idx[buf ^ 1][tid] = source(v0 + 2 * S + tid);
+            __syncthreads();
+        }
+    }
+    __syncthreads();
+
+    // the waves' sums of one column tile at a time (over H), then the
+    // coefficients (n, +-m) of its densities
+    double(*red)[17] = reinterpret_cast<double(*)[17]>(lds);
+    double *o = expn + ecoef_off(kd, Bx, lv);
+    const int nh = (p + 1) * (p + 2) / 2;
+#pragma unroll
+    for (int j = 0; j < 2 * NB; ++j) {
+        if (pack && j == 1) break;
+        const bool im = j >= NB;
+        for (int w = 0; w < KG; ++w) {
+            __syncthreads();
+            if (kg == w) {
+#pragma unroll
+                for (int a = 0; a < RTW; ++a) {
+                    const int rt = rg * RTW + a;
+                    if (rt < RT) {
+#pragma unroll
+                        for (int q = 0; q < 4; ++q) {
+                            double &x = red[rt * 16 + 4 * q + kr][col];
+                            x = (w == 0 ? 0.0 : x) + acc[a][j][q];
+                        }
                     }
-                    cim[q] = __builtin_amdgcn_mfma_f64_16x16x4f64(a.y, bre, cim[q], 0, 0, 0);
                 }
             }
         }
-    };
-
-    int fill = 0;
-    for (int e = e0; e < e1; ++e) {
-        const int Sb = LOCAL ? lists[e] : Bx;
-        int s = t.sstart[Sb];
-        const int s1 = s + t.scount[Sb];
-        while (s < s1) {
-            const int take = min(s1 - s, P2E3M_S - fill);
-            for (int j = tid; j < take; j += 256) idx[fill + j] = s + j;
-            fill += take;
-            s += take;
-            if (fill == P2E3M_S) {
-                flush(P2E3M_S);
-                fill = 0;
+        __syncthreads();
+        // U(n, m) of column cc, any m, zero outside the table
+        auto U = [&](int n, int m, int cc) -> cplx {
+            const int am = m < 0 ? -m : m;
+            if (n < 0 || am > n) return {0, 0};
+            const int row = n * n + (am > 0 ? 2 * am - 1 : 0);
+            const cplx v = {red[row][cc], am > 0 ? red[row + 1][cc] : 0.0};
+            return m < 0 ? neg_m(v, am) : v;
+        };
+        auto coef = [&](int n, int m, int cc) -> cplx {
+            if (!DIP) return LOCAL ? U(n, m, cc) : conj(U(n, m, cc));
+            const int n1 = LOCAL ? n + 1 : n - 1;
+            const cplx I = {0, 1};
+            const cplx up = U(n1, m + 1, cc) - I * U(n1, m + 1, cc + 1);
+            const cplx dn = U(n1, m - 1, cc) + I * U(n1, m - 1, cc + 1);
+            const cplx uz = U(n1, m, cc + 2);
+            if (LOCAL) return 0.5 * (up - dn) - uz;
+            return conj(uz + 0.5 * (up - dn));
+        };
+        const int perd = pack ? rc : 16 / ND;   // densities of a tile
+        const int d0 = (im ? j - NB : j) * perd;
+        for (int q = tid; q < nh * 16; q += 256) {
+            const int ii = q >> 4, r = q & 15;
+            if (r >= perd || d0 + r >= rc) continue;
+            int n = (int)sqrt(2.0 * ii);
+            while (n * (n + 1) / 2 > ii) --n;
+            while ((n + 1) * (n + 2) / 2 <= ii) ++n;
+            const int m = ii - n * (n + 1) / 2;
+            cplx x = coef(n, m, r * ND), y = {0, 0};
+            if (pack) {
+                y = coef(n, m, 8 + r * ND);
+            } else if (im) {
+                y = x;
+                x = {0, 0};
             }
+            const cplx vp = {x.x - y.y, x.y + y.x};
+            const double sg = (m & 1) ? -1.0 : 1.0;
+            const cplx vm = {sg * (x.x + y.y), sg * (y.x - x.y)};
+            double *dp = o + 2 * ((long)IDX(n, m) * nr + r0 + d0 + r);
+            double *dm = o + 2 * ((long)IDX(n, -m) * nr + r0 + d0 + r);
+            const bool add = LOCAL || im;
+            stc(dp, add ? ldc(dp) + vp : vp);
+            if (m > 0) stc(dm, add ? ldc(dm) + vm : vm);
         }
-    }
-    if (fill > 0) flush(fill);
-    double *o = expn + ecoef_off(kd, Bx, lv);
-#pragma unroll
-    for (int q = 0; q < P2E3M_RTW; ++q) {
-        const int rt = wv + 4 * q;
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            const int row = rt * 16 + 4 * j + kr;
-            if (rt < RT && row < nout && col < rc) {
-                double *pq = o + 2 * ((long)row * nr + r0 + col);
-                const cplx v = {cre[q][j], cim[q][j]};
-                stc(pq, LOCAL ? ldc(pq) + v : v);
-            }
-        }
+        __syncthreads();
     }
 }
 
@@ -2483,38 +2337,55 @@ int f3_ncoeff_qbx(const qbx_kernel_desc *d)
     return kd.ncq;
 }
 
-// Shape of k3_p2e at order p: S sources per chunk in 32 KiB of LDS, threads
-// covering max((p+1)^2, S) (at most 512).  False: the plain kernels.
-static bool p2e3_launch(int p, bool local, P2EShape3 *sh, int *threads, size_t *bytes)
+// k3_p2e over the boxes of every level: its shape at each level's order and
+// the densities' chunks.  32 sources at a time while their table fits 40 KiB of
+// LDS (16 above order 11, 8 above 16).  Two column tiles (32 weights) where
+// they are filled and three row tiles a wave suffice.
+template <bool LOCAL>
+static int launch_p2e(hipStream_t st, KD kd, const TD &td, const std::vector<int> &lstart,
+                      const int *boxes, const int *starts, const int *lists, const double *src,
+                      int ns, const double *str, const double *nrm, double *expn)
 {
-    const int pt = local ? p + 1 : p;
-    P2EShape3 h;
-    h.R = ((pt + 1) * (pt + 2) / 2) | 1;
-    const long per = 8L * (2 * h.R + 2 * NRC_S + 3 + 1);
-    h.S = (int)std::min(64L, 32768L / per);
-    const int nout = (p + 1) * (p + 1);
-    if (h.S < 4 || nout > 512) return false;
-    *sh = h;
-    *threads = 64 * ((std::max(nout, h.S) + 63) / 64);
-    *bytes = 8UL * h.doubles(NRC_S);
-    return true;
-}
-
-// dynamic LDS of k3_p2e_mfma for table row stride R (complex)
-static size_t p2e3m_bytes(int R)
-{
-    return 8UL * (2 * P2E3M_S * R + 2 * P2E3M_S * 16 + 3 * P2E3M_S) + 4UL * P2E3M_S;
-}
-
-static bool p2e3_all_levels(const KD &kd, int nlevels, bool local)
-{
-    for (int l = 0; l < nlevels; ++l) {
-        P2EShape3 sh;
-        int th;
-        size_t by;
-        if (!p2e3_launch(kd.order[l], local, &sh, &th, &by)) return false;
+    const int nd = kd.dip ? 3 : 1;
+    for (int l = 0, l1; l < kd.nlevels; l = l1) {
+        // the boxes of consecutive levels of one order in one launch
+        for (l1 = l + 1; l1 < kd.nlevels && kd.order[l1] == kd.order[l];) ++l1;
+        const int i0 = lstart[l], nb = lstart[l1] - i0;
+        if (nb == 0) continue;
+        P2EShape h;
+        h.pt = LOCAL ? kd.order[l] + (kd.dip ? 1 : 0) : kd.order[l];
+        h.rows = (h.pt + 1) * (h.pt + 1);
+        h.RT = (h.rows + 15) / 16;
+        h.S = 32;
+        while (h.S > 8 && h.RT * 16 * (h.S + 2) * 8 > 40960) h.S /= 2;
+        h.SS = h.S + 2;
+        for (int r0 = 0; r0 < kd.nr;) {
+            const bool two = (kd.nr - r0) * nd > 16 && h.RT <= 12;
+            h.NB = two ? 2 : 1;
+            h.RTW = two ? 3 : h.RT <= 24 ? 6 : 8;
+            h.RG = h.RT <= h.RTW ? 1 : h.RT <= 2 * h.RTW ? 2 : 4;
+            const int per = h.NB * (16 / nd);
+            kd.r0 = r0;
+            kd.rc = std::min(per, kd.nr - r0);
+            h.bytes = 8UL * std::max(h.RT * 16 * h.SS + h.S * 32 * h.NB, h.RT * 16 * 17);
+#define P2E3_GO(D, N, T)                                                                   \
+    hipLaunchKernelGGL((k3_p2e<LOCAL, D, N, T>), dim3(nb), dim3(256), h.bytes, st, kd, td, i0, \
+                       h, boxes, starts, lists, src, ns, str, nrm, expn)
+            if (kd.dip) {
+                if (two) P2E3_GO(true, 2, 3);
+                else if (h.RTW == 6) P2E3_GO(true, 1, 6);
+                else P2E3_GO(true, 1, 8);
+            } else {
+                if (two) P2E3_GO(false, 2, 3);
+                else if (h.RTW == 6) P2E3_GO(false, 1, 6);
+                else P2E3_GO(false, 1, 8);
+            }
+#undef P2E3_GO
+            r0 += kd.rc;
+        }
     }
-    return true;
+    QBX_HIP(hipGetLastError());
+    return QBX_OK;
 }
 
 int f3_form_multipoles(qbx_ctx *ctx, void *stream, const qbx_tree *T, const qbx_trav *R,
@@ -2526,49 +2397,9 @@ int f3_form_multipoles(qbx_ctx *ctx, void *stream, const qbx_tree *T, const qbx_
     QBX_CHECK(!kd.dip || nrm, "double layer needs normals");
     hipStream_t st = S(stream);
     QBX_TRY(zero_fill(mpole, (exp_bytes(kd)) / 8, st));
-    if (p2e3_all_levels(kd, T->nlevels, false)) {
-        const TD td = make_td(T);
-        for (int l = 0; l < T->nlevels; ++l) {
-            const int i0 = R->h_level_start_source_box_nrs[l];
-            const int i1 = R->h_level_start_source_box_nrs[l + 1];
-            if (i1 == i0) continue;
-            P2EShape3 sh;
-            int th;
-            size_t by;
-            p2e3_launch(kd.order[l], false, &sh, &th, &by);
-            if (kd.nr >= 4 && (kd.order[l] + 1) * (kd.order[l] + 1) <= 16 * 4 * P2E3M_RTW) {
-                for (int r0 = 0; r0 < kd.nr; r0 += 16) {
-                    kd.r0 = r0;
-                    kd.rc = std::min(16, kd.nr - r0);
-                    hipLaunchKernelGGL(k3_p2e_mfma<false>, dim3(i1 - i0), dim3(256),
-                                       p2e3m_bytes(sh.R), st, kd, td, l, i0, sh.R,
-                                       R->source_boxes.p, nullptr, nullptr, T->sources.p,
-                                       T->nsources, str, nrm, mpole);
-                }
-                continue;
-            }
-#define L3_P2MH(N)                                                                         \
-    hipLaunchKernelGGL((k3_p2e<N, false>), dim3(i1 - i0), dim3(th), by, st, kd, td, l, i0, sh, \
-                       R->source_boxes.p, nullptr, nullptr, T->sources.p, T->nsources, str,  \
-                       nrm, mpole)
-            FOR_RHS_CHUNKS3(kd, NRC_S, L3_P2MH);
-#undef L3_P2MH
-        }
-        QBX_HIP(hipGetLastError());
-        return QBX_OK;
-    }
-    const Flat fl = make_flat(kd, R->h_level_start_source_box_nrs);
-    const long nthr = fl.tstart[fl.nl];
-    if (nthr > 0) {
-        const TD td = make_td(T);
-#define L3_P2M(N)                                                                          \
-    hipLaunchKernelGGL(k3_p2m<N>, dim3(cdiv(nthr, 128)), dim3(128), 0, st, kd, td, fl,     \
-                       R->source_boxes.p, T->sources.p, T->nsources, str, nrm, mpole)
-        FOR_RHS_CHUNKS3(kd, NRC_S, L3_P2M);
-#undef L3_P2M
-    }
-    QBX_HIP(hipGetLastError());
-    return QBX_OK;
+    return launch_p2e<false>(st, kd, make_td(T), R->h_level_start_source_box_nrs,
+                             R->source_boxes.p, nullptr, nullptr, T->sources.p, T->nsources, str,
+                             nrm, mpole);
 }
 
 // Launch k3_trans_real<OPK, p> over nb output boxes of level l (orders p <= 15;
@@ -2771,50 +2602,10 @@ int f3_form_locals(qbx_ctx *ctx, void *stream, const qbx_tree *T, const qbx_trav
     QBX_CHECK(!kd.dip || nrm, "double layer needs normals");
     hipStream_t st = S(stream);
     if (!accumulate) QBX_TRY(zero_fill(local, (exp_bytes(kd)) / 8, st));
-    if (R->n4 > 0 && p2e3_all_levels(kd, T->nlevels, true)) {
-        const TD td = make_td(T);
-        for (int l = 0; l < T->nlevels; ++l) {
-            const int i0 = R->h_level_start_ttp_box_nrs[l];
-            const int i1 = R->h_level_start_ttp_box_nrs[l + 1];
-            if (i1 == i0) continue;
-            P2EShape3 sh;
-            int th;
-            size_t by;
-            p2e3_launch(kd.order[l], true, &sh, &th, &by);
-            if (kd.nr >= 4 && (kd.order[l] + 1) * (kd.order[l] + 1) <= 16 * 4 * P2E3M_RTW) {
-                for (int r0 = 0; r0 < kd.nr; r0 += 16) {
-                    kd.r0 = r0;
-                    kd.rc = std::min(16, kd.nr - r0);
-                    hipLaunchKernelGGL(k3_p2e_mfma<true>, dim3(i1 - i0), dim3(256),
-                                       p2e3m_bytes(sh.R), st, kd, td, l, i0, sh.R,
-                                       R->ttp_boxes.p, R->l4_starts.p, R->l4_lists.p,
-                                       T->sources.p, T->nsources, str, nrm, local);
-                }
-                continue;
-            }
-#define L3_P2LH(N)                                                                         \
-    hipLaunchKernelGGL((k3_p2e<N, true>), dim3(i1 - i0), dim3(th), by, st, kd, td, l, i0, sh, \
-                       R->ttp_boxes.p, R->l4_starts.p, R->l4_lists.p, T->sources.p,         \
-                       T->nsources, str, nrm, local)
-            FOR_RHS_CHUNKS3(kd, NRC_S, L3_P2LH);
-#undef L3_P2LH
-        }
-        QBX_HIP(hipGetLastError());
-        return QBX_OK;
-    }
-    const Flat fl = make_flat(kd, R->h_level_start_ttp_box_nrs);
-    const long nthr = fl.tstart[fl.nl];
-    if (nthr > 0 && R->n4 > 0) {
-        const TD td = make_td(T);
-#define L3_P2L(N)                                                                          \
-    hipLaunchKernelGGL(k3_p2l<N>, dim3(cdiv(nthr, 128)), dim3(128), 0, st, kd, td, fl,     \
-                       R->ttp_boxes.p, R->l4_starts.p, R->l4_lists.p, T->sources.p,        \
-                       T->nsources, str, nrm, local)
-        FOR_RHS_CHUNKS3(kd, NRC_S, L3_P2L);
-#undef L3_P2L
-    }
-    QBX_HIP(hipGetLastError());
-    return QBX_OK;
+    if (R->n4 == 0) return QBX_OK;
+    return launch_p2e<true>(st, kd, make_td(T), R->h_level_start_ttp_box_nrs, R->ttp_boxes.p,
+                            R->l4_starts.p, R->l4_lists.p, T->sources.p, T->nsources, str, nrm,
+                            local);
 }
 
 int f3_refine_locals(qbx_ctx *ctx, void *stream, const qbx_tree *T, const qbx_trav *R,
