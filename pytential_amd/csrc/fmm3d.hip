@@ -86,25 +86,6 @@ struct TD {
     const int *sstart, *scount, *scumul;
 };
 
-struct Flat {
-    int nl;
-    long tstart[FML + 1];
-    int istart[FML];
-    int nper[FML];
-};
-
-__device__ __forceinline__ bool flat_locate(const Flat &f, long gid, int &lv, int &i, int &j)
-{
-    if (gid >= f.tstart[f.nl]) return false;
-    int l = 0;
-    while (gid >= f.tstart[l + 1]) ++l;
-    const long r = gid - f.tstart[l];
-    lv = l;
-    i = f.istart[l] + (int)(r / f.nper[l]);
-    j = (int)(r % f.nper[l]);
-    return true;
-}
-
 struct v3 {
     double x, y, z;
 };
@@ -724,127 +705,7 @@ __global__ void __launch_bounds__(M2L_THREADS) k3_m2l(KD kd, TD t, const int *tt
     }
 }
 
-// M2L for many right-hand sides on the FP64 matrix cores: per target box
-// out(k,l)[r] = sum_(n,m) T(n+k, m+l) h^-n a(n,m)[r] (the sum of k3_m2l), a
-// complex product of the (k,l) x (n,m) operator -- entries gathered from the
-// entry's unit-offset table, staged in LDS -- with the multipole coefficients
-// of up to 16 right-hand sides, on v_mfma_f64_16x16x4f64 (lane i holds
-// A[i%16][k0 + i/16] and B[k0 + i/16][i%16]; D register j of lane i is
-// D[4j + i/16][i%16]).  Wave w takes the 16-row tiles w, w + 4, ... over all
-// entries; the epilogue scales by (-1)^k h^(-k-1) as k3_m2l.
-constexpr int M2L3M_RTW = 4;             // row tiles per wave: (p + 1)^2 <= 256
-constexpr int M2L3M_T = 2 * 15 + 1;      // table side for p <= 15
-
-__global__ void __launch_bounds__(256)
-k3_m2l_mfma(KD kd, TD t, Flat fl, const int *ttp, const int *starts, const int *lists,
-            const double *mpole, double *local, const int *allreal)
-{
-    __shared__ double Ts[2 * M2L3M_T * M2L3M_T];
-    __shared__ short nof[256], mof[256];
-    __shared__ double ihp[32];
-    if (allreal && *allreal) return;  // k3_trans_real's case
-    int lv, i, unused;
-    if (!flat_locate(fl, blockIdx.x, lv, i, unused)) return;
-    const int e0 = starts[i], e1 = starts[i + 1];
-    if (e0 == e1) return;
-    const int Bx = ttp[i];
-    const int p = kd.order[lv];
-    const int nc = kd.ncl[lv];
-    const int RT = (nc + 15) / 16, KS = (nc + 3) / 4;
-    const int tnl = (2 * p + 1) * (2 * p + 1);  // table entries used: IDX(N, M), N <= 2p
-    const double ih = 1.0 / kd.h[lv];
-    const int W = kd.W, S1 = 2 * W + 1, tn = kd.tabn;
-    const int tid = threadIdx.x, wv = tid >> 6, lane = tid & 63;
-    const int col = lane & 15, kr = lane >> 4;
-    const int rc = kd.rc, r0 = kd.r0;
-    for (int q = tid; q < 256; q += 256) {
-        int n = (int)sqrt((double)q);
-        while (n * n > q) --n;
-        while ((n + 1) * (n + 1) <= q) ++n;
-        nof[q] = (short)n;
-        mof[q] = (short)(q - n * n - n);
-    }
-    if (tid < 32) {
-        double s = 1.0;
-        for (int k = 0; k < tid; ++k) s *= ih;
-        ihp[tid] = s;
-    }
-    __syncthreads();  // nof, mof, ihp (the epilogue reads them even with no entry)
-    const int bx = t.coords[Bx], by = t.coords[(size_t)t.nboxes + Bx],
-              bz = t.coords[2 * (size_t)t.nboxes + Bx];
-    f3_d4 cre[M2L3M_RTW], cim[M2L3M_RTW];
-#pragma unroll
-    for (int q = 0; q < M2L3M_RTW; ++q) cre[q] = cim[q] = f3_d4{0, 0, 0, 0};
-    for (int e = e0; e < e1; ++e) {
-        const int A = lists[e];
-        const int dx = bx - t.coords[A] + W;
-        const int dy = by - t.coords[(size_t)t.nboxes + A] + W;
-        const int dz = bz - t.coords[2 * (size_t)t.nboxes + A] + W;
-        if ((unsigned)dx >= (unsigned)S1 || (unsigned)dy >= (unsigned)S1 ||
-            (unsigned)dz >= (unsigned)S1)
-            continue;  // uniform over the block
-        const double *a = mpole + ecoef_off(kd, A, lv);
-        const double *T = kd.tab_m2l + 2L * ((dx * S1 + dy) * S1 + dz) * tn * tn;
-        __syncthreads();  // previous table consumed (and nof/ihp written)
-        for (int q = tid; q < tnl; q += 256) {
-            Ts[2 * q] = T[2 * q];
-            Ts[2 * q + 1] = T[2 * q + 1];
-        }
-        __syncthreads();
-        for (int ks = 0; ks < KS; ++ks) {
-            const int kq = ks * 4 + kr;  // (n, m) of the B row / A column
-            double bre = 0.0, bim = 0.0;
-            int n = 0, m = 0;
-            if (kq < nc) {
-                n = nof[kq];
-                m = mof[kq];
-                if (col < rc) {
-                    const cplx b = ldcn(kd, a, kq, r0 + col);
-                    bre = ihp[n] * b.x;
-                    bim = ihp[n] * b.y;
-                }
-            }
-#pragma unroll
-            for (int q = 0; q < M2L3M_RTW; ++q) {
-                const int rt = wv + 4 * q;
-                if (rt < RT) {
-                    const int row = rt * 16 + col;
-                    double are = 0.0, aim = 0.0;
-                    if (row < nc && kq < nc) {
-                        const int N = n + nof[row], M = m + mof[row];
-                        if (M >= -N && M <= N) {
-                            are = Ts[2 * IDX(N, M)];
-                            aim = Ts[2 * IDX(N, M) + 1];
-                        }
-                    }
-                    cre[q] = __builtin_amdgcn_mfma_f64_16x16x4f64(are, bre, cre[q], 0, 0, 0);
-                    cre[q] = __builtin_amdgcn_mfma_f64_16x16x4f64(-aim, bim, cre[q], 0, 0, 0);
-                    cim[q] = __builtin_amdgcn_mfma_f64_16x16x4f64(are, bim, cim[q], 0, 0, 0);
-                    cim[q] = __builtin_amdgcn_mfma_f64_16x16x4f64(aim, bre, cim[q], 0, 0, 0);
-                }
-            }
-        }
-    }
-    double *o = local + ecoef_off(kd, Bx, lv);
-#pragma unroll
-    for (int q = 0; q < M2L3M_RTW; ++q) {
-        const int rt = wv + 4 * q;
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            const int row = rt * 16 + 4 * j + kr;
-            if (rt < RT && row < nc && col < rc) {
-                const int k = nof[row];
-                const double sc = ((k & 1) ? -1.0 : 1.0) * ihp[k + 1];
-                double *dst = o + 2 * ((long)row * kd.nr + r0 + col);
-                dst[0] += sc * cre[q][j];
-                dst[1] += sc * cim[q][j];
-            }
-        }
-    }
-}
-
-// Box translations for many real densities on the FP64 matrix cores.  Real
-// strengths give M_n^{-m} = (-1)^m conj(M_n^m) and L_n^{-m} = (-1)^m
+// Box translations on the FP64 matrix cores.  Real strengths give M_n^{-m} = (-1)^m conj(M_n^m) and L_n^{-m} = (-1)^m
 // conj(L_n^m) for every multipole and local, so a translation out = A in
 // forms only the output rows i = (k, l), l >= 0, from the input columns
 // j = (n, m), m >= 0: out_i = sum_j A1 a_j + A2 conj(a_j) with A1 = A(i, j)
@@ -872,8 +733,24 @@ k3_m2l_mfma(KD kd, TD t, Flat fl, const int *ttp, const int *starts, const int *
 // contracted.  The K-steps of each entry are dealt round-robin to the four
 // waves, each wave holding every row tile; the waves' sums are added in LDS
 // at the end and the epilogue writes row (k, l) and its mirror (k, -l).
-// With allreal given the kernel runs only when *allreal is set (the complex
-// kernels take the other case); without, the caller has stated it.
+//
+// SPLIT (M2L): strengths of any kind, two columns to a density.  Every expansion is
+// M = Mr + i Mi with both parts conjugate-symmetric, Mr = (M + J M)/2, Mi =
+// (M - J M)/(2i), (J M)_n^m = (-1)^m conj(M_n^{-m}); the columns of Mr and Mi
+// are translated as real densities and the epilogue adds Lr + i Li.  One to
+// three densities take this route too: 2 of 16 columns filled, yet a third of
+// the serial vector kernel's time (M2M and L2L of few densities stay on it:
+// few boxes a level, and there the vector kernels are twice as fast): 38170
+// list-2 pairs at order 10, one density, 5.3 -> 1.7 ms.
+//
+// With allreal given the kernel runs only when *allreal is set, SPLIT only
+// when it is not; without, the caller has stated which.
+//
+// M2L's operand gather: T_{n+k}^{m+l} lies at n^2 + n + m + (k^2 + k + l) +
+// 2nk, so that a row tile costs three integer operations a K-step instead of
+// twenty (the masks of the general form are not needed: rows and columns
+// beyond the last meet zeros of B or are not stored).  32 real densities at
+// order 8, 875275 pairs (495 GFLOP executed): 17.6 -> 12.9 ms, 38 TFLOP/s.
 constexpr int TR3_ECH = 256;  // entries whose offsets are staged at once
 
 __host__ __device__ constexpr int tri_n(int j)  // n of triangular index j
@@ -883,9 +760,9 @@ __host__ __device__ constexpr int tri_n(int j)  // n of triangular index j
     return n;
 }
 
-template <int OPK, int P, int NCT>
+template <int OPK, int P, int NCT, bool SPLIT>
 __global__ void __launch_bounds__(256)
-k3_trans_real(KD kd, TD t, int lv, int i0, const int *boxes, const int *starts,
+k3_trans_real(KD kd, TD t, int i0, const int *boxes, const int *starts,
               const int *lists, const double *in, double *out, const int *allreal)
 {
     constexpr int R = (P + 1) * (P + 2) / 2;      // coefficients with m >= 0
@@ -910,9 +787,10 @@ k3_trans_real(KD kd, TD t, int lv, int i0, const int *boxes, const int *starts,
     __shared__ long eoff[TR3_ECH];
     __shared__ int nent;
     double *Ts = lds, *Bs = lds + 2 * TNL;
-    if (allreal && *allreal == 0) return;
+    if (allreal && (*allreal != 0) == SPLIT) return;
     const int i = i0 + blockIdx.x;
     const int Bx = boxes[i];
+    const int lv = t.level[Bx];
     // the entry range: list 2, the children, or the parent
     int e0 = 0, e1 = 0;
     if (OPK == 0) {
@@ -961,7 +839,15 @@ k3_trans_real(KD kd, TD t, int lv, int i0, const int *boxes, const int *starts,
         rowk[rt] = rho < R2 ? k : -1;
         rowl[rt] = ii - k * (k + 1) / 2;
         rowpr[rt] = rho & 1;
+        if (OPK == 0) {
+            // the row's share of the table offset, and 2k, in bytes
+            const int kk = rho < R2 ? k : 0, ll = rho < R2 ? rowl[rt] : 0;
+            rowk[rt] = 16 * (kk * kk + kk + ll) + ((col ^ kr) & 1 ? 8 : 0);
+            rowl[rt] = 32 * kk;
+        }
     }
+    // M2L: the sign of column part kr % 2 (re, im) in row part col % 2
+    const double sneg = (col & 1) == 0 && (kr & 1) ? -1.0 : 1.0;
     const int bx = t.coords[Bx], by = t.coords[(size_t)t.nboxes + Bx],
               bz = t.coords[2 * (size_t)t.nboxes + Bx];
     // the staged data of an entry: table doubles and (re, im) of the B pairs;
@@ -986,12 +872,24 @@ k3_trans_real(KD kd, TD t, int lv, int i0, const int *boxes, const int *starts,
             const int f = tid + 256 * u;
             const int j = f / RC, r = f % RC;
             br[u][0] = br[u][1] = 0.0;
-            if (f < R * RC && r < rc) {
+            if (f < R * RC && (SPLIT ? r >> 1 : r) < rc) {
                 const int n = jn[j];
                 const int m = j - n * (n + 1) / 2;
-                const double *z = a + 2 * ((long)(n * n + n + m) * nr + r0 + r);
-                br[u][0] = z[0];
-                br[u][1] = z[1];
+                const long i1 = (long)(n * n + n + m) * nr + r0;
+                if (SPLIT) {
+                    const double *z = a + 2 * (i1 + (r >> 1)), *y = z - 4L * m * nr;
+                    const double sg = (m & 1) ? -1.0 : 1.0;
+                    if (r & 1) {
+                        br[u][0] = 0.5 * (z[1] + sg * y[1]);
+                        br[u][1] = -0.5 * (z[0] - sg * y[0]);
+                    } else {
+                        br[u][0] = 0.5 * (z[0] + sg * y[0]);
+                        br[u][1] = 0.5 * (z[1] - sg * y[1]);
+                    }
+                } else {
+                    br[u][0] = a[2 * (i1 + r)];
+                    br[u][1] = a[2 * (i1 + r) + 1];
+                }
             }
         }
         return true;
@@ -1063,6 +961,39 @@ k3_trans_real(KD kd, TD t, int lv, int i0, const int *boxes, const int *starts,
             __syncthreads();
             have = ee + 1 < cn ? fetch(ee + 1) : false;
             if (!cur) continue;
+            if (OPK == 0) {
+                for (int ks = kg; ks < KS; ks += KG) {
+                    const int kap = ks * 4 + kr;  // B row / A column
+                    const bool kin = kap < R2;
+                    const int j = kin ? kap >> 1 : 0;
+                    double b[NCT];
+#pragma unroll
+                    for (int c = 0; c < NCT; ++c)
+                        b[c] = kin ? Bs[kap * RC + c * 16 + col] : 0.0;
+                    const int n = jn[j], m = j - n * (n + 1) / 2;
+                    const int cb = 16 * (n * n + n + m);   // bytes
+                    const double s2 = m == 0 ? 0.0 : ((m + kr) & 1) ? -sneg : sneg;
+                    const char *tb = reinterpret_cast<const char *>(Ts);
+                    double c1[RTW], c2[RTW];
+#pragma unroll
+                    for (int rt = 0; rt < RTW; ++rt) {
+                        const int o1 = rowk[rt] + cb + n * rowl[rt];
+                        c1[rt] = *reinterpret_cast<const double *>(tb + o1);
+                        c2[rt] = *reinterpret_cast<const double *>(tb + o1 - 32 * m);
+                    }
+#pragma unroll
+                    for (int rt = 0; rt < RTW; ++rt) {
+                        const double v = s2 * c2[rt] + sneg * c1[rt];
+                        if (rg * RTW + rt < RT) {
+#pragma unroll
+                            for (int c = 0; c < NCT; ++c)
+                                acc[rt][c] = __builtin_amdgcn_mfma_f64_16x16x4f64(
+                                    v, b[c], acc[rt][c], 0, 0, 0);
+                        }
+                    }
+                }
+                continue;
+            }
             for (int ks = (kg - step + KG * 4) % KG; ks < KS; ks += KG) {
                 const int kap = ks * 4 + kr;  // B row / A column
                 const int j = kap >> 1, pk = kap & 1;
@@ -1092,12 +1023,7 @@ k3_trans_real(KD kd, TD t, int lv, int i0, const int *boxes, const int *starts,
                     const int off = rowpr[rt] == pk ? 0 : 1;
                     int i1, i2;
                     bool ok1, ok2;
-                    if (OPK == 0) {
-                        const int N = n + k, base = N * N + N;
-                        i1 = base + m + l;
-                        i2 = base + l - m;
-                        ok1 = ok2 = kin && k >= 0;
-                    } else if (OPK == 1) {
+                    if (OPK == 1) {
                         const int K = k - n, base = K * K + K;
                         i1 = base + l - m;
                         i2 = base + l + m;
@@ -1123,7 +1049,7 @@ k3_trans_real(KD kd, TD t, int lv, int i0, const int *boxes, const int *starts,
                     const int rklo = tri_n(min(8 * rtg, R - 1)),
                               rkhi = tri_n(min(8 * rtg + 7, R - 1));
                     const bool live =
-                        rtg < RT && (OPK == 0 || (OPK == 1 ? nlo <= rkhi : nhi >= rklo));
+                        rtg < RT && (OPK == 1 ? nlo <= rkhi : nhi >= rklo);
                     double v = (v1[rt] ? c1[rt] : 0.0) + s2 * (v2[rt] ? c2[rt] : 0.0);
                     v = (rowpr[rt] == 0 && pk == 1) ? -v : v;
                     if (live) {
@@ -1161,32 +1087,26 @@ k3_trans_real(KD kd, TD t, int lv, int i0, const int *boxes, const int *starts,
             }
         }
         __syncthreads();
-        for (int q = tid; q < R * 16; q += 256) {
-            const int ii = q >> 4, cc = q & 15;
-            const int r = c * 16 + cc;
+        constexpr int DC = SPLIT ? 8 : 16;   // densities of a tile
+        for (int q = tid; q < R * DC; q += 256) {
+            const int ii = q / DC, cc = q % DC;
+            const int r = c * DC + cc;
             if (r >= rc) continue;
             const int k = jn[ii];
             const int l = ii - k * (k + 1) / 2;
-            const double sc = osc[k];
-            const double re = sc * red[2 * ii][cc], im = sc * red[2 * ii + 1][cc];
+            const double sc = osc[k], sl = (l & 1) ? -sc : sc;
+            const int cx = SPLIT ? 2 * cc : cc;
+            cplx v = {red[2 * ii][cx], red[2 * ii + 1][cx]};
+            cplx u = conj(v);                   // (k, -l): (-1)^l of it
+            if (SPLIT) {
+                const cplx y = {red[2 * ii][cx + 1], red[2 * ii + 1][cx + 1]};
+                v += cplx{-y.y, y.x};
+                u += cplx{y.y, y.x};
+            }
             double *dst = o + 2 * ((long)(k * k + k + l) * nr + r0 + r);
             double *dm = o + 2 * ((long)(k * k + k - l) * nr + r0 + r);
-            const double sl = (l & 1) ? -1.0 : 1.0;
-            if (OPK == 1) {
-                dst[0] = re;
-                dst[1] = im;
-                if (l > 0) {
-                    dm[0] = sl * re;
-                    dm[1] = -sl * im;
-                }
-            } else {
-                dst[0] += re;
-                dst[1] += im;
-                if (l > 0) {
-                    dm[0] += sl * re;
-                    dm[1] -= sl * im;
-                }
-            }
+            stc(dst, OPK == 1 ? sc * v : ldc(dst) + sc * v);
+            if (l > 0) stc(dm, OPK == 1 ? sl * u : ldc(dm) + sl * u);
         }
     }
 }
@@ -2250,22 +2170,6 @@ static TD make_td(const qbx_tree *T)
     return t;
 }
 
-static Flat make_flat(const KD &kd, const std::vector<int> &level_starts)
-{
-    Flat f;
-    memset(&f, 0, sizeof(f));
-    f.nl = kd.nlevels;
-    long t = 0;
-    for (int l = 0; l < kd.nlevels; ++l) {
-        f.tstart[l] = t;
-        f.istart[l] = level_starts[l];
-        f.nper[l] = kd.ncl[l];
-        t += (long)(level_starts[l + 1] - level_starts[l]) * f.nper[l];
-    }
-    f.tstart[kd.nlevels] = t;
-    return f;
-}
-
 // Run LAUNCH(N) over the right-hand-side chunks: N = 1 for a single
 // right-hand side, CH otherwise; kd.r0 / kd.rc are set per chunk.
 #define FOR_RHS_CHUNKS3(kd, CH, LAUNCH)                                                 \
@@ -2404,26 +2308,26 @@ int f3_form_multipoles(qbx_ctx *ctx, void *stream, const qbx_tree *T, const qbx_
 
 // Launch k3_trans_real<OPK, p> over nb output boxes of level l (orders p <= 15;
 // 32 right-hand sides per block, 16 for M2M and L2L above order 9).
-template <int OPK>
-static int launch_trans_real(hipStream_t st, KD kd, const TD &td, int l, int p, int i0,
-                             int nb, const int *boxes, const int *starts, const int *lists,
+template <int OPK, bool SPLIT>
+static int launch_trans_real(hipStream_t st, KD kd, const TD &td, int p, int i0, int nb,
+                             const int *boxes, const int *starts, const int *lists,
                              const double *in, double *out, const int *allreal)
 {
-    const int rcb = (OPK != 0 && p >= 10) ? 16 : 32;
+    const int rcb = SPLIT ? 8 : (OPK != 0 && p >= 10) ? 16 : 32;
     for (int r0 = 0; r0 < kd.nr; r0 += rcb) {
         kd.r0 = r0;
         kd.rc = std::min(rcb, kd.nr - r0);
 #define TR_CASE(PP)                                                                        \
     case PP:                                                                               \
-        hipLaunchKernelGGL((k3_trans_real<OPK, PP, (OPK != 0 && PP >= 10) ? 1 : 2>), dim3(nb), \
-                           dim3(256), 0, st, kd, td,                                       \
-                           l, i0, boxes, starts, lists, in, out, allreal);                 \
+        hipLaunchKernelGGL(                                                                \
+            (k3_trans_real<OPK, PP, (SPLIT || (OPK != 0 && PP >= 10)) ? 1 : 2, SPLIT>),    \
+            dim3(nb), dim3(256), 0, st, kd, td, i0, boxes, starts, lists, in, out, allreal); \
         break;
         switch (p) {
             TR_CASE(1) TR_CASE(2) TR_CASE(3) TR_CASE(4) TR_CASE(5) TR_CASE(6) TR_CASE(7)
             TR_CASE(8) TR_CASE(9) TR_CASE(10) TR_CASE(11) TR_CASE(12) TR_CASE(13)
             TR_CASE(14) TR_CASE(15)
-        default: set_error("real-strength translation: order %d out of range", p);
+        default: set_error("matrix-core translation: order %d out of range", p);
             return QBX_ERR_INVALID;
         }
 #undef TR_CASE
@@ -2433,10 +2337,10 @@ static int launch_trans_real(hipStream_t st, KD kd, const TD &td, int l, int p, 
 }
 
 // Which kernels run a box translation: the real-strength matrix-core kernel
-// (stated by the caller, or decided on the device by *flag), the complex one,
-// or both, each returning at once in the other's case.
+// (stated by the caller, or decided on the device by *flag), the one for any
+// strengths, or both, each returning at once in the other's case.
 struct RealSel {
-    bool real, complex_;
+    bool real, other;
     const int *flag;  // passed to both kernels (null: no device decision)
 };
 
@@ -2465,10 +2369,10 @@ int f3_coarsen_multipoles(qbx_ctx *ctx, void *stream, const qbx_tree *T, const q
             const int p = kd.order[l];
             const RealSel rs = real_sel(d, kd, allreal, p <= 15 && kd.order[l + 1] == p);
             if (rs.real)
-                QBX_TRY(launch_trans_real<1>(st, kd, td, l, p, i0, i1 - i0,
-                                             R->source_parent_boxes.p, nullptr, nullptr, mpole,
-                                             mpole, rs.flag));
-            if (rs.complex_) {
+                QBX_TRY((launch_trans_real<1, false>(st, kd, td, p, i0, i1 - i0,
+                                                     R->source_parent_boxes.p, nullptr, nullptr,
+                                                     mpole, mpole, rs.flag)));
+            if (rs.other) {
 #define L3_M2M(N)                                                                          \
     hipLaunchKernelGGL(k3_m2m<N>, dim3(cdiv(nthr, 128)), dim3(128), 0, st, kd, td, l, i0,  \
                        i1, R->source_parent_boxes.p, mpole, rs.flag)
@@ -2545,39 +2449,23 @@ int f3_multipole_to_local(qbx_ctx *ctx, void *stream, const qbx_tree *T, const q
     hipStream_t st = S(stream);
     QBX_TRY(zero_fill(local, (exp_bytes(kd)) / 8, st));
     const RealSel rs = real_sel(d, kd, allreal, kd.pmax <= 15);
-    if (R->nttp_boxes > 0 && R->n2 > 0 && kd.nr >= 4 && kd.pmax <= 15) {
-        // many right-hand sides: on the matrix cores, 16 per launch (complex)
+    if (R->nttp_boxes > 0 && R->n2 > 0 && kd.pmax <= 15) {
+        // the boxes of consecutive levels of one order in one launch (a
+        // kernel's tile counts are fixed by its order)
         const TD td = make_td(T);
-        if (rs.complex_) {
-            Flat fl;
-            fl.nl = kd.nlevels;
-            long nb = 0;
-            for (int l = 0; l < kd.nlevels; ++l) {
-                fl.tstart[l] = nb;
-                fl.istart[l] = R->h_level_start_ttp_box_nrs[l];
-                fl.nper[l] = 1;
-                nb += R->h_level_start_ttp_box_nrs[l + 1] - R->h_level_start_ttp_box_nrs[l];
-            }
-            fl.tstart[kd.nlevels] = nb;
-            for (int r0 = 0; r0 < kd.nr; r0 += 16) {
-                kd.r0 = r0;
-                kd.rc = std::min(16, kd.nr - r0);
-                hipLaunchKernelGGL(k3_m2l_mfma, dim3(nb), dim3(256), 0, st, kd, td, fl,
-                                   R->ttp_boxes.p, R->l2_starts.p, R->l2_lists.p, mpole, local,
-                                   rs.flag);
-            }
-        }
-        // real strengths: the conjugate-symmetric kernel, level by level (its
-        // tile counts are fixed by the level's order)
-        if (rs.real) {
-            for (int l = 0; l < kd.nlevels; ++l) {
-                const int i0 = R->h_level_start_ttp_box_nrs[l];
-                const int nbl = R->h_level_start_ttp_box_nrs[l + 1] - i0;
-                if (nbl == 0) continue;
-                QBX_TRY(launch_trans_real<0>(st, kd, td, l, kd.order[l], i0, nbl,
-                                             R->ttp_boxes.p, R->l2_starts.p, R->l2_lists.p,
-                                             mpole, local, rs.flag));
-            }
+        const std::vector<int> &ls = R->h_level_start_ttp_box_nrs;
+        for (int l = 0, l1; l < kd.nlevels; l = l1) {
+            for (l1 = l + 1; l1 < kd.nlevels && kd.order[l1] == kd.order[l];) ++l1;
+            const int i0 = ls[l], nb = ls[l1] - i0, p = kd.order[l];
+            if (nb == 0) continue;
+            if (rs.real)
+                QBX_TRY((launch_trans_real<0, false>(st, kd, td, p, i0, nb, R->ttp_boxes.p,
+                                                     R->l2_starts.p, R->l2_lists.p, mpole, local,
+                                                     rs.flag)));
+            if (rs.other)
+                QBX_TRY((launch_trans_real<0, true>(st, kd, td, p, i0, nb, R->ttp_boxes.p,
+                                                    R->l2_starts.p, R->l2_lists.p, mpole, local,
+                                                    rs.flag)));
         }
     } else if (R->nttp_boxes > 0 && R->n2 > 0) {
         const TD td = make_td(T);
@@ -2623,9 +2511,9 @@ int f3_refine_locals(qbx_ctx *ctx, void *stream, const qbx_tree *T, const qbx_tr
             const int p = kd.order[l];
             const RealSel rs = real_sel(d, kd, allreal, p <= 15 && kd.order[l - 1] == p);
             if (rs.real)
-                QBX_TRY(launch_trans_real<2>(st, kd, td, l, p, i0, i1 - i0, R->ttp_boxes.p,
-                                             nullptr, nullptr, local, local, rs.flag));
-            if (rs.complex_) {
+                QBX_TRY((launch_trans_real<2, false>(st, kd, td, p, i0, i1 - i0, R->ttp_boxes.p,
+                                                     nullptr, nullptr, local, local, rs.flag)));
+            if (rs.other) {
 #define L3_L2L(N)                                                                          \
     hipLaunchKernelGGL(k3_l2l<N>, dim3(cdiv(nthr, 128)), dim3(128), 0, st, kd, td, l, i0,  \
                        i1, R->ttp_boxes.p, local, rs.flag)
