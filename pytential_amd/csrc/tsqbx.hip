@@ -18,6 +18,7 @@
 // into registers; lane groups reduce with shuffles.  Output overwrites
 // pot / grad at the QBX targets, like the reference.
 #include "qbx_internal.h"
+#include "qbx_math.h"
 
 namespace qbx {
 
@@ -310,21 +311,65 @@ __global__ void __launch_bounds__(256) k_tsqbx(double kre, double kim, int nctt,
     }
 }
 
+// G of one (target, source) pair of the Laplace target-specific sum, S or D:
+// a_n = rt^n / rs^{n+1} P_n(ct) by its own recurrence
+//   (n+1) a_{n+1} = (2n+1) x a_n - n y a_{n-1},  x = tc.sc / rs^2, y = rt^2 / rs^2
+// (and its derivative along the source's nu), one reciprocal square root and
+// no division.
+template <int OP, int P>
+__device__ __forceinline__ double tsq_laplace(const double *tc, double rt2, double sx, double sy,
+                                              double sz, const double *nu)
+{
+    const double ir = qbx_rsqrt(sx * sx + sy * sy + sz * sz);
+    const double w = ir * ir;
+    const double x = (tc[0] * sx + tc[1] * sy + tc[2] * sz) * w, y = rt2 * w;
+    double a0 = 0.0, a1 = ir, sum = ir;
+    double b0 = 0.0, b1 = 0.0, dx = 0.0, dy = 0.0, dsum = 0.0;
+    if (OP == 1) {
+        const double sn = (nu[0] * sx + nu[1] * sy + nu[2] * sz) * w;
+        dx = (tc[0] * nu[0] + tc[1] * nu[1] + tc[2] * nu[2]) * w - 2.0 * x * sn;
+        dy = -2.0 * y * sn;
+        b1 = dsum = -a1 * sn;
+    }
+#pragma unroll
+    for (int n = 0; n < P; ++n) {
+        const double c1 = (2.0 * n + 1.0) / (n + 1.0), c0 = (double)n / (n + 1.0);
+        const double a = (c1 * x) * a1 - (c0 * y) * a0;
+        sum += a;
+        if (OP == 1) {
+            const double b = c1 * (dx * a1 + x * b1) - c0 * (dy * a0 + y * b0);
+            dsum += b;
+            b0 = b1;
+            b1 = b;
+        }
+        a0 = a1;
+        a1 = a;
+    }
+    return OP == 1 ? dsum : sum;
+}
+
 // The target-specific sum for many densities (3D Laplace S and D) on the
-// FP64 matrix cores: pot[t][r] (+)= sum_s G(t, s) q[s][r] with G the
-// unit-strength term of tsq_pair_sd -- real for Laplace, computed once per
-// (target, source) pair for all right-hand sides.  A block per unit of
-// tsq_plan: up to TSQ_ROWS QBX targets whose centers share target box it (the
-// A rows: lane i evaluates G for row i % 16 and source k0 + i / 16, exactly
-// the A operand of v_mfma_f64_16x16x4f64), K = the box's list-1 sources in
-// steps of four, shared round-robin by the four waves, columns two tiles of
-// 16 right-hand sides (blockIdx.y chunks of 32).  The waves' partial sums
-// are added in LDS in wave order and written once.
+// FP64 matrix cores: pot[t][r] (+)= sum_s G(t, s) q[s][r], G real, computed
+// once per (target, source) pair for all right-hand sides.  A block per unit
+// of tsq_plan: up to TSQ_ROWS = 64 QBX targets whose centers share target box
+// it, in row tiles of 16 (lane i evaluates G for row i % 16 and source
+// k0 + i / 16, exactly the A operand of v_mfma_f64_16x16x4f64), 32 right-hand
+// sides (blockIdx.y) as two column tiles.  The box's list-1 sources pass
+// through LDS TSQM_CH at a time without regard to box borders, the next
+// chunk's loads in flight while one is summed.  Each wave takes a row tile;
+// with two or one the waves split the sources and add in LDS.  Imaginary
+// parts of the strengths, where a chunk holds any, take a second pass.
+//
+// Bound by the strengths read from L2 (a unit reads its 5900 sources' 32
+// complex strengths; with 16 targets to a unit that was 58 GB) next to 35
+// vector instructions and two matrix products per 64 pairs.  307200 targets,
+// 32 densities, order 3: 15.0 -> 10.0 ms (10.4 without the units' order by
+// XCD; whole eighths of the list to an XCD, 20: the coarse boxes come first).
 typedef double tsq_d4 __attribute__((ext_vector_type(4)));
-constexpr int TSQM_RB = 32;
+constexpr int TSQM_RB = 32, TSQM_CH = 64, TSQM_WS = 48;   // W row stride: banks
 
 template <int OP, int P>
-__global__ void __launch_bounds__(256) k3_tsqbx_mr(int nr, const int *ubox, const int *rows,
+__global__ void __launch_bounds__(256) k3_tsqbx_mr(int nunits, int nr, const int *ubox, const int *rows,
                                                    const int *tree_ttc, const double *ctr,
                                                    int nc, const double *tgt, int nt,
                                                    const double *src, int ns,
@@ -333,94 +378,158 @@ __global__ void __launch_bounds__(256) k3_tsqbx_mr(int nr, const int *ubox, cons
                                                    const double *q, const double *dip,
                                                    double scale, double *pot, int accumulate)
 {
-    __shared__ double part[4][TSQ_ROWS][TSQM_RB][2];
-    const int u = blockIdx.x;
+    __shared__ double sp[(OP == 1 ? 6 : 3) * TSQM_CH];
+    __shared__ double W[TSQM_CH * TSQM_WS];
+    __shared__ int pre[257], first[256], wsum[4], idx[2][TSQM_CH];
+    // eight consecutive units, whose boxes share sources, on one XCD (blocks
+    // go round the eight)
+    const int bi = blockIdx.x;
+    const int u = (bi & ~63) + (bi & 7) * 8 + ((bi >> 3) & 7);
+    if (u >= nunits) return;
     const int it = ubox[u];
     const int tid = threadIdx.x, wv = tid >> 6, lane = tid & 63;
     const int col = lane & 15, kr = lane >> 4;
     const int rb0 = blockIdx.y * TSQM_RB;
     const int nrb = min(TSQM_RB, nr - rb0);
-    // this lane's A row: target ti of center c
-    const int ti = rows[TSQ_ROWS * u + col];
-    const bool rin = ti >= 0;
-    double tc[3] = {0, 0, 0}, cc[3] = {0, 0, 0}, rt = 1.0;
-    if (rin) {
+    // row tiles in use (rows are filled from the front), waves to a tile
+    int ntile = 1;
+    while (ntile < 4 && rows[TSQ_ROWS * u + 16 * ntile] >= 0) ++ntile;
+    const int KG = ntile == 1 ? 4 : ntile == 2 ? 2 : 1;
+    // the wave without a tile (three tiles) is another in each unit
+    const int tile = KG == 1 ? (wv + u) & 3 : wv / KG, kg = wv % KG;
+    const int ti = tile < ntile ? rows[TSQ_ROWS * u + 16 * tile + col] : -1;
+    double tc[3] = {0, 0, 0}, cc[3] = {0, 0, 0};
+    if (ti >= 0) {
         const int c = tree_ttc[ti];
         for (int m = 0; m < 3; ++m) {
             cc[m] = ctr[(size_t)m * nc + c];
             tc[m] = tgt[(size_t)m * nt + ti] - cc[m];
         }
-        rt = sqrt(tc[0] * tc[0] + tc[1] * tc[1] + tc[2] * tc[2]);
     }
-    const zc k0 = {0, 0};
-    tsq_d4 cre[2], cim[2];
-    for (int h = 0; h < 2; ++h) cre[h] = cim[h] = tsq_d4{0, 0, 0, 0};
-    int step = 0;  // K-step counter over the whole list, dealt to the waves
-    for (int e = l1s[it]; e < l1s[it + 1]; ++e) {
-        const int sb = l1l[e];
-        const int s0 = sstart[sb], n = scount[sb];
-        const int nks = (n + 3) / 4;
-        // the K-steps of this box that fall to this wave
-        int ks = (wv - step) & 3;
-        for (; ks < nks; ks += 4) {
-            const int k = ks * 4 + kr;
-            const bool kin = k < n;
-            const int s = s0 + (kin ? k : 0);
-            double g = 0.0;
-            if (rin && kin) {
-                double sc[3], nu[3] = {0, 0, 0};
-                for (int m = 0; m < 3; ++m) sc[m] = src[(size_t)m * ns + s] - cc[m];
-                const double rs = sqrt(sc[0] * sc[0] + sc[1] * sc[1] + sc[2] * sc[2]);
-                const double ct = (tc[0] * sc[0] + tc[1] * sc[1] + tc[2] * sc[2]) / (rt * rs);
-                if (OP == 1)
-                    for (int m = 0; m < 3; ++m) nu[m] = dip[(size_t)m * ns + s];
-                g = tsq_pair_sd<0, OP, P>(k0, tc, rt, nullptr, sc, rs, ct, nu).x;
+    const double rt2 = tc[0] * tc[0] + tc[1] * tc[1] + tc[2] * tc[2];
+    const int e1 = l1s[it + 1];
+    int imag = 0;
+    for (int pass = 0; pass < 2; ++pass) {
+        tsq_d4 acc[2] = {{0, 0, 0, 0}, {0, 0, 0, 0}};
+        for (int eb = l1s[it]; eb < e1; eb += 256) {
+            const int e = eb + tid;
+            int cnt = 0;
+            if (e < e1) {
+                cnt = scount[l1l[e]];
+                first[tid] = sstart[l1l[e]];
             }
-            double bre[2] = {0, 0}, bim[2] = {0, 0};
-            for (int h = 0; h < 2; ++h) {
-                const int r = h * 16 + col;
-                if (kin && r < nrb) {
-                    bre[h] = q[2 * ((size_t)s * nr + rb0 + r)];
-                    bim[h] = q[2 * ((size_t)s * nr + rb0 + r) + 1];
+            int run = cnt;
+            for (int o = 1; o < 64; o <<= 1) {
+                const int y = __shfl_up(run, o);
+                if (lane >= o) run += y;
+            }
+            if (lane == 63) wsum[wv] = run;
+            __syncthreads();
+            for (int w = 0; w < wv; ++w) run += wsum[w];
+            pre[tid + 1] = run;
+            if (tid == 0) pre[0] = 0;
+            __syncthreads();
+            const int total = pre[256];
+            if (total == 0) continue;
+            auto source = [&](int v) {
+                v = min(v, total - 1);
+                int lo = 0, hi = 256;
+                while (hi - lo > 1) {
+                    const int mid = (lo + hi) >> 1;
+                    if (pre[mid] <= v) lo = mid; else hi = mid;
+                }
+                return first[lo] + v - pre[lo];
+            };
+            double x[OP == 1 ? 2 : 1], wr[8];
+            auto fetch = [&](int v0, const int *ix) {
+                // coordinates (and normals): component tid / 64 of a source
+                const int si = ix[tid & 63], m = tid >> 6;
+                if (m < 3) {
+                    x[0] = src[(size_t)m * ns + si];
+                    if (OP == 1) x[OP == 1 ? 1 : 0] = dip[(size_t)m * ns + si];
+                }
+                const int n = total - v0;
+#pragma unroll
+                for (int w = 0; w < 8; ++w) {
+                    const int k = (tid >> 5) + 8 * w, r = tid & 31;
+                    wr[w] = 0.0;
+                    if (k < n && r < nrb) {
+                        const double *z = q + 2 * ((size_t)ix[k] * nr + rb0 + r);
+                        const double zr = z[0], zi = z[1];
+                        imag |= zi != 0.0;
+                        wr[w] = pass ? zi : zr;
+                    }
+                }
+            };
+            if (tid < TSQM_CH) {
+                idx[0][tid] = source(tid);
+                idx[1][tid] = source(TSQM_CH + tid);
+            }
+            __syncthreads();
+            fetch(0, idx[0]);
+            for (int v0 = 0, buf = 1; v0 < total; v0 += TSQM_CH, buf ^= 1) {
+                const int m = tid >> 6;
+                if (m < 3) {
+                    sp[m * TSQM_CH + (tid & 63)] = x[0];
+                    if (OP == 1) sp[(3 + m) * TSQM_CH + (tid & 63)] = x[OP == 1 ? 1 : 0];
+                }
+#pragma unroll
+                for (int w = 0; w < 8; ++w)
+                    W[((tid >> 5) + 8 * w) * TSQM_WS + (tid & 31)] = wr[w];
+                __syncthreads();
+                if (v0 + TSQM_CH < total) fetch(v0 + TSQM_CH, idx[buf]);
+                const int nks = min(TSQM_CH, total - v0 + 3) / 4;
+                if (tile < ntile)
+                    for (int ks = kg; ks < nks; ks += KG) {
+                        const int k = 4 * ks + kr;
+                        double nu[3] = {0, 0, 0};
+                        if (OP == 1)
+                            for (int j = 0; j < 3; ++j) nu[j] = sp[(3 + j) * TSQM_CH + k];
+                        const double g = tsq_laplace<OP, P>(
+                            tc, rt2, sp[k] - cc[0], sp[TSQM_CH + k] - cc[1],
+                            sp[2 * TSQM_CH + k] - cc[2], nu);
+                        acc[0] = __builtin_amdgcn_mfma_f64_16x16x4f64(
+                            g, W[k * TSQM_WS + col], acc[0], 0, 0, 0);
+                        if (nrb > 16)
+                            acc[1] = __builtin_amdgcn_mfma_f64_16x16x4f64(
+                                g, W[k * TSQM_WS + 16 + col], acc[1], 0, 0, 0);
+                    }
+                if (tid < TSQM_CH) idx[buf ^ 1][tid] = source(v0 + 2 * TSQM_CH + tid);
+                __syncthreads();
+            }
+        }
+        // the waves of a tile added (in W), then stored: D register j of lane i
+        // is row 4 j + i / 16, column i % 16
+        for (int w = 1; w < KG; ++w) {
+            __syncthreads();
+            if (kg == w)
+                for (int h = 0; h < 2; ++h)
+                    for (int j = 0; j < 4; ++j) W[(tile * 8 + 4 * h + j) * 64 + lane] = acc[h][j];
+            __syncthreads();
+            if (kg == 0)
+                for (int h = 0; h < 2; ++h)
+                    for (int j = 0; j < 4; ++j) acc[h][j] += W[(tile * 8 + 4 * h + j) * 64 + lane];
+        }
+        if (tile < ntile && kg == 0)
+            for (int j = 0; j < 4; ++j) {
+                const int tr = rows[TSQ_ROWS * u + 16 * tile + 4 * j + kr];
+                if (tr < 0) continue;
+                for (int h = 0; h < 2; ++h) {
+                    const int r = 16 * h + col;
+                    if (r >= nrb) continue;
+                    double *dst = pot + 2 * ((size_t)tr * nr + rb0 + r);
+                    const double v = scale * acc[h][j];
+                    if (pass) {
+                        dst[1] += v;
+                    } else if (accumulate) {
+                        dst[0] += v;
+                    } else {
+                        dst[0] = v;
+                        dst[1] = 0.0;
+                    }
                 }
             }
-            // real strengths (the usual case) need no imaginary-part products;
-            // the test is wave-uniform
-            const bool anyim = __ballot(bim[0] != 0.0 || bim[1] != 0.0) != 0;
-            for (int h = 0; h < 2; ++h) {
-                cre[h] = __builtin_amdgcn_mfma_f64_16x16x4f64(g, bre[h], cre[h], 0, 0, 0);
-                if (anyim)
-                    cim[h] = __builtin_amdgcn_mfma_f64_16x16x4f64(g, bim[h], cim[h], 0, 0, 0);
-            }
-        }
-        step = (step + nks) & 3;
-    }
-    // D register j of lane i: row 4 j + i / 16, column i % 16
-    for (int h = 0; h < 2; ++h)
-        for (int j = 0; j < 4; ++j) {
-            part[wv][4 * j + kr][h * 16 + col][0] = cre[h][j];
-            part[wv][4 * j + kr][h * 16 + col][1] = cim[h][j];
-        }
-    __syncthreads();
-    for (int e = tid; e < TSQ_ROWS * TSQM_RB; e += 256) {
-        const int row = e / TSQM_RB, r = e % TSQM_RB;
-        const int tr = rows[TSQ_ROWS * u + row];
-        if (tr < 0 || r >= nrb) continue;
-        double vr = 0.0, vi = 0.0;
-        for (int w = 0; w < 4; ++w) {
-            vr += part[w][row][r][0];
-            vi += part[w][row][r][1];
-        }
-        vr *= scale;
-        vi *= scale;
-        double *dst = pot + 2 * ((size_t)tr * nr + rb0 + r);
-        if (accumulate) {
-            dst[0] += vr;
-            dst[1] += vi;
-        } else {
-            dst[0] = vr;
-            dst[1] = vi;
-        }
+        if (pass == 0 && !__syncthreads_or(imag)) break;
     }
 }
 
@@ -674,9 +783,9 @@ int tsqbx_nrhs(qbx_ctx *ctx, void *stream, const qbx_tree *T, const qbx_trav *R,
     const unit_plan &V = G->tsq_plan;
     if (V.nunits == 0) return QBX_OK;
     hipStream_t st = S(stream);
-    const dim3 grid(V.nunits, cdiv(nrhs, TSQM_RB));
+    const dim3 grid(64 * cdiv(V.nunits, 64), cdiv(nrhs, TSQM_RB));
 #define TSQM_CASE(OPV, PP)                                                                  \
-    hipLaunchKernelGGL((k3_tsqbx_mr<OPV, PP>), grid, dim3(256), 0, st, nrhs, V.unit_box.p,  \
+    hipLaunchKernelGGL((k3_tsqbx_mr<OPV, PP>), grid, dim3(256), 0, st, V.nunits, nrhs, V.unit_box.p, \
                        G->tsq_rows.p, G->tree_ttc.p, G->centers.p, G->ncenters,            \
                        T->targets.p, T->ntargets, T->sources.p, T->nsources,               \
                        R->l1_starts.p, R->l1_lists.p, T->box_source_starts.p,              \

@@ -1,0 +1,49 @@
+"""GPU: the many-density target-specific sum against the one-density kernel,
+at 1, 16, 17 and 32 densities (one and two column tiles, filled and not), real
+and complex, at the lowest and highest QBX orders, with one to four row tiles
+of targets to a unit and list 1 longer than a tile of 256 entries."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+torch = pytest.importorskip("torch")
+
+
+@pytest.mark.parametrize("pq,kind,nrhs,cplx,leaf", [(0, "S", 1, False, 6), (1, "D", 16, False, 60),
+                                                    (3, "S", 17, True, 300),
+                                                    (5, "D", 32, True, 60),
+                                                    (8, "S", 32, False, 900)])
+def test_many_densities_equal_one(pq, kind, nrhs, cplx, leaf):
+    from pytential_amd import fmm as F
+    from pytential_amd.qbx import QBXLayerPotentialSource
+    from pytential_amd.surface import ellipsoid
+    d = ellipsoid(1, order=3, fine_order=5)
+    src = QBXLayerPotentialSource(d, fine_order=5, qbx_order=pq, fmm_order=3,
+                                  _max_leaf_refine_weight=leaf)
+    geo = src.qbx_fmm_geometry_data((("self", +1),))
+    n1 = np.diff(geo.traversal().neighbor_source_boxes_starts.cpu().numpy())
+    print(f"pq={pq} {kind} nrhs={nrhs}: lists up to {n1.max()}", flush=True)
+    rng = np.random.default_rng(pq)
+    dens = rng.normal(size=(d.ndofs, nrhs))
+    if cplx:
+        dens = dens + 1j * rng.normal(size=dens.shape)
+    st, nrm = None, None
+
+    def wr(n):
+        return F.QBXExpansionWrangler(geo, "laplace", 0.0, kind, pq, [3] * geo.tree().nlevels,
+                                      use_target_specific_qbx=True, nrhs=n)
+    w, w1 = wr(nrhs), wr(1)
+    st, nrm = w.reorder_sources(src.quad_density(dens).reshape(-1, nrhs) if nrhs > 1
+                                else src.quad_density(dens[:, 0]), src.dev["quad_weights"],
+                                src.dev["quad_normals"] if kind == "D" else None)
+    many = torch.zeros((w.tree.ntargets, nrhs), dtype=torch.complex128, device="cuda")
+    from pytential_amd import _lib
+    w._a("qbx_eval_target_specific_qbx_locals_nrhs", w.tree.h, w.traversal.h, w.geo.h,
+         _lib.LAPLACE3D, _lib.TSQBX_D if kind == "D" else _lib.TSQBX_S, pq, nrhs,
+         F._p(st), F._p(nrm), F._p(many), 0)
+    st = st.reshape(-1, nrhs)
+    for c in range(nrhs):
+        one = w1.eval_target_specific_qbx_locals(st[:, c].contiguous(), nrm) * (4 * np.pi)
+        # the bound between forms of the same sum that the repository states
+        assert float((many[:, c] - one).abs().max()) < 1e-12 * float(one.abs().max())
