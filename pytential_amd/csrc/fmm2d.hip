@@ -137,6 +137,44 @@ __device__ __forceinline__ cplx ldpt(const double *x, int n, int i)
     return {x[i], x[(size_t)n + i]};
 }
 
+// The sources of a list of boxes in order, for a one-wave block: load() takes
+// 64 entries, lane l reading entry l's first source and count, and sums the
+// counts; at(v) is source v of them all, its box found by bisection.  A wave
+// that walks box by box waits for each box's number, range and data in turn.
+struct WaveSources {
+    int *pre, *first;   // LDS, 65 and 64
+    int total;
+
+    __device__ __forceinline__ void load(const TD &t, const int *lists, int e, int e1)
+    {
+        const int lane = threadIdx.x;
+        int run = 0;
+        __syncthreads();
+        if (e + lane < e1) {
+            const int Sb = lists[e + lane];
+            run = t.scount[Sb];
+            first[lane] = t.sstart[Sb];
+        }
+        for (int o = 1; o < 64; o <<= 1) {
+            const int y = __shfl_up(run, o);
+            if (lane >= o) run += y;
+        }
+        pre[lane + 1] = run;
+        if (lane == 0) pre[0] = 0;
+        __syncthreads();
+        total = pre[64];
+    }
+
+    __device__ __forceinline__ int at(int v) const
+    {
+        int lo = 0;
+#pragma unroll
+        for (int w = 32; w >= 1; w >>= 1)
+            if (pre[lo + w] <= v) lo += w;
+        return first[lo] + v - pre[lo];
+    }
+};
+
 // coefficient 0 (Helmholtz: n = 0, centred), right-hand side 0 of box b;
 // coefficient n, right-hand side r at [2 (n nr + r)]
 __device__ __forceinline__ long ecoef_off(const KD &kd, int b, int lv)
@@ -444,6 +482,116 @@ __global__ void k_p2l(KD kd, TD t, Flat fl, const int *ttp, const int *starts, c
         }
 }
 
+// Laplace P2M / P2L, a wavefront per box and 64 sources at a time: each lane
+// writes its source's powers (basis of coefficient l without the constant
+// factor) to LDS by recurrence, then NL lanes per share of the sources sum
+// them against the strengths.  Every level in one launch.  Latency bound; a
+// thread per coefficient, raising each source to its power anew, took 108 us
+// for the list-4 sums of a 16384-node curve (37436 (box, source) pairs, order 15)
+// and 30 us for its multipoles, now 8.9 and 5.6.
+constexpr int LAP_PMAX = 40;   // 41 x 65 complex powers: 42.6 KB
+
+template <int NRC, bool LOCAL>
+__global__ void __launch_bounds__(64) k_p2e_lap(KD kd, TD t, const int *boxes, const int *starts,
+                                                const int *lists, const double *src, int ns,
+                                                const double *str, const double *nrm,
+                                                double *expn)
+{
+    extern __shared__ double lds[];
+    __shared__ double Qs[64 * 2 * NRC];
+    __shared__ int pre[65], first[64];
+    const int i = blockIdx.x;
+    int e0 = 0, e1 = 1;
+    if (LOCAL) {
+        e0 = starts[i];
+        e1 = starts[i + 1];
+        if (e0 == e1) return;
+    }
+    const int Bx = boxes[i];
+    const int lv = t.level[Bx], p = kd.order[lv];
+    const double R = kd.rscale[lv], iR = 1.0 / R;
+    const cplx c = boxc(t, Bx);
+    const int lane = threadIdx.x, rc = kd.rc, r0 = kd.r0, nr = kd.nr;
+    const bool dip = kd.dip;
+    cplx *Z = reinterpret_cast<cplx *>(lds);   // [p + 1][65]
+    int NL = 16;
+    while (NL < p + 1) NL <<= 1;
+    const int l = lane & (NL - 1), share = lane / NL, SH = 64 / NL;
+    cplx acc[NRC];
+#pragma unroll
+    for (int q = 0; q < NRC; ++q) acc[q] = {0, 0};
+    WaveSources ws{pre, first, 0};
+    for (int e = e0; e < e1; e += 64) {
+        if (LOCAL)
+            ws.load(t, lists, e, e1);
+        else
+            ws.load(t, boxes + i, 0, 1);
+        for (int v0 = 0; v0 < ws.total; v0 += 64) {
+            const int n = min(64, ws.total - v0);
+            __syncthreads();
+            if (lane < n) {
+                const int si = ws.at(v0 + lane);
+                const cplx w = ldpt(src, ns, si) - c;
+                const cplx iw = LOCAL ? cinv(w) : cplx{0, 0};
+                const cplx tt = LOCAL ? R * iw : iR * w;
+                cplx z = {1, 0};
+                int j = 0;
+                if (LOCAL) {
+                    if (dip) {
+                        z = ldpt(nrm, ns, si) * iw;
+                    } else {
+                        Z[lane] = clogz(-w);
+                        z = tt;
+                        j = 1;
+                    }
+                } else if (dip) {
+                    Z[lane] = {0, 0};
+                    z = ldpt(nrm, ns, si);
+                    j = 1;
+                }
+                for (; j <= p; ++j) {
+                    Z[j * 65 + lane] = z;
+                    z = z * tt;
+                }
+#pragma unroll
+                for (int q = 0; q < NRC; ++q)
+                    if (q < rc) {
+                        const cplx v = ldq(kd, str, si, r0 + q);
+                        Qs[2 * (lane * NRC + q)] = v.x;
+                        Qs[2 * (lane * NRC + q) + 1] = v.y;
+                    }
+            }
+            __syncthreads();
+            if (l <= p)
+                for (int s = share; s < n; s += SH) {
+                    const cplx z = Z[l * 65 + s];
+#pragma unroll
+                    for (int q = 0; q < NRC; ++q)
+                        if (q < rc)
+                            acc[q] += cplx{Qs[2 * (s * NRC + q)], Qs[2 * (s * NRC + q) + 1]} * z;
+                }
+        }
+    }
+    // the factors: -1/l (S), -1/R (D multipoles), 1
+    const double f = dip ? (LOCAL ? 1.0 : -iR) : (l > 0 ? -1.0 / l : 1.0);
+#pragma unroll
+    for (int q = 0; q < NRC; ++q)
+        for (int m = NL; m < 64; m <<= 1) {
+            acc[q].x += __shfl_xor(acc[q].x, m);
+            acc[q].y += __shfl_xor(acc[q].y, m);
+        }
+    if (share == 0 && l <= p) {
+        double *o = expn + ecoef_off(kd, Bx, lv) + 2L * l * nr;
+#pragma unroll
+        for (int q = 0; q < NRC; ++q)
+            if (q < rc) {
+                double *d = o + 2 * (r0 + q);
+                const cplx v = f * acc[q];
+                stc(d, LOCAL ? ldc(d) + v : v);
+            }
+    }
+}
+
 // -------------------------------------------------------------------------
 // Helmholtz P2M / P2L through LDS, one block per box.  Sources are taken S
 // at a time.  Phase A (one lane per source) runs the source's sequence once:
@@ -462,7 +610,7 @@ struct P2EShape {
 };
 
 template <int NRC, bool LOCAL>
-__global__ void __launch_bounds__(256) k_p2e_h(KD kd, TD t, int lv, int i0, P2EShape sh, const int *boxes,
+__global__ void __launch_bounds__(256) k_p2e_h(KD kd, TD t, int i0, P2EShape sh, const int *boxes,
                         const int *starts, const int *lists, const double *src, int ns,
                         const double *str, const double *nrm, double *expn)
 {
@@ -475,7 +623,7 @@ __global__ void __launch_bounds__(256) k_p2e_h(KD kd, TD t, int lv, int i0, P2ES
         e1 = starts[i + 1];
         if (e0 == e1) return;
     }
-    const int p = kd.order[lv];
+    const int lv = t.level[Bx], p = kd.order[lv];
     const int S = sh.S, R = sh.R;
     double *Gp = lds, *Gm = Gp + 2 * S * R, *Qs = Gm + 2 * S * R, *Nu = Qs + 2 * S * NRC;
     int *idx = (int *)(Nu + 2 * S);
@@ -862,6 +1010,101 @@ __global__ void k_m2m(KD kd, TD t, const double *B, int lvp, int i0, int i1, con
         }
     }
     store_add<NRC>(kd, mpole + ecoef_off(kd, P, lvp) + 2L * m * kd.nr, acc);
+}
+
+// Laplace M2M (OP 0: parents of level lv from their children) and L2L (OP 1:
+// boxes of level lv from their parents).  NL lanes (the coefficients, a power
+// of two) per input box, 4 NL or NL per output box, several output boxes to a
+// block of 256; the inputs, scaled by the ratio of the levels' scales, and the
+// binomials are staged in LDS, so that the Horner chains wait for no memory:
+// as one thread per coefficient over global reads a level took 19 us at order
+// 15 (M2M, 7.3 L2L), now 5.7 and 5.2.
+template <int OP, int NRC>
+__global__ void __launch_bounds__(256) k_lap_shift(KD kd, TD t, const double *B, int lv, int i0,
+                                                   int i1, const int *boxes, double *expn)
+{
+    extern __shared__ double lds[];
+    const int lin = OP == 0 ? lv + 1 : lv - 1;
+    const int p1 = kd.order[lin], p2 = kd.order[lv];
+    int NL = 16;
+    while (NL < p2 + 1) NL <<= 1;
+    constexpr int NE = OP == 0 ? 4 : 1;
+    const int nslot = 256 / (NE * NL);
+    const int tid = threadIdx.x, l = tid & (NL - 1), e = (tid / NL) & (NE - 1),
+              slot = tid / (NE * NL);
+    const int pb = OP == 0 ? p2 : p1;            // binomials C(n, k), n <= pb
+    double *Bs = lds;                             // [pb + 1][pb + 1]
+    cplx *A = reinterpret_cast<cplx *>(Bs + ((pb + 1) * (pb + 1) + 1) / 2 * 2);
+    for (int q = tid; q < (pb + 1) * (pb + 1); q += 256)
+        Bs[q] = B[(q / (pb + 1)) * BINOM_N + q % (pb + 1)];
+    const int i = i0 + blockIdx.x * nslot + slot;
+    const double R1 = kd.rscale[lin], R2 = kd.rscale[lv];
+    int P = -1, C = -1;
+    if (i < i1) {
+        P = boxes[i];
+        if (OP == 0) {
+            C = t.child[(size_t)e * t.nboxes + P];
+            if (C >= 0 && t.scumul[C] == 0) C = -1;
+        } else {
+            C = t.parent[P];
+        }
+    }
+    cplx *a = A + (slot * NE + e) * (p1 + 1) * NRC;
+    if (C >= 0) {
+        const double *g = expn + ecoef_off(kd, C, lin);
+        const double r = OP == 0 ? R1 / R2 : 1.0;
+        for (int k = l; k <= p1; k += NL) {
+            double rk = 1.0;
+            for (int j = 0; j < k; ++j) rk *= r;
+#pragma unroll
+            for (int q = 0; q < NRC; ++q)
+                a[k * NRC + q] = q < kd.rc ? rk * ldcn(kd, g, k, kd.r0 + q) : cplx{0, 0};
+        }
+    }
+    __syncthreads();
+    cplx h[NRC];
+#pragma unroll
+    for (int q = 0; q < NRC; ++q) h[q] = {0, 0};
+    if (C >= 0 && l <= p2) {
+        if (OP == 0) {
+            const cplx u = (1.0 / R2) * (boxc(t, C) - boxc(t, P));
+#pragma unroll
+            for (int q = 0; q < NRC; ++q) h[q] = l > 0 ? (-1.0 / l) * a[q] : a[q];
+            const int kmax = min(l, p1);
+            for (int k = 1; k <= kmax; ++k) {
+                const double b = Bs[(l - 1) * (pb + 1) + k - 1];
+#pragma unroll
+                for (int q = 0; q < NRC; ++q) h[q] = h[q] * u + b * a[k * NRC + q];
+            }
+            for (int k = kmax; k < l; ++k)
+#pragma unroll
+                for (int q = 0; q < NRC; ++q) h[q] = h[q] * u;
+        } else if (l <= p1) {
+            const cplx u = (1.0 / R1) * (boxc(t, P) - boxc(t, C));
+            for (int k = p1; k >= l; --k) {
+                const double b = Bs[k * (pb + 1) + l];
+#pragma unroll
+                for (int q = 0; q < NRC; ++q) h[q] = h[q] * u + b * a[k * NRC + q];
+            }
+            double rp = 1.0;
+            for (int k = 0; k < l; ++k) rp *= R2 / R1;
+#pragma unroll
+            for (int q = 0; q < NRC; ++q) h[q] = rp * h[q];
+        }
+    }
+    if (OP == 0) {
+        // the four children's shifts, over the staged inputs
+        __syncthreads();
+#pragma unroll
+        for (int q = 0; q < NRC; ++q) A[tid * NRC + q] = h[q];
+        __syncthreads();
+        if (e > 0) return;
+        for (int c = 1; c < 4; ++c)
+#pragma unroll
+            for (int q = 0; q < NRC; ++q) h[q] += A[(tid + c * NL) * NRC + q];
+    }
+    if (P >= 0 && C + (OP == 0 ? 1 : 0) >= 0 && l <= p2)
+        store_add<NRC>(kd, expn + ecoef_off(kd, P, lv) + 2L * l * kd.nr, h);
 }
 
 // M2L with one block per target-or-target-parent box (fl: one entry per box):
@@ -1770,6 +2013,7 @@ __global__ void __launch_bounds__(64) k_p2p(KD kd, TD t, const int *ubox, const 
     __shared__ double sx[CH], sy[CH], snx[CH], sny[CH];
     __shared__ double sq[CH * 2 * NRC];
     __shared__ __align__(16) double htab[4 * HANKEL_NSER];
+    __shared__ int pre[65], first[64];
     const int u = blockIdx.x;
     const int it = ubox[u];
     const int B = tboxes[it];
@@ -1812,16 +2056,14 @@ __global__ void __launch_bounds__(64) k_p2p(KD kd, TD t, const int *ubox, const 
         __syncthreads();
     };
 
-    int fill = 0;
+    WaveSources ws{pre, first, 0};
     const int e1 = starts[it + 1];
-    for (int e = starts[it]; e < e1; ++e) {
-        const int Sb = lists[e];
-        int s = t.sstart[Sb];
-        const int s1 = s + t.scount[Sb];
-        while (s < s1) {
-            const int take = min(s1 - s, CH - fill);
-            for (int j = lane; j < take; j += 64) {
-                const int si = s + j, d = fill + j;
+    for (int e = starts[it]; e < e1; e += 64) {
+        ws.load(t, lists, e, e1);
+        for (int v0 = 0; v0 < ws.total; v0 += CH) {
+            const int n = min(CH, ws.total - v0);
+            for (int d = lane; d < n; d += 64) {
+                const int si = ws.at(v0 + d);
                 sx[d] = src[si];
                 sy[d] = src[(size_t)ns + si];
                 if (dip) {
@@ -1836,15 +2078,9 @@ __global__ void __launch_bounds__(64) k_p2p(KD kd, TD t, const int *ubox, const 
                         sq[2 * (d * NRC + q) + 1] = p[1];
                     }
             }
-            fill += take;
-            s += take;
-            if (fill == CH) {
-                flush(CH);
-                fill = 0;
-            }
+            flush(n);
         }
     }
-    if (fill > 0) flush(fill);
 #pragma unroll
     for (int q = 0; q < NRC; ++q)
         for (int m = G / 2; m >= 1; m >>= 1) {
@@ -2059,7 +2295,7 @@ struct P2QTile {
     static constexpr int CH = NRC == 1 ? 256 : 64;
 };
 
-template <int PQ, int NRC, int KN = -1, int DP = -1>
+template <int PQ, int NRC, int KN, int DP>
 __global__ void __launch_bounds__(64) k_p2qbxl(KD kd, TD t, const int *ubox, const int *ut0,
                                                const int *box_g, const int *gcs,
                                                const int *gcl, const double *ctr,
@@ -2072,6 +2308,7 @@ __global__ void __launch_bounds__(64) k_p2qbxl(KD kd, TD t, const int *ubox, con
     __shared__ double sx[CH], sy[CH], snx[CH], sny[CH];
     __shared__ double sq[CH * 2 * NRC];
     __shared__ __align__(16) double htab[4 * HANKEL_NSER];
+    __shared__ int pre[65], first[64];
     const int u = blockIdx.x;
     const int it = ubox[u];
     const int G = box_g[it];
@@ -2114,16 +2351,14 @@ __global__ void __launch_bounds__(64) k_p2qbxl(KD kd, TD t, const int *ubox, con
         __syncthreads();
     };
 
-    int fill = 0;
+    WaveSources ws{pre, first, 0};
     const int e1 = l1s[it + 1];
-    for (int e = l1s[it]; e < e1; ++e) {
-        const int Sb = l1l[e];
-        int s = t.sstart[Sb];
-        const int s1 = s + t.scount[Sb];
-        while (s < s1) {
-            const int take = min(s1 - s, CH - fill);
-            for (int j = lane; j < take; j += 64) {
-                const int si = s + j, d = fill + j;
+    for (int e = l1s[it]; e < e1; e += 64) {
+        ws.load(t, l1l, e, e1);
+        for (int v0 = 0; v0 < ws.total; v0 += CH) {
+            const int n = min(CH, ws.total - v0);
+            for (int d = lane; d < n; d += 64) {
+                const int si = ws.at(v0 + d);
                 sx[d] = src[si];
                 sy[d] = src[(size_t)ns + si];
                 if (dip) {
@@ -2138,15 +2373,9 @@ __global__ void __launch_bounds__(64) k_p2qbxl(KD kd, TD t, const int *ubox, con
                         sq[2 * (d * NRC + q) + 1] = pq[1];
                     }
             }
-            fill += take;
-            s += take;
-            if (fill == CH) {
-                flush(CH);
-                fill = 0;
-            }
+            flush(n);
         }
     }
-    if (fill > 0) flush(fill);
     qacc_group_reduce<PQ, NRC>(A, G);
     if (active && sub == 0) qbx_store<PQ, NRC>(kd, qexp, c, A, accumulate);
 }
@@ -3347,21 +3576,63 @@ static Flat make_flat(const KD &kd, const std::vector<int> &level_starts, bool h
 
 static inline long exp_bytes(const KD &kd) { return 16L * kd.lcoef[kd.nlevels] * kd.nr; }
 
-// Helmholtz P2M (LDS kernel) of the source boxes at level l; the levels are
-// independent (each writes its own boxes)
+// 2D Laplace at orders the LDS kernels hold
+static bool lap_fits(const KD &kd)
+{
+    bool ok = kd.kernel == QBX_LAPLACE2D;
+    for (int l = 0; l < kd.nlevels; ++l) ok = ok && kd.order[l] <= LAP_PMAX;
+    return ok;
+}
+
+// dynamic LDS of k_p2e_lap: the powers to the largest order
+static size_t lap_p2e_bytes(const KD &kd)
+{
+    int p = 0;
+    for (int l = 0; l < kd.nlevels; ++l) p = std::max(p, kd.order[l]);
+    return sizeof(cplx) * 65 * (p + 1);
+}
+
+// M2M (OP 0) or L2L (OP 1) of one level by k_lap_shift
+template <int OP>
+static void lap_shift_level(hipStream_t st, KD &kd, const TD &td, const double *B, int lv, int i0,
+                            int i1, const int *boxes, double *expn)
+{
+    const int p1 = kd.order[OP == 0 ? lv + 1 : lv - 1], p2 = kd.order[lv];
+    int NL = 16;
+    while (NL < p2 + 1) NL <<= 1;
+    const int ne = OP == 0 ? 4 : 1, nslot = 256 / (ne * NL), pb = OP == 0 ? p2 : p1;
+#define L_SHIFT(N)                                                                         \
+    hipLaunchKernelGGL((k_lap_shift<OP, N>), dim3(cdiv(i1 - i0, nslot)), dim3(256),        \
+                       sizeof(double) * (((pb + 1) * (pb + 1) + 1) / 2 * 2) +              \
+                           sizeof(cplx) * (N) * std::max(256, nslot * ne * (p1 + 1)),      \
+                       st, kd, td, B, lv, i0, i1, boxes, expn)
+    FOR_RHS_CHUNKS(kd, NRC_Q, L_SHIFT);
+#undef L_SHIFT
+}
+
+// first level above l of another order
+static int next_order(const KD &kd, int l)
+{
+    int l1 = l + 1;
+    while (l1 < kd.nlevels && kd.order[l1] == kd.order[l]) ++l1;
+    return l1;
+}
+
+// Helmholtz P2M (LDS kernel) of the source boxes at levels l .. l1 - 1, of one
+// order; the levels are independent (each writes its own boxes)
 static void p2m_level_h(hipStream_t st, KD &kd, const TD &td, const qbx_tree *T,
-                        const qbx_trav *R, int l, const double *str, const double *nrm,
+                        const qbx_trav *R, int l, int l1, const double *str, const double *nrm,
                         double *mpole)
 {
     const int i0 = R->h_level_start_source_box_nrs[l];
-    const int i1 = R->h_level_start_source_box_nrs[l + 1];
+    const int i1 = R->h_level_start_source_box_nrs[l1];
     if (i1 == i0) return;
     P2EShape sh;
     int th;
     size_t by;
     p2e_launch(kd, kd.order[l], &sh, &th, &by);
 #define L_P2MH(N)                                                                          \
-    hipLaunchKernelGGL((k_p2e_h<N, false>), dim3(i1 - i0), dim3(th), by, st, kd, td, l, i0, sh, \
+    hipLaunchKernelGGL((k_p2e_h<N, false>), dim3(i1 - i0), dim3(th), by, st, kd, td, i0, sh, \
                        R->source_boxes.p, nullptr, nullptr, T->sources.p, T->nsources, str,  \
                        nrm, mpole)
     FOR_RHS_CHUNKS(kd, NRC_S, L_P2MH);
@@ -3406,7 +3677,7 @@ static int p2m_multistream(qbx_ctx *ctx, hipStream_t *sts, int nst, hipEvent_t *
     for (size_t k = 0; k < order.size(); ++k) {
         const int j = (int)(std::min_element(load.begin(), load.end()) - load.begin());
         load[j] -= order[k].first;
-        p2m_level_h(sts[j], kd, td, T, R, order[k].second, str, nrm, mpole);
+        p2m_level_h(sts[j], kd, td, T, R, order[k].second, order[k].second + 1, str, nrm, mpole);
     }
     QBX_HIP(hipGetLastError());
     for (int k = 1; k < nst; ++k) {
@@ -3592,10 +3863,24 @@ int qbx_form_multipoles(qbx_ctx *ctx, void *stream, const qbx_tree *T, const qbx
         }
         if (ok) {
             const TD td = make_td(T);
-            for (int l = 0; l < T->nlevels; ++l) p2m_level_h(st, kd, td, T, R, l, str, nrm, mpole);
+            for (int l = 0, l1; l < T->nlevels; l = l1) {
+                l1 = next_order(kd, l);
+                p2m_level_h(st, kd, td, T, R, l, l1, str, nrm, mpole);
+            }
             QBX_HIP(hipGetLastError());
             return QBX_OK;
         }
+    }
+    if (lap_fits(kd)) {
+        const TD td = make_td(T);
+#define L_P2ML(N)                                                                          \
+    hipLaunchKernelGGL((k_p2e_lap<N, false>), dim3(R->nsource_boxes), dim3(64),            \
+                       lap_p2e_bytes(kd), st, kd, td, R->source_boxes.p, nullptr, nullptr, \
+                       T->sources.p, T->nsources, str, nrm, mpole)
+        if (R->nsource_boxes > 0) FOR_RHS_CHUNKS(kd, NRC_S, L_P2ML);
+#undef L_P2ML
+        QBX_HIP(hipGetLastError());
+        return QBX_OK;
     }
     const Flat fl = make_flat(kd, R->h_level_start_source_box_nrs, true);
     const long nthr = fl.tstart[fl.nl];
@@ -3644,6 +3929,10 @@ static int coarsen_multipoles_from(qbx_ctx *ctx, void *stream, const qbx_tree *T
                 hipLaunchKernelGGL(k_shift_mfma<0>, dim3(i1 - i0), dim3(256), 0, st, kd, td, l,
                                    i0, R->source_parent_boxes.p, mpole);
             }
+            continue;
+        }
+        if (lap_fits(kd)) {
+            lap_shift_level<0>(st, kd, td, B, l, i0, i1, R->source_parent_boxes.p, mpole);
             continue;
         }
         HtLaunch hl;
@@ -3941,16 +4230,17 @@ int qbx_form_locals(qbx_ctx *ctx, void *stream, const qbx_tree *T, const qbx_tra
         }
         if (ok) {
             const TD td = make_td(T);
-            for (int l = 0; l < T->nlevels; ++l) {
+            for (int l = 0, l1; l < T->nlevels; l = l1) {
+                l1 = next_order(kd, l);
                 const int i0 = R->h_level_start_ttp_box_nrs[l];
-                const int i1 = R->h_level_start_ttp_box_nrs[l + 1];
+                const int i1 = R->h_level_start_ttp_box_nrs[l1];
                 if (i1 == i0) continue;
                 P2EShape sh;
                 int th;
                 size_t by;
                 p2e_launch(kd, kd.order[l], &sh, &th, &by);
 #define L_P2LH(N)                                                                          \
-    hipLaunchKernelGGL((k_p2e_h<N, true>), dim3(i1 - i0), dim3(th), by, st, kd, td, l, i0, sh, \
+    hipLaunchKernelGGL((k_p2e_h<N, true>), dim3(i1 - i0), dim3(th), by, st, kd, td, i0, sh, \
                        R->ttp_boxes.p, R->l4_starts.p, R->l4_lists.p, T->sources.p,         \
                        T->nsources, str, nrm, local)
                 FOR_RHS_CHUNKS(kd, NRC_S, L_P2LH);
@@ -3959,6 +4249,17 @@ int qbx_form_locals(qbx_ctx *ctx, void *stream, const qbx_tree *T, const qbx_tra
             QBX_HIP(hipGetLastError());
             return QBX_OK;
         }
+    }
+    if (lap_fits(kd)) {
+        const TD td = make_td(T);
+#define L_P2LL(N)                                                                          \
+    hipLaunchKernelGGL((k_p2e_lap<N, true>), dim3(R->nttp_boxes), dim3(64),                \
+                       lap_p2e_bytes(kd), st, kd, td, R->ttp_boxes.p, R->l4_starts.p,      \
+                       R->l4_lists.p, T->sources.p, T->nsources, str, nrm, local)
+        if (R->nttp_boxes > 0 && R->n4 > 0) FOR_RHS_CHUNKS(kd, NRC_S, L_P2LL);
+#undef L_P2LL
+        QBX_HIP(hipGetLastError());
+        return QBX_OK;
     }
     const Flat fl = make_flat(kd, R->h_level_start_ttp_box_nrs, true);
     const long nthr = fl.tstart[fl.nl];
@@ -4006,6 +4307,10 @@ static int refine_locals_from(qbx_ctx *ctx, void *stream, const qbx_tree *T, con
                 hipLaunchKernelGGL(k_shift_mfma<1>, dim3(i1 - i0), dim3(256), 0, st, kd, td, l,
                                    i0, R->ttp_boxes.p, local);
             }
+            continue;
+        }
+        if (lap_fits(kd)) {
+            lap_shift_level<1>(st, kd, td, B, l, i0, i1, R->ttp_boxes.p, local);
             continue;
         }
         HtLaunch hl;
@@ -4075,49 +4380,34 @@ int qbx_form_global_qbx_locals(qbx_ctx *ctx, void *stream, const qbx_tree *T, co
         QBX_HIP(hipGetLastError());
         return QBX_OK;
     }
-    if (kd.kernel == QBX_HELMHOLTZ2D && kd.nr == 1) {
-        // one Helmholtz density: the kernel and source kind fixed at compile time
-#define L_P2QH(PQV, DV)                                                                    \
-    hipLaunchKernelGGL((k_p2qbxl<PQV, 1, QBX_HELMHOLTZ2D, DV>), dim3(U.nunits), dim3(64), 0, \
-                       st, kd, td, U.unit_box.p, U.unit_t0.p, U.box_g.p,                   \
-                       G->gc_by_tbox_starts.p, G->gc_by_tbox.p, G->centers.p, G->radii.p,  \
-                       G->ncenters, R->l1_starts.p, R->l1_lists.p, T->sources.p,           \
-                       T->nsources, str, nrm, qexp, accumulate)
-#define L_P2QHD(PQV)          \
-    if (kd.dip)               \
-        L_P2QH(PQV, 1);       \
-    else                      \
-        L_P2QH(PQV, 0)
-        kd.r0 = 0;
-        kd.rc = 1;
-        switch (kd.pq) {
-        case 0: L_P2QHD(0); break;
-        case 1: L_P2QHD(1); break;
-        case 2: L_P2QHD(2); break;
-        case 3: L_P2QHD(3); break;
-        case 4: L_P2QHD(4); break;
-        case 5: L_P2QHD(5); break;
-        case 6: L_P2QHD(6); break;
-        case 7: L_P2QHD(7); break;
-        case 8: L_P2QHD(8); break;
-        case 9: L_P2QHD(9); break;
-        case 10: L_P2QHD(10); break;
-        case 11: L_P2QHD(11); break;
-        case 12: L_P2QHD(12); break;
-        default: set_error("qbx_order out of range"); return QBX_ERR_INVALID;
-        }
-#undef L_P2QHD
-#undef L_P2QH
-        QBX_HIP(hipGetLastError());
-        return QBX_OK;
-    }
+    // the kernel and source kind fixed at compile time
+#define L_P2QK(PQV, N, KV, DV)                                                             \
+    hipLaunchKernelGGL((k_p2qbxl<PQV, N, KV, DV>), dim3(U.nunits), dim3(64), 0, st, kd, td, \
+                       U.unit_box.p, U.unit_t0.p, U.box_g.p, G->gc_by_tbox_starts.p,        \
+                       G->gc_by_tbox.p, G->centers.p, G->radii.p, G->ncenters,              \
+                       R->l1_starts.p, R->l1_lists.p, T->sources.p, T->nsources, str, nrm,  \
+                       qexp, accumulate)
+#define L_P2QD(PQV, N)                                                                     \
+    case PQV:                                                                              \
+        if (kd.kernel == QBX_LAPLACE2D) {                                                  \
+            if (kd.dip) L_P2QK(PQV, N, QBX_LAPLACE2D, 1);                                  \
+            else L_P2QK(PQV, N, QBX_LAPLACE2D, 0);                                         \
+        } else {                                                                           \
+            if (kd.dip) L_P2QK(PQV, N, QBX_HELMHOLTZ2D, 1);                                \
+            else L_P2QK(PQV, N, QBX_HELMHOLTZ2D, 0);                                       \
+        }                                                                                  \
+        break;
 #define L_P2Q(N)                                                                           \
-    DISPATCH_PQ_NR(kd.pq, N, k_p2qbxl, dim3(U.nunits), dim3(64), 0, st, kd, td,            \
-                   U.unit_box.p, U.unit_t0.p, U.box_g.p, G->gc_by_tbox_starts.p,            \
-                   G->gc_by_tbox.p, G->centers.p, G->radii.p, G->ncenters, R->l1_starts.p,  \
-                   R->l1_lists.p, T->sources.p, T->nsources, str, nrm, qexp, accumulate)
+    switch (kd.pq) {                                                                       \
+        L_P2QD(0, N) L_P2QD(1, N) L_P2QD(2, N) L_P2QD(3, N) L_P2QD(4, N) L_P2QD(5, N)      \
+        L_P2QD(6, N) L_P2QD(7, N) L_P2QD(8, N) L_P2QD(9, N) L_P2QD(10, N) L_P2QD(11, N)    \
+        L_P2QD(12, N)                                                                      \
+    default: set_error("qbx_order out of range"); return QBX_ERR_INVALID;                  \
+    }
     FOR_RHS_CHUNKS(kd, NRC_Q, L_P2Q);
 #undef L_P2Q
+#undef L_P2QD
+#undef L_P2QK
     QBX_HIP(hipGetLastError());
     return QBX_OK;
 }
