@@ -692,6 +692,49 @@ struct SWaveSums {
 // and 16 complex products of the waves took half of 560 instruction slots.
 constexpr int P2Q_CH = 256;
 
+// First sources and running source counts of the CH list entries from e0 (a
+// thread each of a block of CH): entry i's sources are pre[i] .. pre[i + 1] - 1
+// of the tile.  wsum: a word per wave.  Ends with a barrier.
+template <int CH>
+__device__ __forceinline__ void list_counts(const TD &t, int e0, int e1, const int *lists,
+                                            int *first, int *pre, int *wsum)
+{
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int e = e0 + tid;
+    int cnt = 0;
+    if (e < e1) {
+        const int Sb = lists[e];
+        cnt = t.scount[Sb];
+        first[tid] = t.sstart[Sb];
+    }
+    int run = cnt;
+    for (int o = 1; o < 64; o <<= 1) {
+        const int y = __shfl_up(run, o);
+        if (lane >= o) run += y;
+    }
+    if (lane == 63) wsum[wave] = run;
+    __syncthreads();
+    for (int w = 0; w < wave; ++w) run += wsum[w];
+    pre[tid + 1] = run;
+    if (tid == 0) pre[0] = 0;
+    __syncthreads();
+}
+
+// source v of the tile
+template <int CH>
+__device__ __forceinline__ int list_source(const int *first, const int *pre, int v)
+{
+    int lo = 0, hi = CH;  // pre[lo] <= v < pre[hi]
+    while (hi - lo > 1) {
+        const int mid = (lo + hi) >> 1;
+        if (pre[mid] <= v)
+            lo = mid;
+        else
+            hi = mid;
+    }
+    return first[lo] + v - pre[lo];
+}
+
 template <int PQ, int DIP>
 __global__ void __launch_bounds__(256) kh_p2qbxl_reg(HD hd, TD t, const int *ubox,
                                                      const int *uc0, const int *gcs,
@@ -730,37 +773,14 @@ __global__ void __launch_bounds__(256) kh_p2qbxl_reg(HD hd, TD t, const int *ubo
     }
     const int e1 = starts[it + 1];
     for (int e0 = starts[it]; e0 < e1; e0 += P2Q_CH) {
-        // the entries' first sources and running counts
-        const int e = e0 + tid;
-        int cnt = 0;
-        if (e < e1) {
-            const int Sb = lists[e];
-            cnt = t.scount[Sb];
-            first[tid] = t.sstart[Sb];
-        }
-        int run = cnt;
-        for (int o = 1; o < 64; o <<= 1) {
-            const int y = __shfl_up(run, o);
-            if (lane >= o) run += y;
-        }
-        if (lane == 63) wsum[wave] = run;
-        __syncthreads();
-        for (int w = 0; w < wave; ++w) run += wsum[w];
-        pre[tid + 1] = run;
-        if (tid == 0) pre[0] = 0;
-        __syncthreads();
+        list_counts<P2Q_CH>(t, e0, e1, lists, first, pre, wsum);
         const int total = pre[P2Q_CH];
         double2 rxy = {0, 0}, rzq = {0, 0};
         double rqi = 0;
         v3 rnu = {0, 0, 0};
         auto fetch = [&](int v) {
             if (v >= total) return;
-            int lo = 0, hi = P2Q_CH;   // pre[lo] <= v < pre[hi]
-            while (hi - lo > 1) {
-                const int mid = (lo + hi) >> 1;
-                if (pre[mid] <= v) lo = mid; else hi = mid;
-            }
-            const int si = first[lo] + v - pre[lo];
+            const int si = list_source<P2Q_CH>(first, pre, v);
             const double *q = str + 2 * ((size_t)si * hd.nr + hd.r0);
             rxy = {src[si], src[(size_t)ns + si]};
             rzq = {src[2 * (size_t)ns + si], q[0]};
@@ -828,6 +848,263 @@ __global__ void __launch_bounds__(256) kh_p2qbxl_reg(HD hd, TD t, const int *ubo
         double *dst = qexp + 2 * (((size_t)ci * NC + lane) * hd.nr + hd.r0);
         dst[0] += v.x;
         dst[1] += v.y;
+    }
+}
+
+// P2L for one density at a time, charges only, in registers (order P <= P2L_PMAX
+// and the sine's reduced range as in P2QBXL).  A block takes a box; its list-4
+// sources pass through LDS as in kh_p2qbxl_reg, a lane per source.  The 2 (P+1)^2
+// real sums of SWaveSums do not fit a lane at box orders, so the columns m are
+// dealt to ROLES wavefronts (largest first to the emptiest), each of which
+// repeats the radial sequence and keeps at most 64 sums; the wavefronts of a
+// role share the sources of a role.  The lanes' sums are added by a
+// reduce-scatter, 63 exchanges for 64 sums.
+//
+// FP64 VALU bound.  14.3e6 (box, source) pairs at order 10: 8.5 ms with waves
+// of 8 sources at a time in LDS, their radial sequences by 8 lanes and a thread
+// per coefficient; now 1.5
+// (1.65 with 8 roles at this order, for more wavefronts in flight).
+constexpr int P2L_PMAX = 12;
+constexpr int p2l_roles(int P) { return P <= 4 ? 1 : P <= 6 ? 2 : P <= 10 ? 4 : 8; }
+constexpr int p2l_threads(int P) { return 64 * (p2l_roles(P) > 4 ? p2l_roles(P) : 4); }
+
+template <int P>
+struct P2LCols {
+    static constexpr int ROLES = p2l_roles(P);
+    int role[P + 1] = {}, off[P + 1] = {}, size[ROLES] = {};
+    constexpr P2LCols()
+    {
+        bool done[P + 1] = {};
+        for (int i = 0; i <= P; ++i) {
+            int b = -1, bs = 0;
+            for (int m = 0; m <= P; ++m) {
+                const int sz = m == 0 ? 2 * (P + 1) : 4 * (P + 1 - m);
+                if (!done[m] && sz > bs) {
+                    b = m;
+                    bs = sz;
+                }
+            }
+            int r = 0;
+            for (int q = 1; q < ROLES; ++q)
+                if (size[q] < size[r]) r = q;
+            role[b] = r;
+            off[b] = size[r];
+            size[r] += bs;
+            done[b] = true;
+        }
+    }
+    constexpr int most() const
+    {
+        int x = 0;
+        for (int q = 0; q < ROLES; ++q) x = size[q] > x ? size[q] : x;
+        return x;
+    }
+};
+
+// The recurrences' constants, c of SWaveSums::add at [m][n] and 2 n - 1 at
+// [n][n].  Read afresh for each source by scalar loads (an offset that the
+// compiler cannot see through): as literals they were carried around the source
+// loop in registers, which cost the block its second wavefront per SIMD.
+struct P2LConst {
+    double c[P2L_PMAX + 1][P2L_PMAX + 1] = {};
+    constexpr P2LConst()
+    {
+        for (int n = 1; n <= P2L_PMAX; ++n) {
+            for (int m = 0; m < n; ++m)
+                c[m][n] = ((n - 1.0) * (n - 1.0) - (double)m * m) /
+                          (4.0 * (n - 1.0) * (n - 1.0) - 1.0);
+            c[n][n] = 2.0 * n - 1.0;
+        }
+    }
+};
+static __constant__ P2LConst c_p2l{};
+
+// column M of one source into its sums u
+template <int P, int M>
+__device__ __forceinline__ void p2l_column(const double *tc, const cplx *g, double z, cplx wm,
+                                           double *u)
+{
+    double a1 = 0.0, a0 = 1.0;
+#pragma unroll
+    for (int n = M; n <= P; ++n) {
+        if (n > M) {
+            const double v = n == M + 1 ? z : z * a0 - tc[M * (P2L_PMAX + 1) + n] * a1;
+            a1 = a0;
+            a0 = v;
+        }
+        if (M == 0) {
+            u[2 * n] += g[n].x * a0;
+            u[2 * n + 1] += g[n].y * a0;
+        } else {
+            const cplx A = n == M ? wm : a0 * wm;
+            u[4 * (n - M)] += g[n].x * A.x;
+            u[4 * (n - M) + 1] += g[n].y * A.y;
+            u[4 * (n - M) + 2] += g[n].y * A.x;
+            u[4 * (n - M) + 3] += g[n].x * A.y;
+        }
+    }
+}
+
+// columns M.. of role R (wm: w^M, 1 at M = 0)
+template <int P, int R, int M>
+__device__ __forceinline__ void p2l_columns(const double *tc, const cplx *g, double z, cplx w,
+                                            cplx wm, double *a)
+{
+    constexpr P2LCols<P> C{};
+    if constexpr (C.role[M] == R) p2l_column<P, M>(tc, g, z, wm, a + C.off[M]);
+    if constexpr (M < P) p2l_columns<P, R, M + 1>(tc, g, z, w, M == 0 ? w : wm * w, a);
+}
+
+// the sums of role R of one source into a
+template <int P, int R>
+__device__ __forceinline__ void p2l_add(double k, double ik, v3 d, cplx q, double *a)
+{
+    int toff = 0;
+    asm volatile("" : "+s"(toff));
+    const double *tc = &c_p2l.c[0][0] + toff;
+    const double r2 = d.x * d.x + d.y * d.y + d.z * d.z;
+    const double ir = qbx_rsqrt(r2);
+    const double ix = ir * ik;
+    double sn, cs;
+    qbx_sincos_core(k * (r2 * ir), &sn, &cs);
+    cplx g[P + 2];
+    const cplx h0 = {sn * ix, -cs * ix};
+    const cplx h1 = {(h0.x - cs) * ix, (h0.y - sn) * ix};
+    g[0] = q * h0;
+    g[1] = q * h1;
+#pragma unroll
+    for (int n = 2; n <= P; ++n) {
+        const double f = tc[n * (P2L_PMAX + 2)] * ix;
+        g[n] = {f * g[n - 1].x - g[n - 2].x, f * g[n - 1].y - g[n - 2].y};
+    }
+    p2l_columns<P, R, 0>(tc, g, d.z * ir, cplx{d.x * ir, d.y * ir}, cplx{1.0, 0.0}, a);
+}
+
+// lane l's sum over the lanes of v[l]
+template <int O = 32>
+__device__ __forceinline__ double reduce_scatter64(double *v, int lane)
+{
+    const bool up = lane & O;
+#pragma unroll
+    for (int i = 0; i < O; ++i) {
+        const double keep = up ? v[i + O] : v[i], give = up ? v[i] : v[i + O];
+        v[i] = keep + __shfl_xor(give, O);
+    }
+    if constexpr (O > 1) return reduce_scatter64<O / 2>(v, lane);
+    return v[0];
+}
+
+template <int P>
+__global__ void __launch_bounds__(p2l_threads(P), P == 10 ? 1 : 2) kh_p2l_reg(HD hd, TD t, const int *boxes,
+                                                  const int *starts, const int *lists,
+                                                  const double *src, int ns,
+                                                  const double *str, double *local)
+{
+    constexpr P2LCols<P> C{};
+    constexpr int CH = p2l_threads(P);
+    constexpr int ROLES = C.ROLES, SH = CH / 64 / ROLES, NA = (C.most() + 63) / 64 * 64;
+    __shared__ double2 sxy[CH], szq[CH];  // x, y; z, Re q
+    __shared__ double sqi[CH];
+    __shared__ int pre[CH + 1], first[CH], wsum[CH / 64];
+    __shared__ double red[CH / 64][NA];  // a row per wavefront: role + ROLES * share
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int role = wave % ROLES, share = wave / ROLES;
+    const int it = blockIdx.x;
+    const int e1 = starts[it + 1];
+    if (starts[it] == e1) return;
+    const int B = boxes[it];
+    const v3 c = boxc(t, B);
+    const double k = hd.k, ik = 1.0 / k;
+    double acc[NA];
+#pragma unroll
+    for (int i = 0; i < NA; ++i) acc[i] = 0.0;
+    for (int e0 = starts[it]; e0 < e1; e0 += CH) {
+        list_counts<CH>(t, e0, e1, lists, first, pre, wsum);
+        const int total = pre[CH];
+        double2 rxy = {0, 0}, rzq = {0, 0};
+        double rqi = 0;
+        auto fetch = [&](int v) {
+            if (v >= total) return;
+            const int si = list_source<CH>(first, pre, v);
+            const double *q = str + 2 * ((size_t)si * hd.nr + hd.r0);
+            rxy = {src[si], src[(size_t)ns + si]};
+            rzq = {src[2 * (size_t)ns + si], q[0]};
+            rqi = q[1];
+        };
+        fetch(tid);
+        for (int v0 = 0; v0 < total; v0 += CH) {
+            sxy[tid] = rxy;
+            szq[tid] = rzq;
+            sqi[tid] = rqi;
+            __syncthreads();
+            fetch(v0 + CH + tid);
+            const int n = min(CH, total - v0);
+            for (int j = share * 64 + lane; j < n; j += 64 * SH) {
+                const double2 xy = sxy[j], zq = szq[j];
+                const v3 d = {xy.x - c.x, xy.y - c.y, zq.x - c.z};
+                const cplx q = {zq.y, sqi[j]};
+                if (role == 0)
+                    p2l_add<P, 0>(k, ik, d, q, acc);
+                else if (role == 1)
+                    p2l_add<P, 1>(k, ik, d, q, acc);
+                else if (role == 2)
+                    p2l_add<P, 2>(k, ik, d, q, acc);
+                else if (role == 3)
+                    p2l_add<P, 3>(k, ik, d, q, acc);
+                else if constexpr (ROLES > 4) {
+                    if (role == 4)
+                        p2l_add<P, 4>(k, ik, d, q, acc);
+                    else if (role == 5)
+                        p2l_add<P, 5>(k, ik, d, q, acc);
+                    else if (role == 6)
+                        p2l_add<P, 6>(k, ik, d, q, acc);
+                    else
+                        p2l_add<P, 7>(k, ik, d, q, acc);
+                }
+            }
+            __syncthreads();
+        }
+    }
+#pragma unroll
+    for (int i = 0; i < NA; i += 64) red[wave][i + lane] = reduce_scatter64(acc + i, lane);
+    __syncthreads();
+    if (tid < (P + 1) * (P + 1)) {
+        int n, m;
+        nm_of(tid, n, m);
+        const int am = abs(m);
+        int w0 = 0, o = 0;
+#pragma unroll
+        for (int i = 0; i <= P; ++i)
+            if (i == am) {
+                w0 = C.role[i];
+                o = C.off[i] + (i == 0 ? 2 : 4) * (n - i);
+            }
+        double u[4] = {0, 0, 0, 0};
+        for (int h = 0; h < SH; ++h)
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+                if (j < 2 || am > 0) u[j] += red[w0 + ROLES * h][o + j];
+        // (c_n^m)^2 = prod (2i+1)/(2i) prod (4l^2-1)/(l^2-m^2) / (4 pi)
+        double num = 1.0, den = FOURPI;
+        for (int i = 1; i <= am; ++i) {
+            num *= 2 * i + 1;
+            den *= 2 * i;
+        }
+        for (int l = am + 1; l <= n; ++l) {
+            num *= 4 * l * l - 1;
+            den *= l * l - am * am;
+        }
+        double cn = sqrt(num / den);
+        if (m > 0 && (m & 1)) cn = -cn;
+        const cplx v = am == 0 ? cplx{u[0], u[1]}
+                       : m > 0 ? cplx{u[0] + u[1], u[2] - u[3]}
+                               : cplx{u[0] - u[1], u[2] + u[3]};
+        const int lv = t.level[B];
+        const cplx ikv = {0.0, k * ipow(hd.s[lv], n) * cn};
+        const cplx r = ikv * v;
+        double *dst = local + ecoef_off(hd, B, lv) + 2 * ((long)tid * hd.nr + hd.r0);
+        dst[0] += r.x;
+        dst[1] += r.y;
     }
 }
 
@@ -2782,9 +3059,40 @@ int h3_form_locals(qbx_ctx *ctx, void *stream, const qbx_tree *T, const qbx_trav
     if (!accumulate) QBX_TRY(zero_fill(local, exp_doubles(hd), st));
     if (R->n4 == 0 || R->nttp_boxes == 0) return QBX_OK;
     const TD td = make_td(T);
-    return launch_p2e<1>(st, hd, td, R->nttp_boxes, R->ttp_boxes.p, R->l4_starts.p,
-                         R->l4_lists.p, nullptr, 0, nullptr, T->sources.p, T->nsources, str, nrm,
-                         hd.pmax, local);
+    // runs of levels of one order: charges with few enough coefficients in
+    // registers (distances to a box center are below the tree's diagonal),
+    // the others through LDS
+    const std::vector<int> &ls = R->h_level_start_ttp_box_nrs;
+    const bool core = !hd.dip && fabs(hd.k) * 1.75 * hd.h[0] <= QBX_SINCOS_MAX;
+    for (int l = 0, l1; l < T->nlevels; l = l1) {
+        const int p = hd.order[l];
+        for (l1 = l + 1; l1 < T->nlevels && hd.order[l1] == p;) ++l1;
+        const int i0 = ls[l], n = ls[l1] - i0;
+        if (n <= 0) continue;
+        if (!core || p > P2L_PMAX) {
+            QBX_TRY(launch_p2e<1>(st, hd, td, n, R->ttp_boxes.p + i0, R->l4_starts.p + i0,
+                                  R->l4_lists.p, nullptr, 0, nullptr, T->sources.p, T->nsources,
+                                  str, nrm, p, local));
+            continue;
+        }
+        for (int r = 0; r < hd.nr; ++r) {
+            hd.r0 = r;
+            hd.rc = 1;
+            switch (p) {
+#define H3_P2L(P)                                                                           \
+    case P:                                                                                 \
+        hipLaunchKernelGGL(kh_p2l_reg<P>, dim3(n), dim3(p2l_threads(P)), 0, st, hd, td,                \
+                           R->ttp_boxes.p + i0, R->l4_starts.p + i0, R->l4_lists.p,         \
+                           T->sources.p, T->nsources, str, local);                          \
+        break;
+                H3_P2L(0) H3_P2L(1) H3_P2L(2) H3_P2L(3) H3_P2L(4) H3_P2L(5) H3_P2L(6)
+                H3_P2L(7) H3_P2L(8) H3_P2L(9) H3_P2L(10) H3_P2L(11) H3_P2L(12)
+#undef H3_P2L
+            }
+        }
+    }
+    QBX_HIP(hipGetLastError());
+    return QBX_OK;
 }
 
 int h3_eval_targets(qbx_ctx *ctx, void *stream, const qbx_tree *T, const qbx_trav *R,
