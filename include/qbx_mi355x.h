@@ -318,7 +318,7 @@ enum {
     QBX_TUNE_M2QBXL_UNIT_ITER = 3,  /* M2QBXL: list-3 boxes per lane (1..64) */
     QBX_TUNE_L2QBXL_LANES = 4,      /* 2D Helmholtz one-density L2QBXL: lanes per
                                        center (1, 2, 4, 8) */
-    QBX_TUNE_DRIVE_STREAMS = 5,     /* qbx_drive_fmm and, in 2D, qbx_drive_fmm_adjoint: 4 =
+    QBX_TUNE_DRIVE_STREAMS = 5,     /* qbx_drive_fmm and qbx_drive_fmm_adjoint: 4 =
                                        their stage DAG on the caller's stream and up to
                                        three side streams (default); 1 = every
                                        stage on the caller's stream, so that many contexts

@@ -868,6 +868,22 @@ constexpr int P2L_PMAX = 12;
 constexpr int p2l_roles(int P) { return P <= 4 ? 1 : P <= 6 ? 2 : P <= 10 ? 4 : 8; }
 constexpr int p2l_threads(int P) { return 64 * (p2l_roles(P) > 4 ? p2l_roles(P) : 4); }
 
+// c_n^m of SWaveSums without its sign, for n <= P2L_PMAX:
+// (c_n^m)^2 = prod (2i+1)/(2i) prod (4l^2-1)/(l^2-m^2) / (4 pi)
+__device__ __forceinline__ double sph_norm(int n, int m)
+{
+    double num = 1.0, den = FOURPI;
+    for (int i = 1; i <= m; ++i) {
+        num *= 2 * i + 1;
+        den *= 2 * i;
+    }
+    for (int l = m + 1; l <= n; ++l) {
+        num *= 4 * l * l - 1;
+        den *= l * l - m * m;
+    }
+    return sqrt(num / den);
+}
+
 template <int P>
 struct P2LCols {
     static constexpr int ROLES = p2l_roles(P);
@@ -1084,17 +1100,7 @@ __global__ void __launch_bounds__(p2l_threads(P), P == 10 ? 1 : 2) kh_p2l_reg(HD
 #pragma unroll
             for (int j = 0; j < 4; ++j)
                 if (j < 2 || am > 0) u[j] += red[w0 + ROLES * h][o + j];
-        // (c_n^m)^2 = prod (2i+1)/(2i) prod (4l^2-1)/(l^2-m^2) / (4 pi)
-        double num = 1.0, den = FOURPI;
-        for (int i = 1; i <= am; ++i) {
-            num *= 2 * i + 1;
-            den *= 2 * i;
-        }
-        for (int l = am + 1; l <= n; ++l) {
-            num *= 4 * l * l - 1;
-            den *= l * l - am * am;
-        }
-        double cn = sqrt(num / den);
+        double cn = sph_norm(n, am);
         if (m > 0 && (m & 1)) cn = -cn;
         const cplx v = am == 0 ? cplx{u[0], u[1]}
                        : m > 0 ? cplx{u[0] + u[1], u[2] - u[3]}
@@ -2223,17 +2229,18 @@ __global__ void __launch_bounds__(448) kh_adj_e2qbxl(HD hd, TD t, int nunits,
                 y[w] = ldc(qadj + 2 * ((size_t)ci * nco + w));
             __syncthreads();
             if (tid < ncin) {
-                const double *gj = hd.gaunt + (long)tid * ncg * (hd.pg + 1);
                 for (int o = 0; o < nco; ++o) {
                     int nu, mu;
                     nm_of(o, nu, mu);
-                    const double *gg = gj + (long)o * (hd.pg + 1);
+                    // G(j, o) = (-1)^(m - mu) G(o, j): consecutive lanes' rows
+                    const double *gg = hd.gaunt + ((long)o * ncg + tid) * (hd.pg + 1);
+                    const int sw = (m - mu) & 1;
                     cplx cf = {0.0, 0.0};
                     const int imax = min(n, nu);
                     for (int ii = 0; ii <= imax; ++ii) {
                         const int l = abs(n - nu) + 2 * ii;
                         if (abs(m - mu) > l) continue;
-                        const int ex = (nu + l - n) / 2;
+                        const int ex = (nu + l - n) / 2 + sw;
                         cf += ((ex & 1) ? -gg[ii] : gg[ii]) * X[IDX(l, m - mu)];
                     }
                     acc += conj(cf) * y[o];
@@ -2328,17 +2335,17 @@ __global__ void __launch_bounds__(448) kh_adj_e2qbxl_z(HD hd, TD t, int nunits,
         if (tid < ncin) {
             int n, m;
             nm_of(tid, n, m);
-            const double *gj = hd.gaunt + (long)tid * ncg * (hd.pg + 1);
             cplx acc = {0.0, 0.0};
             for (int o = 0; o < nco; ++o) {
                 int nu, mu;
                 nm_of(o, nu, mu);
-                const double *gg = gj + (long)o * (hd.pg + 1);
+                // G(j, o) = (-1)^(m - mu) G(o, j): consecutive lanes' rows
+                const double *gg = hd.gaunt + ((long)o * ncg + tid) * (hd.pg + 1);
                 const int imax = min(n, nu);
                 for (int ii = 0; ii <= imax; ++ii) {
                     const int l = abs(n - nu) + 2 * ii;
                     if (abs(m - mu) > l) continue;
-                    const int ex = (nu + l - n) / 2;
+                    const int ex = (nu + l - n) / 2 + ((m - mu) & 1);
                     acc += ((ex & 1) ? -gg[ii] : gg[ii]) * Z[IDX(l, m - mu) * 16 + o];
                 }
             }
@@ -2348,12 +2355,10 @@ __global__ void __launch_bounds__(448) kh_adj_e2qbxl_z(HD hd, TD t, int nunits,
     }
 }
 
-// P2QBXL^T: a 64-lane block per (group of up to GC_GROUP centers of one
-// target box, share blockIdx.y of its list-1 sources), lanes over the
-// sources, each summing over the group's centers; one atomic per source.
-// PQ >= 0: the S waves in registers (s_waves_reg); PQ = -1: any order, the
-// radial sequence in LDS.
-template <int PQ>
+// P2QBXL^T of any order and argument: a 64-lane block per (group of up to
+// GC_GROUP centers of one target box, share blockIdx.y of its list-1 sources),
+// lanes over the sources, each summing over the group's centers, the radial
+// sequence in LDS; one atomic per source.  kh_adj_s2s takes the orders it can.
 __global__ void __launch_bounds__(64) kh_adj_p2qbxl(HD hd, TD t, int nunits, const int *unit_box,
                                                     const int *unit_c0, const int *gcs,
                                                     const int *gcl, const double *ctrs,
@@ -2361,17 +2366,16 @@ __global__ void __launch_bounds__(64) kh_adj_p2qbxl(HD hd, TD t, int nunits, con
                                                     const int *lists, const double *src,
                                                     int ns, const double *qadj, double *sadj)
 {
-    constexpr int NCR = PQ >= 0 ? (PQ + 1) * (PQ + 1) : 1;
     __shared__ double cq[2 * GC_GROUP * (MAXPQ + 1) * (MAXPQ + 1)];
     __shared__ double cc[3 * GC_GROUP];
-    __shared__ double rads[PQ >= 0 ? 1 : 64 * 2 * (MAXPQ + 1)];
-    __shared__ double jts[PQ >= 0 ? 1 : 64 * (MAXPQ + 3)];
+    __shared__ double rads[64 * 2 * (MAXPQ + 1)];
+    __shared__ double jts[64 * (MAXPQ + 3)];
     const int u = blockIdx.x;
     if (u >= nunits) return;
     const int itb = unit_box[u];
     const int g0 = gcs[itb] + unit_c0[u], ng = min(GC_GROUP, gcs[itb + 1] - g0);
     const int lane = threadIdx.x;
-    const int pq = PQ >= 0 ? PQ : hd.pq, nco = hd.ncq;
+    const int pq = hd.pq, nco = hd.ncq;
     cplx *Lq = reinterpret_cast<cplx *>(cq);
     for (int w = lane; w < ng * nco; w += 64) {
         const int ci = gcl[g0 + w / nco];
@@ -2399,33 +2403,146 @@ __global__ void __launch_bounds__(64) kh_adj_p2qbxl(HD hd, TD t, int nunits, con
             cplx acc = {0.0, 0.0};
             for (int q = 0; q < ng; ++q) {
                 const v3 d = sub(sp, v3{cc[3 * q], cc[3 * q + 1], cc[3 * q + 2]});
-                const cplx *L = Lq + q * nco;
-                if constexpr (PQ >= 0) {
-                    cplx F[NCR];
-                    s_waves_reg<PQ>(hd.k, d, F);
-                    // sum conj(h_n) Y_n^m L = sum conj((-1)^m F[n, -m]) L
-#pragma unroll
-                    for (int nn = 0; nn <= PQ; ++nn)
-#pragma unroll
-                        for (int mm = -nn; mm <= nn; ++mm) {
-                            cplx f = conj(F[IDX(nn, -mm)]);
-                            if (mm & 1) f = -f;
-                            acc += f * L[IDX(nn, mm)];
-                        }
-                } else {
-                    cplx *rad = reinterpret_cast<cplx *>(rads) + lane * (MAXPQ + 1);
-                    double *jt = jts + lane * (MAXPQ + 3);
-                    const double rr = sqrt(d.x * d.x + d.y * d.y + d.z * d.z);
-                    radial_seq(1, pq, hd.k * rr, rad, jt);
-                    for (int nn = 0; nn <= pq; ++nn) rad[nn] = conj(rad[nn]);
-                    cplx a1[1] = {{0.0, 0.0}};
-                    sum_waves<1>(hd, reinterpret_cast<const double *>(L), pq, d, rad, a1);
-                    acc += a1[0];
-                }
+                cplx *rad = reinterpret_cast<cplx *>(rads) + lane * (MAXPQ + 1);
+                double *jt = jts + lane * (MAXPQ + 3);
+                const double rr = sqrt(d.x * d.x + d.y * d.y + d.z * d.z);
+                radial_seq(1, pq, hd.k * rr, rad, jt);
+                for (int nn = 0; nn <= pq; ++nn) rad[nn] = conj(rad[nn]);
+                cplx a1[1] = {{0.0, 0.0}};
+                sum_waves<1>(hd, reinterpret_cast<const double *>(Lq + q * nco), pq, d, rad, a1);
+                acc += a1[0];
             }
             atomic_addc(sadj + 2 * (size_t)si, cplx{0.0, -hd.k} * acc);
         }
         base += cnt;
+    }
+}
+
+// sum_{n <= P, m} conj(h_n(k r)) Y_n^m(d) L_n^m from the coefficients of the
+// real and imaginary parts of (x + i y)^m Q_n^m(z) (SWaveSums), m >= 0: cf[(n, m)]
+// = (U, V), U = c ((-1)^m L_n^m + L_n^-m), V = i c ((-1)^m L_n^m - L_n^-m).
+template <int P>
+__device__ __forceinline__ cplx s_waves_dot(double k, double ik, v3 d, const double *cf)
+{
+    int toff = 0;
+    asm volatile("" : "+s"(toff));  // see P2LConst; neither are cf's values carried along
+    const double *tc = &c_p2l.c[0][0] + toff;
+    const double2 *uv = reinterpret_cast<const double2 *>(cf) + toff;
+    const double r2 = d.x * d.x + d.y * d.y + d.z * d.z;
+    const double ir = qbx_rsqrt(r2);
+    const double z = d.z * ir;
+    const cplx w = {d.x * ir, d.y * ir};
+    cplx S[P + 1];
+    cplx wm = w;
+#pragma unroll
+    for (int m = 0; m <= P; ++m) {
+        if (m > 1) wm = wm * w;
+        double a1 = 0.0, a0 = 1.0;
+#pragma unroll
+        for (int n = m; n <= P; ++n) {
+            const double2 U = uv[2 * (n * (n + 1) / 2 + m)];
+            if (n > m) {
+                const double a = n == m + 1 ? z : z * a0 - tc[m * (P2L_PMAX + 1) + n] * a1;
+                a1 = a0;
+                a0 = a;
+            }
+            if (m == 0) {
+                S[n] = {a0 * U.x, a0 * U.y};
+            } else {
+                const double2 V = uv[2 * (n * (n + 1) / 2 + m) + 1];
+                const cplx A = n == m ? wm : a0 * wm;
+                S[n].x += A.x * U.x + A.y * V.x;
+                S[n].y += A.x * U.y + A.y * V.y;
+            }
+        }
+    }
+    const double ix = ir * ik;
+    double sn, cs;
+    qbx_sincos_core(k * (r2 * ir), &sn, &cs);
+    cplx h0 = {sn * ix, cs * ix};  // conj(h_n)
+    cplx acc = h0 * S[0];
+    if (P > 0) {
+        cplx h1 = {(h0.x - cs) * ix, (h0.y + sn) * ix};
+        acc += h1 * S[1];
+#pragma unroll
+        for (int n = 2; n <= P; ++n) {
+            const double f = tc[n * (P2L_PMAX + 2)] * ix;
+            const cplx h2 = {f * h1.x - h0.x, f * h1.y - h0.y};
+            acc += h2 * S[n];
+            h0 = h1;
+            h1 = h2;
+        }
+    }
+    return acc;
+}
+
+// P2QBXL^T (BOX false: groups of up to GC_GROUP centers of one target box, its
+// list-1 sources) and P2L^T (BOX: a box, its list-4 sources) in registers,
+// orders <= P2L_PMAX, arguments within the sine's reduced range: a lane per
+// source, the list's sources dealt to the lanes without regard to box borders
+// as in kh_p2qbxl_reg and in turn to the blockIdx.y shares, the coefficients in
+// LDS.  One atomic per (group, source).
+//
+// FP64 VALU bound with the LDS broadcasts of the coefficients close behind.
+// 2.4e8 (center, source) pairs at order 3: 4.5 ms with lanes walking box by box
+// and sixteen complex products of the waves, now 1.9; 3.1e6 (box, source)
+// pairs at order 10: 1.7 ms with the radial sequences in LDS, now 0.17.
+template <int P, bool BOX>
+__global__ void __launch_bounds__(256) kh_adj_s2s(HD hd, TD t, const int *items,
+                                                  const int *unit_c0, const int *gcs,
+                                                  const int *gcl, const double *ctrs, int nctr,
+                                                  const int *starts, const int *lists,
+                                                  const double *src, int ns,
+                                                  const double *coef, double *sadj)
+{
+    constexpr int CH = 256, NC = (P + 1) * (P + 2) / 2, G = BOX ? 1 : GC_GROUP;
+    __shared__ __align__(16) double cf[G * NC * 4];
+    __shared__ double cc[3 * G];
+    __shared__ int pre[CH + 1], first[CH], wsum[CH / 64];
+    const int tid = threadIdx.x, u = blockIdx.x;
+    const int it = BOX ? u : items[u];
+    const int e1 = starts[it + 1];
+    if (starts[it] == e1) return;
+    const int B = BOX ? items[u] : 0, lv = BOX ? t.level[B] : 0;
+    const int g0 = BOX ? 0 : gcs[it] + unit_c0[u];
+    const int ng = BOX ? 1 : min(GC_GROUP, gcs[it + 1] - g0);
+    for (int w = tid; w < ng * NC; w += CH) {
+        const int q = w / NC, i = w % NC;
+        int n = 0;
+        while ((n + 1) * (n + 2) / 2 <= i) ++n;
+        const int m = i - n * (n + 1) / 2;
+        const double *L = BOX ? coef + ecoef_off(hd, B, lv)
+                              : coef + 2 * (size_t)gcl[g0 + q] * hd.ncq;
+        const double c = sph_norm(n, m) * (BOX ? ipow(hd.s[lv], n) : 1.0);
+        cplx lp = c * ldc(L + 2 * IDX(n, m)), lm = {0.0, 0.0};
+        if (m > 0) {
+            if (m & 1) lp = -lp;
+            lm = c * ldc(L + 2 * IDX(n, -m));
+        }
+        cf[4 * w] = lp.x + lm.x;
+        cf[4 * w + 1] = lp.y + lm.y;
+        cf[4 * w + 2] = lm.y - lp.y;
+        cf[4 * w + 3] = lp.x - lm.x;
+    }
+    if (tid < 3 * ng) {
+        const int dd = tid % 3;
+        cc[tid] = BOX ? t.centers[(size_t)dd * t.nboxes + B]
+                      : ctrs[(size_t)dd * nctr + gcl[g0 + tid / 3]];
+    }
+    const double k = hd.k, ik = 1.0 / k;
+    for (int e0 = starts[it]; e0 < e1; e0 += CH) {
+        list_counts<CH>(t, e0, e1, lists, first, pre, wsum);
+        const int total = pre[CH];
+        for (int v = blockIdx.y * CH + tid; v < total; v += CH * gridDim.y) {
+            const int si = list_source<CH>(first, pre, v);
+            const v3 sp = ld3(src, ns, si);
+            cplx acc = {0.0, 0.0};
+            for (int q = 0; q < ng; ++q)
+                acc += s_waves_dot<P>(k, ik, sub(sp, v3{cc[3 * q], cc[3 * q + 1], cc[3 * q + 2]}),
+                                      cf + 4 * q * NC);
+            atomic_addc(sadj + 2 * (size_t)si, cplx{0.0, -k} * acc);
+        }
+        __syncthreads();  // the tile's counts consumed
     }
 }
 
@@ -3313,6 +3430,8 @@ static int adjoint_launch(hipStream_t st, const qbx_tree *T, const qbx_trav *R,
     const int ntb = R->ntarget_boxes, nc = G->ncenters;
     // groups of up to GC_GROUP global centers of one target box
     const unit_plan &U = G->gc_group_plan;
+    // arguments of the S waves within the sine's reduced range (as in P2QBXL)
+    const bool core = fabs(hd.k) * 1.75 * hd.h[0] <= QBX_SINCOS_MAX;
     int ncl_max = 1;
     for (int l = 0; l < hd.nlevels; ++l) ncl_max = std::max(ncl_max, hd.ncl[l]);
     switch (stage) {
@@ -3349,18 +3468,22 @@ static int adjoint_launch(hipStream_t st, const qbx_tree *T, const qbx_trav *R,
     case QBX_ADJ_P2QBXL:
         if (U.nunits > 0) {
 #define H3_AP2Q(PQV)                                                                       \
-    hipLaunchKernelGGL(kh_adj_p2qbxl<PQV>, dim3(U.nunits, ADJ_SHARES), dim3(64), 0, st, hd, \
-                       td, U.nunits, U.unit_box.p, U.unit_t0.p, G->gc_by_tbox_starts.p,    \
-                       G->gc_by_tbox.p, G->centers.p, nc, R->l1_starts.p, R->l1_lists.p,   \
-                       T->sources.p, T->nsources, in, out)
-            switch (hd.pq) {
-            case 0: H3_AP2Q(0); break;
-            case 1: H3_AP2Q(1); break;
-            case 2: H3_AP2Q(2); break;
-            case 3: H3_AP2Q(3); break;
-            case 4: H3_AP2Q(4); break;
-            case 5: H3_AP2Q(5); break;
-            default: H3_AP2Q(-1); break;
+    case PQV:                                                                              \
+        hipLaunchKernelGGL((kh_adj_s2s<PQV, false>), dim3(U.nunits, ADJ_SHARES), dim3(256), \
+                           0, st, hd, td, U.unit_box.p, U.unit_t0.p,                       \
+                           G->gc_by_tbox_starts.p, G->gc_by_tbox.p, G->centers.p, nc,      \
+                           R->l1_starts.p, R->l1_lists.p, T->sources.p, T->nsources, in,   \
+                           out);                                                           \
+        break;
+            switch (core ? hd.pq : -1) {
+                H3_AP2Q(0) H3_AP2Q(1) H3_AP2Q(2) H3_AP2Q(3) H3_AP2Q(4) H3_AP2Q(5)
+            default:
+                hipLaunchKernelGGL(kh_adj_p2qbxl, dim3(U.nunits, ADJ_SHARES), dim3(64), 0, st,
+                                   hd, td, U.nunits, U.unit_box.p, U.unit_t0.p,
+                                   G->gc_by_tbox_starts.p, G->gc_by_tbox.p, G->centers.p, nc,
+                                   R->l1_starts.p, R->l1_lists.p, T->sources.p, T->nsources, in,
+                                   out);
+                break;
             }
 #undef H3_AP2Q
         }
@@ -3413,10 +3536,31 @@ static int adjoint_launch(hipStream_t st, const qbx_tree *T, const qbx_trav *R,
         }
         break;
     case QBX_ADJ_P2L:
-        if (R->nttp_boxes > 0 && R->n4 > 0)
-            hipLaunchKernelGGL(kh_adj_p2e<true>, dim3(R->nttp_boxes), dim3(64), 0, st, hd, td,
-                               R->nttp_boxes, R->ttp_boxes.p, R->l4_starts.p, R->l4_lists.p,
-                               T->sources.p, T->nsources, in, out);
+        // runs of levels of one order, as in the forward's P2L
+        for (int l = 0, l1; R->n4 > 0 && l < T->nlevels; l = l1) {
+            const int p = hd.order[l];
+            for (l1 = l + 1; l1 < T->nlevels && hd.order[l1] == p;) ++l1;
+            const int i0 = R->h_level_start_ttp_box_nrs[l];
+            const int n = R->h_level_start_ttp_box_nrs[l1] - i0;
+            if (n <= 0) continue;
+            switch (core ? p : -1) {
+#define H3_AP2L(P)                                                                          \
+    case P:                                                                                 \
+        hipLaunchKernelGGL((kh_adj_s2s<P, true>), dim3(n, 2), dim3(256), 0, st, hd, td,     \
+                           R->ttp_boxes.p + i0, nullptr, nullptr, nullptr, nullptr, 0,      \
+                           R->l4_starts.p + i0, R->l4_lists.p, T->sources.p, T->nsources,   \
+                           in, out);                                                        \
+        break;
+                H3_AP2L(0) H3_AP2L(1) H3_AP2L(2) H3_AP2L(3) H3_AP2L(4) H3_AP2L(5) H3_AP2L(6)
+                H3_AP2L(7) H3_AP2L(8) H3_AP2L(9) H3_AP2L(10) H3_AP2L(11) H3_AP2L(12)
+#undef H3_AP2L
+            default:
+                hipLaunchKernelGGL(kh_adj_p2e<true>, dim3(n), dim3(64), 0, st, hd, td, n,
+                                   R->ttp_boxes.p + i0, R->l4_starts.p + i0, R->l4_lists.p,
+                                   T->sources.p, T->nsources, in, out);
+                break;
+            }
+        }
         break;
     case QBX_ADJ_M2M:
         // out ignored: in (the multipoles' adjoint) is updated in place,
@@ -3477,24 +3621,12 @@ int h3_drive_fmm_adjoint(qbx_ctx *ctx, hipStream_t st, const qbx_tree *T, const 
         hipLaunchKernelGGL(kh_adj_scatter, dim3(cdiv(nt - nc, 256)), dim3(256), 0, st, nt, nc,
                            G->user_to_tree_target.p, pot_adj_user, Pa);
     QBX_HIP(hipGetLastError());
-    auto run = [&](int stage, const double *in, double *out) {
-        return adjoint_launch(st, T, R, G, hd, stage, in, out);
-    };
-    // the forward's stages in reverse: the potentials' adjoint into the QBX
-    // and box locals, those down the tree, then into the multipoles and up
-    QBX_TRY(run(QBX_ADJ_QBXL2P, Pa, Qa));
-    QBX_TRY(run(QBX_ADJ_L2QBXL, Qa, La));
-    QBX_TRY(run(QBX_ADJ_L2P, Pa, La));
-    QBX_TRY(run(QBX_ADJ_L2L, La, nullptr));
-    QBX_TRY(run(QBX_ADJ_M2L, La, Ma));
-    QBX_TRY(run(QBX_ADJ_M2QBXL, Qa, Ma));
-    QBX_TRY(run(QBX_ADJ_M2P, Pa, Ma));
-    QBX_TRY(run(QBX_ADJ_P2L, La, str_adj));
-    QBX_TRY(run(QBX_ADJ_P2QBXL, Qa, str_adj));
-    QBX_TRY(run(QBX_ADJ_P2P, Pa, str_adj));
-    QBX_TRY(run(QBX_ADJ_M2M, Ma, nullptr));
-    QBX_TRY(run(QBX_ADJ_P2M, Ma, str_adj));
-    return QBX_OK;
+    return adjoint_dag(
+        ctx, st,
+        [&](hipStream_t s, int stage, const double *in, double *out) {
+            return adjoint_launch(s, T, R, G, hd, stage, in, out);
+        },
+        Pa, Qa, La, Ma, str_adj);
 }
 
 }  // namespace qbx
