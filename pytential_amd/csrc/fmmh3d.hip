@@ -1568,9 +1568,13 @@ __global__ void __launch_bounds__(64) kh_e2qbxl(HD hd, TD t, int ng, const int *
     }
 }
 
-// shares (blockIdx.y) of the list-1 sources / list-3 boxes per center group
-// in M2QBXL, P2QBXL^T and M2QBXL^T
+// shares (blockIdx.y) of a center group's list-1 sources in P2QBXL^T
 constexpr int ADJ_SHARES = 4;
+// ... and of its list-3 boxes in M2QBXL and M2QBXL^T: the groups of coarse boxes
+// have the long lists and finish last.  163972 centers, M2QBXL: 5.9, 4.5, 4.2,
+// 4.0, 4.2 ms with 1, 2, 4, 8, 16; 41024 centers: 2.1, 1.2, 0.84, 0.69, 0.67,
+// M2QBXL^T 5.3, 3.1, 2.8, 2.4, 2.5.
+constexpr int L3_SHARES = 8;
 
 __device__ __forceinline__ void atomic_addc(double *p, cplx v)
 {
@@ -1578,7 +1582,89 @@ __device__ __forceinline__ void atomic_addc(double *p, cplx v)
     atomicAdd(p + 1, v.y);
 }
 
-// ---- M2QBXL for one density, p_q <= 3, as a product on the matrix cores -----
+// Constants of the columns Y_n^m = c_n^m Q_n^m(z) (x + i y)^m for n <= YT_LMAX (box
+// order + QBX order 3): norm the c_n^m with their sign, rec the factor of Q_{n-2}^m
+// in the recurrence of Q_n^m (leading coefficient 1, see SWaveSums).
+constexpr int YT_LMAX = MAXP + 3;
+struct YTable {
+    double norm[YT_LMAX + 1][YT_LMAX + 1] = {}, rec[YT_LMAX + 1][YT_LMAX + 1] = {};
+    static constexpr double root(double a)  // Newton from above
+    {
+        double x = a > 1.0 ? a : 1.0;
+        for (int i = 0; i < 60; ++i) {
+            const double y = 0.5 * (x + a / x);
+            if (!(y < x)) break;
+            x = y;
+        }
+        return x;
+    }
+    constexpr YTable()
+    {
+        double mm = 1.0 / 12.566370614359172954;  // (c_m^m)^2
+        for (int m = 0; m <= YT_LMAX; ++m) {
+            if (m > 0) mm *= (2.0 * m + 1.0) / (2.0 * m);
+            double c = mm;
+            for (int n = m; n <= YT_LMAX; ++n) {
+                if (n > m) {
+                    c *= (4.0 * n * n - 1.0) / ((double)n * n - (double)m * m);
+                    rec[m][n] = ((n - 1.0) * (n - 1.0) - (double)m * m) /
+                                (4.0 * (n - 1.0) * (n - 1.0) - 1.0);
+                }
+                norm[m][n] = (m & 1) ? -root(c) : root(c);
+            }
+        }
+    }
+};
+static __constant__ YTable c_yt{};
+
+// S waves X_n^m(d) = h_n(k r) Y_n^m(d), n <= L, of nct centers (cxs, three
+// coordinates each) about cd into X[stride q * center + stride i * IDX(n, m)]: a
+// thread per (center, m), which runs the radial recurrence along with its column.
+// With the radial sequence a phase of its own, one lane a center, and a reciprocal
+// square root per step of every column, forming the waves was most of M2QBXL.
+template <bool CORE>
+__device__ __forceinline__ void s_waves_centers(int nct, const double *cxs, v3 cd, double k,
+                                                int L, cplx *X, int sq, int si)
+{
+    for (int w = threadIdx.x; w < nct * (L + 1); w += blockDim.x) {
+        const int q = w / (L + 1), m = w % (L + 1);
+        const v3 d = sub(v3{cxs[3 * q], cxs[3 * q + 1], cxs[3 * q + 2]}, cd);
+        const double r2 = d.x * d.x + d.y * d.y + d.z * d.z;
+        const double ir = qbx_rsqrt(r2);
+        const double x = k * (r2 * ir), ix = qbx_rcp(x), z = d.z * ir;
+        double sn, cs;
+        if (CORE)
+            qbx_sincos_core(x, &sn, &cs);
+        else
+            qbx_sincos(x, &sn, &cs);
+        cplx h = {sn * ix, -cs * ix};                                  // h_n
+        cplx hn = {(sn * ix - cs) * ix, (-cs * ix - sn) * ix};          // h_{n+1}
+        const cplx w1 = {d.x * ir, d.y * ir};
+        cplx wm = {1.0, 0.0};
+        for (int n = 0; n < m; ++n) {
+            wm = wm * w1;
+            const cplx t = ((2.0 * n + 3.0) * ix) * hn - h;
+            h = hn;
+            hn = t;
+        }
+        const double *nm = c_yt.norm[m], *rc = c_yt.rec[m];
+        cplx *Xq = X + sq * q;
+        double a1 = 0.0, a0 = 1.0;
+        for (int n = m; n <= L; ++n) {
+            const cplx y = (nm[n] * a0) * wm;
+            Xq[si * IDX(n, m)] = h * y;
+            if (m > 0) Xq[si * IDX(n, -m)] = h * sgn_conj(y, m);
+            const double a = n < L ? z * a0 - rc[n + 1] * a1 : 0.0;
+            a1 = a0;
+            a0 = a;
+            const cplx t = ((2.0 * n + 3.0) * ix) * hn - h;
+            h = hn;
+            hn = t;
+        }
+    }
+}
+
+// ---- M2QBXL for one density, p_q <= 3, as a matrix product ------------------
 // The M2QBXL sum of kh_e2qbxl regrouped by the waves' index q = (l, m'):
 //   Q_c[o] = sum_D sum_q X_q(c - c_D) Bm_D[q][o],
 //   Bm_D[q = (l, m')][o = (nu, mu)] = 4 pi sum_{j = (n, m' + mu)}
@@ -1586,7 +1672,7 @@ __device__ __forceinline__ void atomic_addc(double *p, cplx v)
 // (the terms with l = |n - nu| + 2 ii, ii <= min(n, nu)).  Bm depends on the
 // box alone (kh_m2qb_mat, once per box and evaluation); the sum over q is,
 // per group of centers and list-3 box, a product of the centers' waves
-// X[centers][q] with Bm_D[q][16] on v_mfma_f64_16x16x4f64.
+// X[centers][q] with Bm_D[q][16].
 __global__ void __launch_bounds__(256) kh_m2qb_mat(HD hd, TD t, int nqmax, const double *mpole,
                                                    double *bm)
 {
@@ -1638,102 +1724,87 @@ __global__ void __launch_bounds__(256) kh_m2qb_mat(HD hd, TD t, int nqmax, const
     }
 }
 
-// a block (four waves) per (group of up to GC_GROUP global centers of one
-// target box, share blockIdx.y of its list-3 boxes); per list-3 box D the
-// radial sequences (a lane per center) and the Y columns (a lane per
-// (center, m)) give the group's waves X[centers][nq] in LDS (rows past the
-// group unused), the waves split the K = nq steps of the 16 x 16 product with
-// Bm_D read from HBM, their partial tiles are added in LDS in wave order and
-// the shares' sums added into the QBX expansions with atomics
-__global__ void __launch_bounds__(256) kh_m2qbxl_mm(HD hd, TD t, int nunits, const int *ubox,
+// a block per (group of up to GC_GROUP global centers of one target box, share
+// blockIdx.y of its list-3 boxes); per list-3 box D the group's waves
+// X[nq][GC_GROUP] in LDS (s_waves_centers), then a thread per (two of the 16
+// coefficients, 32nd of the q's) keeps the sums of all centers over the boxes:
+// 32 products for one 32-byte read of Bm_D and four of X.  The slices are added
+// by shuffles and in LDS, the shares' sums into the QBX expansions with atomics.
+// On v_mfma_f64_16x16x4f64 the four centers left 12 of 16 rows empty and each
+// step took four instructions of 64 cycles: more than the vector products.
+// 163972 centers, 24597 list-3 entries of their boxes, p = 10, p_q = 3: 5.65 ms,
+// now 4.0.
+template <bool CORE>
+__global__ void __launch_bounds__(256) kh_m2qbxl_bm(HD hd, TD t, int nunits, const int *ubox,
                                                     const int *uc0, const int *gcs,
                                                     const int *gcl, const int *l3s,
                                                     const int *l3l, const double *ctrs, int nctr,
                                                     int nqmax, const double *bm, double *qexp)
 {
+    static_assert(GC_GROUP == 4, "a thread's sums are of four centers");
     extern __shared__ double sh[];
+    cplx *X = reinterpret_cast<cplx *>(sh);  // [nqmax][GC_GROUP]
+    __shared__ double red[4][8][8 * 2];
+    __shared__ double cxs[GC_GROUP * 3];
     const int u = blockIdx.x;
     if (u >= nunits) return;
     const int itb = ubox[u];
     const int c0 = gcs[itb] + uc0[u], nct = min(GC_GROUP, gcs[itb + 1] - c0);
     const int e0 = l3s[itb], e1 = l3s[itb + 1];
     if (nct <= 0 || e0 + (int)blockIdx.y >= e1) return;
-    const int Lm = hd.pmax + hd.pq;
     const int nco = hd.ncq;
-    h3_d4 *red = reinterpret_cast<h3_d4 *>(sh);                    // [3][2][64]
-    cplx *X = reinterpret_cast<cplx *>(red + 3 * 2 * 64);           // [GC_GROUP][nqmax]
-    cplx *rad = X + GC_GROUP * nqmax;                               // [GC_GROUP][Lm + 3]
-    double *jt = reinterpret_cast<double *>(rad + GC_GROUP * (Lm + 3));  // [GC_GROUP][Lm + 4]
-    __shared__ double cxs[GC_GROUP * 3];
-    const int tid = threadIdx.x, wv = tid >> 6, lane = tid & 63, col = lane & 15,
-              kr = lane >> 4;
+    const int tid = threadIdx.x, wv = tid >> 6, lane = tid & 63, op = tid & 7, ks = tid >> 3;
     if (tid < GC_GROUP * 3) {
         const int q = tid / 3, dd = tid % 3;
         cxs[tid] = q < nct ? ctrs[(size_t)dd * nctr + gcl[c0 + q]] : 0.0;
     }
-    h3_d4 cre = {0, 0, 0, 0}, cim = {0, 0, 0, 0};
+    cplx acc[GC_GROUP][2];
+#pragma unroll
+    for (int c = 0; c < GC_GROUP; ++c) acc[c][0] = acc[c][1] = {0.0, 0.0};
     for (int e = e0 + blockIdx.y; e < e1; e += gridDim.y) {
         const int D = l3l[e];
         const int lv = t.level[D];
         const int L = hd.order[lv] + hd.pq, nq = (L + 1) * (L + 1);
-        const v3 cd = boxc(t, D);
         __syncthreads();  // the previous entry's X consumed, cxs written
-        if (tid < nct) {
-            const v3 dv = sub(v3{cxs[3 * tid], cxs[3 * tid + 1], cxs[3 * tid + 2]}, cd);
-            const double rr = sqrt(dv.x * dv.x + dv.y * dv.y + dv.z * dv.z);
-            radial_seq(1, L, hd.k * rr, rad + tid * (Lm + 3), jt + tid * (Lm + 4));
-        }
+        // (columns of a short group's missing centers hold old values, which
+        // only enter sums that are not stored)
+        s_waves_centers<CORE>(nct, cxs, boxc(t, D), hd.k, L, X, 1, GC_GROUP);
         __syncthreads();
-        for (int w = tid; w < nct * (L + 1); w += blockDim.x) {
-            const int q = w / (L + 1), m = w % (L + 1);
-            const v3 dv = sub(v3{cxs[3 * q], cxs[3 * q + 1], cxs[3 * q + 2]}, cd);
-            const cplx *rd = rad + q * (Lm + 3);
-            cplx *Xq = X + (long)q * nqmax;
-            ylm_column(m, L, dv, [&](int n, cplx y) {
-                Xq[IDX(n, m)] = rd[n] * y;
-                if (m > 0) Xq[IDX(n, -m)] = rd[n] * sgn_conj(y, m);
-            });
-        }
-        __syncthreads();
-        const double *B = bm + 2L * (long)D * nqmax * 16;
-        const int KS = (nq + 3) / 4;
-        for (int ks = wv; ks < KS; ks += 4) {
-            const int k = ks * 4 + kr;
-            double are = 0.0, aim = 0.0, bre = 0.0, bim = 0.0;
-            if (k < nq) {
-                if (col < nct) {
-                    const cplx a = X[(long)col * nqmax + k];
-                    are = a.x;
-                    aim = a.y;
-                }
-                const cplx b = ldc(B + 2L * (k * 16 + col));
-                bre = b.x;
-                bim = b.y;
-            }
-            cre = __builtin_amdgcn_mfma_f64_16x16x4f64(are, bre, cre, 0, 0, 0);
-            cre = __builtin_amdgcn_mfma_f64_16x16x4f64(-aim, bim, cre, 0, 0, 0);
-            cim = __builtin_amdgcn_mfma_f64_16x16x4f64(are, bim, cim, 0, 0, 0);
-            cim = __builtin_amdgcn_mfma_f64_16x16x4f64(aim, bre, cim, 0, 0, 0);
-        }
-    }
-    // the four waves' partial tiles: D register j of lane i is the entry
-    // (center 4j + i/16, coefficient i%16)
-    if (wv > 0) {
-        red[((wv - 1) * 2 + 0) * 64 + lane] = cre;
-        red[((wv - 1) * 2 + 1) * 64 + lane] = cim;
-    }
-    __syncthreads();
-    if (wv == 0) {
-        for (int h = 0; h < 3; ++h) {
-            cre += red[(h * 2 + 0) * 64 + lane];
-            cim += red[(h * 2 + 1) * 64 + lane];
-        }
+        const double *B = bm + 2L * ((long)D * nqmax * 16 + 2 * op);
+#pragma unroll 2
+        for (int k = ks; k < nq; k += 32) {
+            const cplx b0 = ldc(B + 32L * k), b1 = ldc(B + 32L * k + 2);
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            const int q = 4 * j + kr;
-            if (q < nct && col < nco)
-                atomic_addc(qexp + 2 * ((size_t)gcl[c0 + q] * nco + col), cplx{cre[j], cim[j]});
+            for (int c = 0; c < GC_GROUP; ++c) {
+                const cplx x = X[GC_GROUP * k + c];
+                acc[c][0] += x * b0;
+                acc[c][1] += x * b1;
+            }
         }
+    }
+#pragma unroll
+    for (int c = 0; c < GC_GROUP; ++c)
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+#pragma unroll
+            for (int o = 8; o < 64; o <<= 1) {
+                acc[c][j].x += __shfl_xor(acc[c][j].x, o);
+                acc[c][j].y += __shfl_xor(acc[c][j].y, o);
+            }
+    if (lane < 8)
+#pragma unroll
+        for (int c = 0; c < GC_GROUP; ++c)
+#pragma unroll
+            for (int j = 0; j < 2; ++j) {
+                red[wv][op][4 * c + 2 * j] = acc[c][j].x;
+                red[wv][op][4 * c + 2 * j + 1] = acc[c][j].y;
+            }
+    __syncthreads();
+    if (tid < 16 * GC_GROUP) {
+        const int c = tid >> 4, o = tid & 15, i = 4 * c + 2 * (o & 1);
+        cplx v = {0.0, 0.0};
+        for (int h = 0; h < 4; ++h) v += cplx{red[h][o >> 1][i], red[h][o >> 1][i + 1]};
+        if (c < nct && o < nco) atomic_addc(qexp + 2 * ((size_t)gcl[c0 + c] * nco + o), v);
     }
 }
 
@@ -2256,13 +2327,13 @@ __global__ void __launch_bounds__(448) kh_adj_e2qbxl(HD hd, TD t, int nunits,
 
 // L2QBXL^T / M2QBXL^T with the group's centers summed before the Gaunt
 // contraction (p_q <= 3): per list-3 box D (or the own box) the waves of all
-// the group's centers in LDS (a lane per center for the radial sequences, a
-// lane per (center, m) for the Y columns), Z[q][o] = sum_c conj(X_c[q])
+// the group's centers in LDS (s_waves_centers; for the R waves a lane per center
+// for the radial sequences, a lane per (center, m) for the Y columns), Z[q][o] = sum_c conj(X_c[q])
 // Lq'_c[o] in LDS, then a thread per box coefficient j: sum_o sum_ii
 // (-1)^ex G(j, o, ii) Z[(l, m - mu)][o] -- one contraction per group and box
 // instead of one per center.  Dynamic LDS: X [GC_GROUP][nqmax], Z [nqmax][16],
 // the radial sequences.
-template <int MODE>
+template <int MODE, bool CORE>
 __global__ void __launch_bounds__(448) kh_adj_e2qbxl_z(HD hd, TD t, int nunits,
                                                        const int *unit_box, const int *unit_c0,
                                                        const int *tboxes, const int *starts,
@@ -2307,14 +2378,17 @@ __global__ void __launch_bounds__(448) kh_adj_e2qbxl_z(HD hd, TD t, int nunits,
         const int ncin = (p + 1) * (p + 1);
         const v3 cd = boxc(t, D);
         __syncthreads();  // the previous box's Z consumed; cxs, ys written
-        if (tid < nct) {
-            const v3 dv = sub(v3{cxs[3 * tid], cxs[3 * tid + 1], cxs[3 * tid + 2]}, cd);
-            const double rr = sqrt(dv.x * dv.x + dv.y * dv.y + dv.z * dv.z);
-            radial_seq(MODE == 0 ? 1 : 0, L, hd.k * rr, rad + tid * (Lm + 3),
-                       jt + tid * (Lm + 4));
+        if (MODE == 0) {
+            s_waves_centers<CORE>(nct, cxs, cd, hd.k, L, X, nqmax, 1);
+        } else {
+            if (tid < nct) {
+                const v3 dv = sub(v3{cxs[3 * tid], cxs[3 * tid + 1], cxs[3 * tid + 2]}, cd);
+                const double rr = sqrt(dv.x * dv.x + dv.y * dv.y + dv.z * dv.z);
+                radial_seq(0, L, hd.k * rr, rad + tid * (Lm + 3), jt + tid * (Lm + 4));
+            }
+            __syncthreads();
         }
-        __syncthreads();
-        for (int w = tid; w < nct * (L + 1); w += blockDim.x) {
+        for (int w = tid; MODE == 1 && w < nct * (L + 1); w += blockDim.x) {
             const int q = w / (L + 1), m = w % (L + 1);
             const v3 dv = sub(v3{cxs[3 * q], cxs[3 * q + 1], cxs[3 * q + 2]}, cd);
             const cplx *rd = rad + q * (Lm + 3);
@@ -2336,17 +2410,17 @@ __global__ void __launch_bounds__(448) kh_adj_e2qbxl_z(HD hd, TD t, int nunits,
             int n, m;
             nm_of(tid, n, m);
             cplx acc = {0.0, 0.0};
-            for (int o = 0; o < nco; ++o) {
-                int nu, mu;
-                nm_of(o, nu, mu);
-                // G(j, o) = (-1)^(m - mu) G(o, j): consecutive lanes' rows
-                const double *gg = hd.gaunt + ((long)o * ncg + tid) * (hd.pg + 1);
-                const int imax = min(n, nu);
-                for (int ii = 0; ii <= imax; ++ii) {
-                    const int l = abs(n - nu) + 2 * ii;
-                    if (abs(m - mu) > l) continue;
-                    const int ex = (nu + l - n) / 2 + ((m - mu) & 1);
-                    acc += ((ex & 1) ? -gg[ii] : gg[ii]) * Z[IDX(l, m - mu) * 16 + o];
+            for (int nu = 0, o = 0; nu <= pq; ++nu) {
+                const int imax = min(n, nu), l0 = abs(n - nu);
+                for (int mu = -nu; mu <= nu; ++mu, ++o) {
+                    // G(j, o) = (-1)^(m - mu) G(o, j): consecutive lanes' rows
+                    const double *gg = hd.gaunt + ((long)o * ncg + tid) * (hd.pg + 1);
+                    const int ex = (nu + l0 - n) / 2 + ((m - mu) & 1);
+                    for (int ii = 0; ii <= imax; ++ii) {
+                        const int l = l0 + 2 * ii;
+                        if (abs(m - mu) > l) continue;
+                        acc += (((ex + ii) & 1) ? -gg[ii] : gg[ii]) * Z[IDX(l, m - mu) * 16 + o];
+                    }
                 }
             }
             const double sc = FOURPI * ipow(MODE == 0 ? hd.s[lv] : 1.0 / hd.s[lv], n);
@@ -3341,18 +3415,17 @@ static int h3_e2qbxl(qbx_ctx *ctx, hipStream_t st, const qbx_tree *T, const qbx_
     QBX_CHECK(G->trav == R, "M2QBXL / L2QBXL: geometry was built for another traversal");
     const TD td = make_td(T);
     const int Lm = hd.pmax + hd.pq, nqmax = (Lm + 1) * (Lm + 1);
-    const size_t mm_by = 32 * 3 * 2 * 64 + 16 * ((long)GC_GROUP * nqmax + GC_GROUP * (Lm + 3)) +
-                         8L * GC_GROUP * (Lm + 4);
     const unit_plan &U = G->gc_group_plan;
-    if (mode == 0 && hd.nr == 1 && hd.ncq <= 16 && U.nunits > 0 && mm_by <= 64 * 1024) {
-        // one density, p_q <= 3 (and the waves' tile within 96 KiB of LDS):
-        // the per-box matrices, then the products
+    if (mode == 0 && hd.nr == 1 && hd.ncq <= 16 && U.nunits > 0) {
+        // one density, p_q <= 3: the per-box matrices, then the products
         QBX_TRY(ws_reserve(ctx, st, ctx->ws_h3_m2qb, 2L * T->nboxes * nqmax * 16,
                            "M2QBXL box matrices"));
         hipLaunchKernelGGL(kh_m2qb_mat, dim3(T->nboxes), dim3(256), 0, st, hd, td, nqmax, expn,
                            ctx->ws_h3_m2qb.p);
-        const size_t by = mm_by;
-        hipLaunchKernelGGL(kh_m2qbxl_mm, dim3(U.nunits, ADJ_SHARES), dim3(256), by, st, hd, td,
+        const size_t by = sizeof(cplx) * GC_GROUP * nqmax;
+        auto kern = fabs(hd.k) * 1.75 * hd.h[0] <= QBX_SINCOS_MAX ? kh_m2qbxl_bm<true>
+                                                                  : kh_m2qbxl_bm<false>;
+        hipLaunchKernelGGL(kern, dim3(U.nunits, L3_SHARES), dim3(256), by, st, hd, td,
                            U.nunits, U.unit_box.p, U.unit_t0.p, G->gc_by_tbox_starts.p,
                            G->gc_by_tbox.p, R->l3_starts.p, R->l3_lists.p, G->centers.p,
                            G->ncenters, nqmax, ctx->ws_h3_m2qb.p, qexp);
@@ -3445,13 +3518,15 @@ static int adjoint_launch(hipStream_t st, const qbx_tree *T, const qbx_trav *R,
     case QBX_ADJ_M2QBXL:
         if (U.nunits > 0 && (stage == QBX_ADJ_L2QBXL || R->n3 > 0)) {
             const int th = std::min(448, 64 * ((ncl_max + 63) / 64));
-            const int ny = stage == QBX_ADJ_L2QBXL ? 1 : ADJ_SHARES;
+            const int ny = stage == QBX_ADJ_L2QBXL ? 1 : L3_SHARES;
             const int Lm = hd.pmax + hd.pq, nqmax = (Lm + 1) * (Lm + 1);
             const size_t zby = 16 * ((long)GC_GROUP * nqmax + 16L * nqmax + GC_GROUP * (Lm + 3)) +
                                8L * GC_GROUP * (Lm + 4);
             if (hd.ncq <= 16 && zby <= 96 * 1024) {
                 // the group's centers summed before the contraction
-                auto kz = stage == QBX_ADJ_L2QBXL ? kh_adj_e2qbxl_z<1> : kh_adj_e2qbxl_z<0>;
+                auto kz = stage == QBX_ADJ_L2QBXL ? kh_adj_e2qbxl_z<1, false>
+                          : core                  ? kh_adj_e2qbxl_z<0, true>
+                                                  : kh_adj_e2qbxl_z<0, false>;
                 hipLaunchKernelGGL(kz, dim3(U.nunits, ny), dim3(th), zby, st, hd, td, U.nunits,
                                    U.unit_box.p, U.unit_t0.p, R->target_boxes.p, R->l3_starts.p,
                                    R->l3_lists.p, G->gc_by_tbox_starts.p, G->gc_by_tbox.p,
