@@ -927,7 +927,7 @@ def run_ellipsoid3d(args):
                                   "dL_dsigma_dir_vs_central_diff": e_fd_v,
                                   "gpu_dense_matrix_4096_targets": dense},
         "roofline": {"bound": "valu", "compute": "fp64",
-                     "kernel": "k_h3_p2p_partial" if dom == "forward" else "k_h3_p2p_adjoint",
+                     "kernel": "k_h3_p2p<false>" if dom == "forward" else "k_h3_p2p<true>",
                      "achieved": round(achieved, 3), "peak": FP64_PEAK_TFLOPS,
                      "unit": "TFLOP/s", "frac": round(achieved / FP64_PEAK_TFLOPS, 4),
                      "frac_special40": round(achieved40 / FP64_PEAK_TFLOPS, 4),
