@@ -2332,7 +2332,9 @@ __global__ void __launch_bounds__(448) kh_adj_e2qbxl(HD hd, TD t, int nunits,
 // Lq'_c[o] in LDS, then a thread per box coefficient j: sum_o sum_ii
 // (-1)^ex G(j, o, ii) Z[(l, m - mu)][o] -- one contraction per group and box
 // instead of one per center.  Dynamic LDS: X [GC_GROUP][nqmax], Z [nqmax][16],
-// the radial sequences.
+// the radial sequences: 64 KB at order 10, two blocks a CU, so a block takes seven
+// wavefronts and splits the contraction's outputs o over up to four threads per j
+// (41024 centers: M2QBXL^T 2.4 ms with two wavefronts, 1.8 now; L2QBXL^T 0.62, 0.49).
 template <int MODE, bool CORE>
 __global__ void __launch_bounds__(448) kh_adj_e2qbxl_z(HD hd, TD t, int nunits,
                                                        const int *unit_box, const int *unit_c0,
@@ -2406,15 +2408,20 @@ __global__ void __launch_bounds__(448) kh_adj_e2qbxl_z(HD hd, TD t, int nunits,
             Z[w] = z;
         }
         __syncthreads();
-        if (tid < ncin) {
+        // slices of the outputs o side by side, their sums in X (consumed; it
+        // holds GC_GROUP nqmax >= GC_GROUP ncin)
+        const int pad = 64 * ((ncin + 63) / 64), nsl = min(GC_GROUP, (int)blockDim.x / pad);
+        const int sl = tid / pad, jt_ = tid % pad;
+        if (jt_ < ncin && sl < nsl) {
             int n, m;
-            nm_of(tid, n, m);
+            nm_of(jt_, n, m);
             cplx acc = {0.0, 0.0};
             for (int nu = 0, o = 0; nu <= pq; ++nu) {
                 const int imax = min(n, nu), l0 = abs(n - nu);
                 for (int mu = -nu; mu <= nu; ++mu, ++o) {
+                    if (o % nsl != sl) continue;
                     // G(j, o) = (-1)^(m - mu) G(o, j): consecutive lanes' rows
-                    const double *gg = hd.gaunt + ((long)o * ncg + tid) * (hd.pg + 1);
+                    const double *gg = hd.gaunt + ((long)o * ncg + jt_) * (hd.pg + 1);
                     const int ex = (nu + l0 - n) / 2 + ((m - mu) & 1);
                     for (int ii = 0; ii <= imax; ++ii) {
                         const int l = l0 + 2 * ii;
@@ -2423,6 +2430,14 @@ __global__ void __launch_bounds__(448) kh_adj_e2qbxl_z(HD hd, TD t, int nunits,
                     }
                 }
             }
+            X[sl * ncin + jt_] = acc;
+        }
+        __syncthreads();
+        if (tid < ncin) {
+            int n, m;
+            nm_of(tid, n, m);
+            cplx acc = X[tid];
+            for (int h = 1; h < nsl; ++h) acc += X[h * ncin + tid];
             const double sc = FOURPI * ipow(MODE == 0 ? hd.s[lv] : 1.0 / hd.s[lv], n);
             atomic_addc(xadj + ecoef_off(hd, D, lv) + 2L * tid, sc * acc);
         }
@@ -3527,7 +3542,7 @@ static int adjoint_launch(hipStream_t st, const qbx_tree *T, const qbx_trav *R,
                 auto kz = stage == QBX_ADJ_L2QBXL ? kh_adj_e2qbxl_z<1, false>
                           : core                  ? kh_adj_e2qbxl_z<0, true>
                                                   : kh_adj_e2qbxl_z<0, false>;
-                hipLaunchKernelGGL(kz, dim3(U.nunits, ny), dim3(th), zby, st, hd, td, U.nunits,
+                hipLaunchKernelGGL(kz, dim3(U.nunits, ny), dim3(448), zby, st, hd, td, U.nunits,
                                    U.unit_box.p, U.unit_t0.p, R->target_boxes.p, R->l3_starts.p,
                                    R->l3_lists.p, G->gc_by_tbox_starts.p, G->gc_by_tbox.p,
                                    G->centers.p, nc, nqmax, in, out);
