@@ -81,7 +81,7 @@ constexpr int M2P_UNIT_ITER = 8;   // M2P: list-3 boxes per lane
 constexpr int P2Q_UNIT_ITER = 32;  // P2QBXL: list-1 sources per lane
 constexpr int M2Q_UNIT_ITER = 2;   // M2QBXL: list-3 boxes per lane
 constexpr int GC_GROUP = 4;        // centers per block of the batched 3D P2QBXL
-constexpr int TSQ_ROWS = 64;       // QBX targets per block of the batched 3D TSQBX
+constexpr int TSQ_ROWS = 16;       // QBX targets per block of the batched 3D TSQBX
 int tsqbx_nrhs(qbx_ctx *ctx, void *stream, const qbx_tree *T, const qbx_trav *R,
                const qbx_geo *G, int kernel, int op, int qbx_order, int nrhs,
                const double *strengths_tree, const double *dipvec_tree, double scale,

@@ -351,22 +351,30 @@ __device__ __forceinline__ double tsq_laplace(const double *tc, double rt2, doub
 // The target-specific sum for many densities (3D Laplace S and D) on the
 // FP64 matrix cores: pot[t][r] (+)= sum_s G(t, s) q[s][r], G real, computed
 // once per (target, source) pair for all right-hand sides.  A block per unit
-// of tsq_plan: up to TSQ_ROWS = 64 QBX targets whose centers share target box
-// it, in row tiles of 16 (lane i evaluates G for row i % 16 and source
-// k0 + i / 16, exactly the A operand of v_mfma_f64_16x16x4f64), 32 right-hand
-// sides (blockIdx.y) as two column tiles.  The box's list-1 sources pass
-// through LDS TSQM_CH at a time without regard to box borders, the next
-// chunk's loads in flight while one is summed.  Each wave takes a row tile;
-// with two or one the waves split the sources and add in LDS.  Imaginary
-// parts of the strengths, where a chunk holds any, take a second pass.
+// of tsq_plan: up to TSQ_ROWS = 16 QBX targets whose centers share target box
+// it (lane i evaluates G for row i % 16 and source k + i / 16, exactly the A
+// operand of v_mfma_f64_16x16x4f64), 32 right-hand sides (blockIdx.y) as two
+// column tiles, their imaginary parts as two more that are left out of every
+// step in which they are zero.  The box's list-1 sources are taken four at a
+// time without regard to box borders, the steps dealt to the four waves; each
+// lane reads its source and strengths itself, the next step's while one is
+// summed, the sources' numbers from LDS (a tile of TSQM_CH of them found by
+// bisection while the tile before is summed: a barrier per 16 steps).  The
+// waves add in LDS.
 //
-// Bound by the strengths read from L2 (a unit reads its 5900 sources' 32
-// complex strengths; with 16 targets to a unit that was 58 GB) next to 35
-// vector instructions and two matrix products per 64 pairs.  307200 targets,
-// 32 densities, order 3: 15.0 -> 10.0 ms (10.4 without the units' order by
-// XCD; whole eighths of the list to an XCD, 20: the coarse boxes come first).
+// Bound by the chain of the longest lists where a surface has a few hundred
+// units (a coarse box's targets see most of the sources: 168158 in a list of
+// 76800 targets), else by 35 vector instructions and two matrix products per
+// 64 pairs next to the strengths from L2.  Staging chunks of 64 sources in LDS
+// for units of 64 targets read L2 a quarter as often, but waited for a chunk's
+// loads and two barriers every 64 sources and gave long lists a wave each:
+// 32 densities, order 3, 307200 targets 9.5 ms (now 7.6; whole eighths of the
+// units to an XCD instead of eight consecutive ones, 20: the coarse boxes come
+// first), with complex densities 19.2 (9.4); 7 densities, order 1, 76800
+// targets 16.1 (4.9) and 1200 targets 0.236 (0.072); 64 or 32 targets to a
+// unit here: 8.4, 7.7 ms; 14.3, 8.2; 0.217, 0.120.
 typedef double tsq_d4 __attribute__((ext_vector_type(4)));
-constexpr int TSQM_RB = 32, TSQM_CH = 64, TSQM_WS = 48;   // W row stride: banks
+constexpr int TSQM_RB = 32, TSQM_CH = 256;
 
 template <int OP, int P>
 __global__ void __launch_bounds__(256) k3_tsqbx_mr(int nunits, int nr, const int *ubox, const int *rows,
@@ -378,9 +386,9 @@ __global__ void __launch_bounds__(256) k3_tsqbx_mr(int nunits, int nr, const int
                                                    const double *q, const double *dip,
                                                    double scale, double *pot, int accumulate)
 {
-    __shared__ double sp[(OP == 1 ? 6 : 3) * TSQM_CH];
-    __shared__ double W[TSQM_CH * TSQM_WS];
-    __shared__ int pre[257], first[256], wsum[4], idx[2][TSQM_CH];
+    static_assert(TSQ_ROWS == 16, "a row tile of the matrix cores");
+    __shared__ double red[16 * 64];
+    __shared__ int pre[257], first[256], wsum[4], idx[3][TSQM_CH];
     // eight consecutive units, whose boxes share sources, on one XCD (blocks
     // go round the eight)
     const int bi = blockIdx.x;
@@ -391,13 +399,9 @@ __global__ void __launch_bounds__(256) k3_tsqbx_mr(int nunits, int nr, const int
     const int col = lane & 15, kr = lane >> 4;
     const int rb0 = blockIdx.y * TSQM_RB;
     const int nrb = min(TSQM_RB, nr - rb0);
-    // row tiles in use (rows are filled from the front), waves to a tile
-    int ntile = 1;
-    while (ntile < 4 && rows[TSQ_ROWS * u + 16 * ntile] >= 0) ++ntile;
-    const int KG = ntile == 1 ? 4 : ntile == 2 ? 2 : 1;
-    // the wave without a tile (three tiles) is another in each unit
-    const int tile = KG == 1 ? (wv + u) & 3 : wv / KG, kg = wv % KG;
-    const int ti = tile < ntile ? rows[TSQ_ROWS * u + 16 * tile + col] : -1;
+    const bool two = nrb > 16, in0 = col < nrb, in1 = 16 + col < nrb;
+    // this lane's A row: target ti about its center
+    const int ti = rows[TSQ_ROWS * u + col];
     double tc[3] = {0, 0, 0}, cc[3] = {0, 0, 0};
     if (ti >= 0) {
         const int c = tree_ttc[ti];
@@ -408,128 +412,118 @@ __global__ void __launch_bounds__(256) k3_tsqbx_mr(int nunits, int nr, const int
     }
     const double rt2 = tc[0] * tc[0] + tc[1] * tc[1] + tc[2] * tc[2];
     const int e1 = l1s[it + 1];
-    int imag = 0;
-    for (int pass = 0; pass < 2; ++pass) {
-        tsq_d4 acc[2] = {{0, 0, 0, 0}, {0, 0, 0, 0}};
-        for (int eb = l1s[it]; eb < e1; eb += 256) {
-            const int e = eb + tid;
-            int cnt = 0;
-            if (e < e1) {
-                cnt = scount[l1l[e]];
-                first[tid] = sstart[l1l[e]];
-            }
-            int run = cnt;
-            for (int o = 1; o < 64; o <<= 1) {
-                const int y = __shfl_up(run, o);
-                if (lane >= o) run += y;
-            }
-            if (lane == 63) wsum[wv] = run;
-            __syncthreads();
-            for (int w = 0; w < wv; ++w) run += wsum[w];
-            pre[tid + 1] = run;
-            if (tid == 0) pre[0] = 0;
-            __syncthreads();
-            const int total = pre[256];
-            if (total == 0) continue;
-            auto source = [&](int v) {
-                v = min(v, total - 1);
-                int lo = 0, hi = 256;
-                while (hi - lo > 1) {
-                    const int mid = (lo + hi) >> 1;
-                    if (pre[mid] <= v) lo = mid; else hi = mid;
-                }
-                return first[lo] + v - pre[lo];
-            };
-            double x[OP == 1 ? 2 : 1], wr[8];
-            auto fetch = [&](int v0, const int *ix) {
-                // coordinates (and normals): component tid / 64 of a source
-                const int si = ix[tid & 63], m = tid >> 6;
-                if (m < 3) {
-                    x[0] = src[(size_t)m * ns + si];
-                    if (OP == 1) x[OP == 1 ? 1 : 0] = dip[(size_t)m * ns + si];
-                }
-                const int n = total - v0;
+    tsq_d4 acc[4] = {{0, 0, 0, 0}, {0, 0, 0, 0}, {0, 0, 0, 0}, {0, 0, 0, 0}};
+    for (int eb = l1s[it]; eb < e1; eb += 256) {
+        const int e = eb + tid;
+        int run = 0;
+        __syncthreads();  // the former entries' counts and sources consumed
+        if (e < e1) {
+            run = scount[l1l[e]];
+            first[tid] = sstart[l1l[e]];
+        }
+        for (int o = 1; o < 64; o <<= 1) {
+            const int y = __shfl_up(run, o);
+            if (lane >= o) run += y;
+        }
+        if (lane == 63) wsum[wv] = run;
+        __syncthreads();
+        for (int w = 0; w < wv; ++w) run += wsum[w];
+        pre[tid + 1] = run;
+        if (tid == 0) pre[0] = 0;
+        __syncthreads();
+        const int total = pre[256];
+        if (total == 0) continue;
+        // source of the entries' place v (the last one again beyond the end)
+        auto source = [&](int v) {
+            v = min(v, total - 1);
+            int lo = 0;
 #pragma unroll
-                for (int w = 0; w < 8; ++w) {
-                    const int k = (tid >> 5) + 8 * w, r = tid & 31;
-                    wr[w] = 0.0;
-                    if (k < n && r < nrb) {
-                        const double *z = q + 2 * ((size_t)ix[k] * nr + rb0 + r);
-                        const double zr = z[0], zi = z[1];
-                        imag |= zi != 0.0;
-                        wr[w] = pass ? zi : zr;
-                    }
-                }
-            };
-            if (tid < TSQM_CH) {
-                idx[0][tid] = source(tid);
-                idx[1][tid] = source(TSQM_CH + tid);
+            for (int w = 128; w >= 1; w >>= 1)
+                if (pre[lo + w] <= v) lo += w;
+            return first[lo] + v - pre[lo];
+        };
+        struct Step {
+            double x[3], nu[3], w0[2], w1[2];
+        };
+        auto fetch = [&](Step &d, int si) {
+            for (int m = 0; m < 3; ++m) d.x[m] = src[(size_t)m * ns + si];
+            if (OP == 1)
+                for (int m = 0; m < 3; ++m) d.nu[m] = dip[(size_t)m * ns + si];
+            const double *z = q + 2 * ((size_t)si * nr + rb0 + col);
+            d.w0[0] = d.w0[1] = d.w1[0] = d.w1[1] = 0.0;
+            if (in0) {
+                d.w0[0] = z[0];
+                d.w0[1] = z[1];
             }
+            if (two && in1) {
+                d.w1[0] = z[32];
+                d.w1[1] = z[33];
+            }
+        };
+        auto sum = [&](const Step &d, bool on) {
+            double g = tsq_laplace<OP, P>(tc, rt2, d.x[0] - cc[0], d.x[1] - cc[1],
+                                          d.x[2] - cc[2], d.nu);
+            g = on ? g : 0.0;
+            const double r0 = on ? d.w0[0] : 0.0, i0 = on ? d.w0[1] : 0.0;
+            const double r1 = on ? d.w1[0] : 0.0, i1 = on ? d.w1[1] : 0.0;
+            acc[0] = __builtin_amdgcn_mfma_f64_16x16x4f64(g, r0, acc[0], 0, 0, 0);
+            if (two) acc[1] = __builtin_amdgcn_mfma_f64_16x16x4f64(g, r1, acc[1], 0, 0, 0);
+            if (__ballot(i0 != 0.0 || i1 != 0.0)) {
+                acc[2] = __builtin_amdgcn_mfma_f64_16x16x4f64(g, i0, acc[2], 0, 0, 0);
+                if (two) acc[3] = __builtin_amdgcn_mfma_f64_16x16x4f64(g, i1, acc[3], 0, 0, 0);
+            }
+        };
+        // tile t's numbers in idx[t % 3], written a tile ahead: the barrier of
+        // tile t + 1 keeps every wave within a tile of the others
+        idx[0][tid] = source(tid);
+        Step s0, s1;
+        for (int v0 = 0, buf = 0; v0 < total; v0 += TSQM_CH) {
+            const int nb = buf == 2 ? 0 : buf + 1;
+            idx[nb][tid] = source(v0 + TSQM_CH + tid);
             __syncthreads();
-            fetch(0, idx[0]);
-            for (int v0 = 0, buf = 1; v0 < total; v0 += TSQM_CH, buf ^= 1) {
-                const int m = tid >> 6;
-                if (m < 3) {
-                    sp[m * TSQM_CH + (tid & 63)] = x[0];
-                    if (OP == 1) sp[(3 + m) * TSQM_CH + (tid & 63)] = x[OP == 1 ? 1 : 0];
-                }
-#pragma unroll
-                for (int w = 0; w < 8; ++w)
-                    W[((tid >> 5) + 8 * w) * TSQM_WS + (tid & 31)] = wr[w];
-                __syncthreads();
-                if (v0 + TSQM_CH < total) fetch(v0 + TSQM_CH, idx[buf]);
-                const int nks = min(TSQM_CH, total - v0 + 3) / 4;
-                if (tile < ntile)
-                    for (int ks = kg; ks < nks; ks += KG) {
-                        const int k = 4 * ks + kr;
-                        double nu[3] = {0, 0, 0};
-                        if (OP == 1)
-                            for (int j = 0; j < 3; ++j) nu[j] = sp[(3 + j) * TSQM_CH + k];
-                        const double g = tsq_laplace<OP, P>(
-                            tc, rt2, sp[k] - cc[0], sp[TSQM_CH + k] - cc[1],
-                            sp[2 * TSQM_CH + k] - cc[2], nu);
-                        acc[0] = __builtin_amdgcn_mfma_f64_16x16x4f64(
-                            g, W[k * TSQM_WS + col], acc[0], 0, 0, 0);
-                        if (nrb > 16)
-                            acc[1] = __builtin_amdgcn_mfma_f64_16x16x4f64(
-                                g, W[k * TSQM_WS + 16 + col], acc[1], 0, 0, 0);
-                    }
-                if (tid < TSQM_CH) idx[buf ^ 1][tid] = source(v0 + 2 * TSQM_CH + tid);
-                __syncthreads();
+            // steps wv, wv + 4, ... of the tile's 64, in pairs; the last pair's
+            // second fetch is the next tile's first
+            const int nks = (min(TSQM_CH, total - v0) + 3) / 4;
+            if (v0 == 0) fetch(s0, idx[buf][4 * wv + kr]);
+            for (int ks = wv; ks < TSQM_CH / 4; ks += 8) {
+                fetch(s1, idx[buf][4 * (ks + 4) + kr]);
+                if (ks < nks) sum(s0, v0 + 4 * ks + kr < total);
+                if (ks + 4 >= nks) break;
+                const bool next = ks + 8 >= TSQM_CH / 4;
+                fetch(s0, next ? idx[nb][4 * wv + kr] : idx[buf][4 * (ks + 8) + kr]);
+                sum(s1, v0 + 4 * (ks + 4) + kr < total);
+            }
+            buf = nb;
+        }
+    }
+    for (int w = 1; w < 4; ++w) {
+        __syncthreads();
+        if (wv == w)
+            for (int h = 0; h < 4; ++h)
+                for (int j = 0; j < 4; ++j) red[(4 * h + j) * 64 + lane] = acc[h][j];
+        __syncthreads();
+        if (wv == 0)
+            for (int h = 0; h < 4; ++h)
+                for (int j = 0; j < 4; ++j) acc[h][j] += red[(4 * h + j) * 64 + lane];
+    }
+    if (wv > 0) return;
+    // D register j of lane i is row 4 j + i / 16, column i % 16
+    for (int j = 0; j < 4; ++j) {
+        const int tr = rows[TSQ_ROWS * u + 4 * j + kr];
+        if (tr < 0) continue;
+        for (int h = 0; h < 2; ++h) {
+            const int r = 16 * h + col;
+            if (r >= nrb) continue;
+            double *dst = pot + 2 * ((size_t)tr * nr + rb0 + r);
+            const double vr = scale * acc[h][j], vi = scale * acc[2 + h][j];
+            if (accumulate) {
+                dst[0] += vr;
+                dst[1] += vi;
+            } else {
+                dst[0] = vr;
+                dst[1] = vi;
             }
         }
-        // the waves of a tile added (in W), then stored: D register j of lane i
-        // is row 4 j + i / 16, column i % 16
-        for (int w = 1; w < KG; ++w) {
-            __syncthreads();
-            if (kg == w)
-                for (int h = 0; h < 2; ++h)
-                    for (int j = 0; j < 4; ++j) W[(tile * 8 + 4 * h + j) * 64 + lane] = acc[h][j];
-            __syncthreads();
-            if (kg == 0)
-                for (int h = 0; h < 2; ++h)
-                    for (int j = 0; j < 4; ++j) acc[h][j] += W[(tile * 8 + 4 * h + j) * 64 + lane];
-        }
-        if (tile < ntile && kg == 0)
-            for (int j = 0; j < 4; ++j) {
-                const int tr = rows[TSQ_ROWS * u + 16 * tile + 4 * j + kr];
-                if (tr < 0) continue;
-                for (int h = 0; h < 2; ++h) {
-                    const int r = 16 * h + col;
-                    if (r >= nrb) continue;
-                    double *dst = pot + 2 * ((size_t)tr * nr + rb0 + r);
-                    const double v = scale * acc[h][j];
-                    if (pass) {
-                        dst[1] += v;
-                    } else if (accumulate) {
-                        dst[0] += v;
-                    } else {
-                        dst[0] = v;
-                        dst[1] = 0.0;
-                    }
-                }
-            }
-        if (pass == 0 && !__syncthreads_or(imag)) break;
     }
 }
 

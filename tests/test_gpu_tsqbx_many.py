@@ -47,3 +47,49 @@ def test_many_densities_equal_one(pq, kind, nrhs, cplx, leaf):
         one = w1.eval_target_specific_qbx_locals(st[:, c].contiguous(), nrm) * (4 * np.pi)
         # the bound between forms of the same sum that the repository states
         assert float((many[:, c] - one).abs().max()) < 1e-12 * float(one.abs().max())
+
+
+@pytest.mark.parametrize("pq,kind,nrhs,cplx,leaf", [(1, "S", 16, True, 6), (3, "D", 17, True, 60),
+                                                    (3, "S", 33, False, 300),
+                                                    (5, "S", 4, True, 900)])
+def test_many_densities_match_the_oracle(oracle_lib, pq, kind, nrhs, cplx, leaf):
+    """The kernel's entry point, overwriting and adding, against the oracle's
+    sum: one to three columns of 16 real or imaginary parts, lists of more than
+    256 boxes (leaf 6) and of several tiles of 256 sources with a remainder."""
+    from pytential_amd import _lib
+    from pytential_amd import fmm as F
+    from pytential_amd.qbx import QBXLayerPotentialSource
+    from pytential_amd.surface import ellipsoid
+    d = ellipsoid(1, order=3, fine_order=5)
+    src = QBXLayerPotentialSource(d, fine_order=5, qbx_order=pq, fmm_order=3,
+                                  _max_leaf_refine_weight=leaf)
+    geo = src.qbx_fmm_geometry_data((("self", +1),))
+    tree, trav = geo.tree(), geo.traversal()
+    w = F.QBXExpansionWrangler(geo, "laplace", 0.0, kind, pq, [3] * tree.nlevels,
+                               use_target_specific_qbx=True, nrhs=nrhs)
+    rng = np.random.default_rng(pq)
+    ns = tree.nsources
+    st = rng.normal(size=(ns, nrhs)) + (1j * rng.normal(size=(ns, nrhs)) if cplx else 0j)
+    nrm = rng.normal(size=(3, ns)) if kind == "D" else None
+    print(f"pq={pq} {kind} nrhs={nrhs} complex={cplx} nsources={ns}", flush=True)
+
+    def dev(x):
+        return None if x is None else torch.as_tensor(np.ascontiguousarray(x), device="cuda")
+    dst, dnrm = dev(st), dev(nrm)
+    out = torch.zeros((tree.ntargets, nrhs), dtype=torch.complex128, device="cuda")
+    for accumulate in (0, 1):
+        w._a("qbx_eval_target_specific_qbx_locals_nrhs", tree.h, trav.h, w.geo.h, _lib.LAPLACE3D,
+             _lib.TSQBX_D if kind == "D" else _lib.TSQBX_S, pq, nrhs, F._p(dst), F._p(dnrm),
+             F._p(out), accumulate)
+    got = out.cpu().numpy() / 2
+    starts, lists = geo.center_to_tree_targets()
+    h = [x.cpu().numpy() for x in
+         (tree.sources, tree.targets, geo.flat_centers(), geo.global_qbx_centers(),
+          geo.qbx_center_to_target_box(), starts, lists, trav.neighbor_source_boxes_starts,
+          trav.neighbor_source_boxes_lists, tree.box_source_starts,
+          tree.box_source_counts_nonchild)]
+    for c in range(0, nrhs, 3):
+        ref = oracle_lib.tsqbx("laplace", kind, 0.0, pq, *h, st[:, c], nrm)
+        # the bound of test_gpu_tsqbx.py between forms of the same sum
+        assert np.max(np.abs(ref)) > 0
+        assert np.max(np.abs(got[:, c] - ref)) < 1e-12 * np.max(np.abs(ref))
