@@ -10,6 +10,8 @@ pytestmark = pytest.mark.gpu
 
 torch = pytest.importorskip("torch")
 
+K_ROUNDS = 7.99577
+
 
 @pytest.mark.parametrize("pq,kind,leaf", [(0, "S", 16), (1, "D", 6), (2, "S", 6), (3, "S", 6),
                                           (3, "D", 16), (4, "S", 16), (5, "S", 6), (5, "D", 16),
@@ -48,3 +50,98 @@ def test_qbx_expansions_match_oracle(oracle_lib, pq, kind, leaf):
                             d.strengths(dens[:, r]), return_stages=True)
         # the repository's bound for stages on the same tree
         assert np.max(np.abs(q[:, :, r] - stages["qbx"])) < 1e-12 * np.max(np.abs(stages["qbx"]))
+
+
+def _center_sums_80bit(pq, k, d, q, nu):
+    """i k sum q (nu . grad) h_n(k r) conj(Y_n^m) over sources at d (nu None:
+    the sum without the derivative), numpy longdouble, (re, im) per (n, m)."""
+    L = np.longdouble
+    r = np.sqrt((d * d).sum(0))
+    x, u = L(k) * r, d / r
+    sn, cs = np.sin(x), np.cos(x)
+    h = [(sn / x, -cs / x), (sn / x**2 - cs / x, -cs / x**2 - sn / x)]
+    for n in range(2, pq + 2):
+        h.append(tuple((2 * n - 1) / x * a - b for a, b in zip(h[-1], h[-2])))
+    un, du = 0 * r, 0 * d
+    if nu is not None:
+        un = (nu * u).sum(0)
+        du = (nu - un * u) / r
+    kun = L(k) * un
+    dh = [tuple(-kun * a for a in h[1])]
+    for n in range(1, pq + 1):
+        dh.append(tuple(kun * (a - (n + 1) / x * b) for a, b in zip(h[n - 1], h[n])))
+    out = np.zeros(((pq + 1) ** 2, 2), L)
+    w, dw = (1 + 0 * r, 0 * r), (0 * r, 0 * r)          # (x + i y)^m and its derivative
+    cmm = 1 / np.sqrt(4 * L("3.14159265358979323846264338327950288"))
+
+    def mul(a, b):
+        return a[0] * b[0] - a[1] * b[1], a[0] * b[1] + a[1] * b[0]
+    for m in range(pq + 1):
+        if m > 0:
+            a, b = mul(dw, u), mul(w, du)
+            dw = (a[0] + b[0], a[1] + b[1])
+            w = mul(w, u)
+            cmm = -cmm * np.sqrt(L(2 * m + 1) / (2 * m))
+        a1, a0, b1, b0, c = 0 * r, 1 + 0 * r, 0 * r, 0 * r, cmm
+        for n in range(m, pq + 1):
+            if n > m:
+                f = L((n - 1) ** 2 - m * m) / (4 * (n - 1) ** 2 - 1)
+                a1, a0, b1, b0 = a0, u[2] * a0 - f * a1, b0, u[2] * b0 + du[2] * a0 - f * b1
+                c = c * np.sqrt(L(4 * n * n - 1) / (n * n - m * m))
+            y = (c * a0 * w[0], c * a0 * w[1])
+            dy = (c * (b0 * w[0] + a0 * dw[0]), c * (b0 * w[1] + a0 * dw[1]))
+            for s in (1, -1) if m else (1,):
+                # conj(Y_n^m), and conj(Y_n^{-m}) = (-1)^m Y_n^m
+                g, t = (1, -1) if s > 0 else ((-1) ** m, 1)
+                v = mul(h[n], (g * y[0], g * t * y[1]))
+                if nu is not None:
+                    a, b = mul(dh[n], (g * y[0], g * t * y[1])), mul(h[n], (g * dy[0], g * t * dy[1]))
+                    v = (a[0] + b[0], a[1] + b[1])
+                v = mul(v, q)
+                out[n * n + n + s * m] = (-L(k) * v[1].sum(), L(k) * v[0].sum())
+    return out
+
+
+@pytest.mark.parametrize("kind", ["S", "D"])
+def test_p2qbxl_error_of_80_bit_sums(kind):
+    """Order 5 at a wavenumber whose reciprocal rounds by 1.1e-16, nearly the
+    most there is.  h_n carries the (n + 1)st power of 1 / x: with 1 / x as good
+    as its own rounding the six factors, the recurrences and the sums leave
+    below 1e-15 of a center's expansion (rms over centers); a 1 / x taken as
+    1 / r times the rounded 1 / k adds six times that rounding to every term,
+    6.6e-16 with one sign."""
+    from pytential_amd.qbx import QBXLayerPotentialSource
+    from pytential_amd.surface import ellipsoid
+    pq, k = 5, K_ROUNDS
+    d = ellipsoid(1, order=3, fine_order=5)
+    src = QBXLayerPotentialSource(d, fine_order=5, qbx_order=pq, fmm_order=2,
+                                  _max_leaf_refine_weight=16)
+    geo = src.qbx_fmm_geometry_data((("self", +1),))
+    w = src.make_wrangler(geo, "helmholtz", k, kind)
+    rng = np.random.default_rng(pq)
+    ns = w.tree.nsources
+    q = rng.normal(size=ns) + 1j * rng.normal(size=ns)
+    nu = rng.normal(size=(3, ns))
+    got = w.form_global_qbx_locals(torch.as_tensor(q, device="cuda"),
+                                   torch.as_tensor(nu, device="cuda") if kind == "D" else None)
+    got = got.cpu().numpy().reshape(geo.ncenters, -1)
+    tree, trav = geo.tree(), geo.traversal()
+    pts, cen, c2t, starts, lists, s0, cnt = (
+        t.cpu().numpy() for t in
+        (tree.sources, geo.flat_centers(), geo.qbx_center_to_target_box(),
+         trav.neighbor_source_boxes_starts, trav.neighbor_source_boxes_lists,
+         tree.box_source_starts, tree.box_source_counts_nonchild))
+    L = np.longdouble
+    err = []
+    for c in geo.global_qbx_centers().cpu().numpy()[::5]:
+        idx = np.concatenate([np.arange(s0[b], s0[b] + cnt[b])
+                              for b in lists[starts[c2t[c]]:starts[c2t[c] + 1]]])
+        ref = _center_sums_80bit(pq, k, pts[:, idx].astype(L) - cen[:, c, None].astype(L),
+                                 (q.real[idx].astype(L), q.imag[idx].astype(L)),
+                                 nu[:, idx].astype(L) if kind == "D" else None)
+        e = got[c]
+        err.append(float((((e.real - ref[:, 0]) ** 2 + (e.imag - ref[:, 1]) ** 2)).sum()
+                         / (ref ** 2).sum()))
+    rms = np.sqrt(np.mean(err))
+    print(f"{kind}: {len(err)} centers, rms relative error {rms:.2e}", flush=True)
+    assert rms < 1e-15
