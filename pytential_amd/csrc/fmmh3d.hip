@@ -509,72 +509,6 @@ __global__ void __launch_bounds__(512) kh_p2e(HD hd, TD t, int nitems, const int
     }
 }
 
-// S waves of one source about a center, in registers: F[IDX(n, m)] =
-// h_n(k r) Y_n^m(d) for n <= PF, d = s - c, r = |d| > 0.  h_n by the forward
-// recurrence (as radial_seq: stable for the dominant y_n, the small j_n of
-// x < n accurate to the rounding of |h_n|), Y by the column recurrences, all
-// unrolled.
-// CORE: k r is known to be within the reduced range of qbx_sincos (the device
-// library's sine for larger arguments, never reached, took 50 registers).
-template <int PF, bool CORE = false>
-__device__ __forceinline__ void s_waves_reg(double k, v3 d, cplx *F)
-{
-    const double r2 = d.x * d.x + d.y * d.y + d.z * d.z;
-    const double ir = qbx_rsqrt(r2);
-    const double r = r2 * ir;
-    const double x = k * r, ix = qbx_rcp(x);
-    double sn, cs;
-    if (CORE)
-        qbx_sincos_core(x, &sn, &cs);
-    else
-        qbx_sincos(x, &sn, &cs);
-    double yv[PF + 2], jv[PF + 2];
-    yv[0] = -cs * ix;
-    yv[1] = (-cs * ix - sn) * ix;
-    jv[0] = sn * ix;
-    jv[1] = (sn * ix - cs) * ix;
-#pragma unroll
-    for (int n = 2; n <= PF; ++n) {
-        yv[n] = (2.0 * n - 1.0) * ix * yv[n - 1] - yv[n - 2];
-        jv[n] = (2.0 * n - 1.0) * ix * jv[n - 1] - jv[n - 2];
-    }
-    const double scl = 1.0;
-    const double z = d.z * ir;
-    const cplx w = {d.x * ir, d.y * ir};
-    cplx wm = {1.0, 0.0};
-    double qmm = 0.28209479177387814347;
-#pragma unroll
-    for (int m = 0; m <= PF; ++m) {
-        if (m > 0) {
-            qmm *= -sqrt((2.0 * m + 1.0) / (2.0 * m));
-            wm = wm * w;
-        }
-        double a2 = 0.0, a1 = qmm;
-#pragma unroll
-        for (int n = m; n <= PF; ++n) {
-            double q;
-            if (n == m) {
-                q = qmm;
-            } else if (n == m + 1) {
-                q = sqrt(2.0 * m + 3.0) * z * qmm;
-            } else {
-                const double a = sqrt((4.0 * n * n - 1.0) / ((double)n * n - (double)m * m));
-                const double b = sqrt(((n - 1.0) * (n - 1.0) - (double)m * m) /
-                                      (4.0 * (n - 1.0) * (n - 1.0) - 1.0));
-                q = a * (z * a1 - b * a2);
-            }
-            if (n > m) {
-                a2 = a1;
-                a1 = q;
-            }
-            const cplx hn = {scl * jv[n], yv[n]};
-            const cplx y = q * wm;
-            F[IDX(n, m)] = hn * y;
-            if (m > 0) F[IDX(n, -m)] = hn * sgn_conj(y, m);
-        }
-    }
-}
-
 // 1 / x from y, 1 / x to a few ulp: one Newton step.  The n-th wave takes the
 // (n + 1)st power of 1 / x; from 1 / r times 1 / k as it stands the QBX
 // expansions of order 3 and 5 were 17 and 27% further from 80-bit sums.
@@ -607,14 +541,18 @@ struct SWaveSums {
             for (int j = 0; j < 4; ++j) t[i][j] = 0.0;
     }
 
-    __device__ __forceinline__ void add(double k, double ik, v3 d, cplx q)
+    // DIP: the derivative along nu of every term instead, both factors' by
+    // their own recurrences:
+    //   h_n' = h_{n-1} - (n + 1) / x h_n,  u' = (nu - (nu.u) u) / r
+    template <int DIP>
+    __device__ __forceinline__ void add(double k, double ik, v3 d, cplx q, v3 nu)
     {
         const double r2 = d.x * d.x + d.y * d.y + d.z * d.z;
         const double ir = qbx_rsqrt(r2);
         const double x = k * (r2 * ir), ix = rcp_near(x, ir * ik);
         double sn, cs;
         qbx_sincos_core(x, &sn, &cs);
-        cplx g[PQ + 2];
+        cplx g[PQ + 2], dg[PQ + 1];
         const cplx h0 = {sn * ix, -cs * ix};
         const cplx h1 = {(h0.x - cs) * ix, (h0.y - sn) * ix};
         g[0] = q * h0;
@@ -626,11 +564,27 @@ struct SWaveSums {
         }
         const double z = d.z * ir;
         const cplx w = {d.x * ir, d.y * ir};
-        cplx wm = w;
+        double dz = 0.0;
+        cplx dw = {0.0, 0.0};
+        if (DIP) {
+            const double un = nu.x * w.x + nu.y * w.y + nu.z * z, kun = k * un;
+            dz = (nu.z - un * z) * ir;
+            dw = {(nu.x - un * w.x) * ir, (nu.y - un * w.y) * ir};
+            dg[0] = {-kun * g[1].x, -kun * g[1].y};
+#pragma unroll
+            for (int n = 1; n <= PQ; ++n) {
+                const double f = (n + 1.0) * ix;
+                dg[n] = {kun * (g[n - 1].x - f * g[n].x), kun * (g[n - 1].y - f * g[n].y)};
+            }
+        }
+        cplx wm = w, dwm = dw;
 #pragma unroll
         for (int m = 0; m <= PQ; ++m) {
-            if (m > 1) wm = wm * w;
-            double a1 = 0.0, a0 = 1.0;
+            if (m > 1) {
+                if (DIP) dwm = (double)m * (wm * dw);
+                wm = wm * w;
+            }
+            double a1 = 0.0, a0 = 1.0, b1 = 0.0, b0 = 0.0;   // Q, Q'
 #pragma unroll
             for (int n = m; n <= PQ; ++n) {
                 if (n > m) {
@@ -638,11 +592,23 @@ struct SWaveSums {
                     const double c = ((n - 1.0) * (n - 1.0) - (double)m * m) /
                                      (4.0 * (n - 1.0) * (n - 1.0) - 1.0);
                     const double a = n == m + 1 ? z : z * a0 - c * a1;
+                    if (DIP) {
+                        const double b = n == m + 1 ? dz : z * b0 + dz * a0 - c * b1;
+                        b1 = b0;
+                        b0 = b;
+                    }
                     a1 = a0;
                     a0 = a;
                 }
                 if (m == 0) {
-                    if (n == 0) {
+                    if (DIP) {
+                        s0[n].x += dg[n].x * a0;
+                        s0[n].y += dg[n].y * a0;
+                        if (n > 0) {
+                            s0[n].x += g[n].x * b0;
+                            s0[n].y += g[n].y * b0;
+                        }
+                    } else if (n == 0) {
                         s0[0] += g[0];
                     } else {
                         s0[n].x += g[n].x * a0;
@@ -651,10 +617,19 @@ struct SWaveSums {
                 } else {
                     const cplx A = n == m ? wm : a0 * wm;
                     double *u = t[at(n, m)];
-                    u[0] += g[n].x * A.x;
-                    u[1] += g[n].y * A.y;
-                    u[2] += g[n].y * A.x;
-                    u[3] += g[n].x * A.y;
+                    const cplx f = DIP ? dg[n] : g[n];
+                    u[0] += f.x * A.x;
+                    u[1] += f.y * A.y;
+                    u[2] += f.y * A.x;
+                    u[3] += f.x * A.y;
+                    if (DIP) {
+                        const cplx B = n == m ? dwm : cplx{a0 * dwm.x + b0 * wm.x,
+                                                           a0 * dwm.y + b0 * wm.y};
+                        u[0] += g[n].x * B.x;
+                        u[1] += g[n].y * B.y;
+                        u[2] += g[n].y * B.x;
+                        u[3] += g[n].x * B.y;
+                    }
                 }
             }
         }
@@ -698,6 +673,10 @@ struct SWaveSums {
 // 3.  1.19e9 pairs (737280 sources, 163972 centers): 16.9 -> 6.6 ms.  With a
 // wave per center walking box by box, a box of 80 sources left lanes idle,
 // and 16 complex products of the waves took half of 560 instruction slots.
+// Double layer, order 3, 41024 and 1200 centers' box lists: 3.1 and 0.056 ms;
+// as complex waves to order 4 and gradients formed from them, one wavefront a
+// SIMD at orders 2 and 3 (now 3 and 2): 9.6 and 0.108, with a wave per center
+// walking box by box 20.4 and 0.138.
 constexpr int P2Q_CH = 256;
 
 // First sources and running source counts of the CH list entries from e0 (a
@@ -752,9 +731,7 @@ __global__ void __launch_bounds__(256) kh_p2qbxl_reg(HD hd, TD t, const int *ubo
                                                      const double *str, const double *nrm,
                                                      double *qexp)
 {
-    constexpr int PF = PQ + DIP;
     constexpr int NC = (PQ + 1) * (PQ + 1);
-    constexpr int NF = (PF + 1) * (PF + 1);
     __shared__ double2 sxy[P2Q_CH], szq[P2Q_CH];      // x, y; z, Re q
     __shared__ double sqi[P2Q_CH];
     __shared__ double snu[DIP ? 3 * P2Q_CH : 1];
@@ -772,13 +749,7 @@ __global__ void __launch_bounds__(256) kh_p2qbxl_reg(HD hd, TD t, const int *ubo
     const v3 c = act ? ld3(ctrs, nctr, ci) : v3{0, 0, 0};
     const double k = hd.k, ik = 1.0 / k;
     SWaveSums<PQ> A;
-    cplx acc[NC];
-    if (DIP) {
-#pragma unroll
-        for (int i = 0; i < NC; ++i) acc[i] = {0.0, 0.0};
-    } else {
-        A.zero();
-    }
+    A.zero();
     const int e1 = starts[it + 1];
     for (int e0 = starts[it]; e0 < e1; e0 += P2Q_CH) {
         list_counts<P2Q_CH>(t, e0, e1, lists, first, pre, wsum);
@@ -813,26 +784,15 @@ __global__ void __launch_bounds__(256) kh_p2qbxl_reg(HD hd, TD t, const int *ubo
                     const double2 xy = sxy[j], zq = szq[j];
                     const v3 d = {xy.x - c.x, xy.y - c.y, zq.x - c.z};
                     const cplx qs = {zq.y, sqi[j]};
-                    if (DIP) {
-                        cplx F[NF];
-                        s_waves_reg<PF, true>(k, d, F);
-                        const v3 nu = {snu[j], snu[P2Q_CH + j], snu[2 * P2Q_CH + j]};
-#pragma unroll
-                        for (int nn = 0; nn <= PQ; ++nn)
-#pragma unroll
-                            for (int m = -nn; m <= nn; ++m) {
-                                cplx fv = nu_grad(F, PF, k, nn, -m, nu);
-                                if (m & 1) fv = -fv;
-                                acc[IDX(nn, m)] += qs * fv;
-                            }
-                    } else {
-                        A.add(k, ik, d, qs);
-                    }
+                    const v3 nu = DIP ? v3{snu[j], snu[P2Q_CH + j], snu[2 * P2Q_CH + j]}
+                                      : v3{0, 0, 0};
+                    A.template add<DIP>(k, ik, d, qs, nu);
                 }
             __syncthreads();
         }
     }
-    if (!DIP) A.expansion(acc);
+    cplx acc[NC];
+    A.expansion(acc);
 #pragma unroll
     for (int i = 0; i < NC; ++i)
 #pragma unroll

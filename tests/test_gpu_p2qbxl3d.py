@@ -15,7 +15,8 @@ K_ROUNDS = 7.99577
 
 @pytest.mark.parametrize("pq,kind,leaf", [(0, "S", 16), (1, "D", 6), (2, "S", 6), (3, "S", 6),
                                           (3, "D", 16), (4, "S", 16), (5, "S", 6), (5, "D", 16),
-                                          (6, "S", 16)])
+                                          (6, "S", 16), (0, "D", 6), (2, "D", 16),
+                                          (4, "D", 6)])
 def test_qbx_expansions_match_oracle(oracle_lib, pq, kind, leaf):
     import oracle
 
