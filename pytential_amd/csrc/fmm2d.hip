@@ -141,13 +141,23 @@ __device__ __forceinline__ cplx ldpt(const double *x, int n, int i)
 // 64 entries, lane l reading entry l's first source and count, and sums the
 // counts; at(v) is source v of them all, its box found by bisection.  A wave
 // that walks box by box waits for each box's number, range and data in turn.
+// LEAN forms the lanes' addresses anew in each load(): hoisted out of the list
+// loop they stay in 8 to 12 registers through the caller's pair loop.
+__device__ __forceinline__ int lane_anew()
+{
+    int l = threadIdx.x;
+    asm volatile("" : "+v"(l));
+    return l;
+}
+
+template <bool LEAN = false>
 struct WaveSources {
     int *pre, *first;   // LDS, 65 and 64
     int total;
 
     __device__ __forceinline__ void load(const TD &t, const int *lists, int e, int e1)
     {
-        const int lane = threadIdx.x;
+        const int lane = LEAN ? lane_anew() : (int)threadIdx.x;
         int run = 0;
         __syncthreads();
         if (e + lane < e1) {
@@ -155,14 +165,16 @@ struct WaveSources {
             run = t.scount[Sb];
             first[lane] = t.sstart[Sb];
         }
+#pragma unroll
         for (int o = 1; o < 64; o <<= 1) {
-            const int y = __shfl_up(run, o);
+            const int y = LEAN ? __builtin_amdgcn_ds_bpermute((lane - o) << 2, run)
+                               : __shfl_up(run, o);
             if (lane >= o) run += y;
         }
         pre[lane + 1] = run;
         if (lane == 0) pre[0] = 0;
         __syncthreads();
-        total = pre[64];
+        total = LEAN ? __builtin_amdgcn_readfirstlane(pre[64]) : pre[64];
     }
 
     __device__ __forceinline__ int at(int v) const
@@ -520,7 +532,7 @@ __global__ void __launch_bounds__(64) k_p2e_lap(KD kd, TD t, const int *boxes, c
     cplx acc[NRC];
 #pragma unroll
     for (int q = 0; q < NRC; ++q) acc[q] = {0, 0};
-    WaveSources ws{pre, first, 0};
+    WaveSources<> ws{pre, first, 0};
     for (int e = e0; e < e1; e += 64) {
         if (LOCAL)
             ws.load(t, lists, e, e1);
@@ -1994,14 +2006,19 @@ __device__ void eval_mpole_add(const KD &kd, const double *a, int p, cplx c, dou
 // the unit's TG targets take G lanes apiece, the box's list-1 sources are
 // staged through LDS in chunks of CH (positions, normals, strengths, read
 // coalesced), each target's lanes split a chunk, and the G partial sums are
-// reduced by shuffles in a fixed order.
+// reduced by shuffles in a fixed order.  Four wavefronts a SIMD at least: with
+// eight densities that takes the lean staging (135 -> 123 registers, double
+// layer; 8 densities on 1500 panels and 40000 grid targets: the evaluation 1.22
+// -> 1.17 ms S, 1.28 -> 1.24 D).  With one density the chip is shared with the
+// level chain and the fifth wavefront costs that more than it gives here (4096
+// panels, 512^2: 0.640 -> 0.657 ms with it, P2P alone the same): not lean.
 template <int NRC>
 struct P2PTile {
     static constexpr int CH = NRC == 1 ? 128 : 64;
 };
 
 template <int NRC, bool DER, int KN, int DP>
-__global__ void __launch_bounds__(64) k_p2p(KD kd, TD t, const int *ubox, const int *ut0,
+__global__ void __launch_bounds__(64, 4) k_p2p(KD kd, TD t, const int *ubox, const int *ut0,
                                             const int *box_g, const int *tboxes,
                                             const int *starts, const int *lists,
                                             const int *fstart, const int *fcount,
@@ -2056,13 +2073,13 @@ __global__ void __launch_bounds__(64) k_p2p(KD kd, TD t, const int *ubox, const 
         __syncthreads();
     };
 
-    WaveSources ws{pre, first, 0};
+    WaveSources<(NRC > 1)> ws{pre, first, 0};
     const int e1 = starts[it + 1];
     for (int e = starts[it]; e < e1; e += 64) {
         ws.load(t, lists, e, e1);
         for (int v0 = 0; v0 < ws.total; v0 += CH) {
             const int n = min(CH, ws.total - v0);
-            for (int d = lane; d < n; d += 64) {
+            for (int d = NRC > 1 ? lane_anew() : lane; d < n; d += 64) {
                 const int si = ws.at(v0 + d);
                 sx[d] = src[si];
                 sy[d] = src[(size_t)ns + si];
@@ -2351,7 +2368,7 @@ __global__ void __launch_bounds__(64) k_p2qbxl(KD kd, TD t, const int *ubox, con
         __syncthreads();
     };
 
-    WaveSources ws{pre, first, 0};
+    WaveSources<> ws{pre, first, 0};
     const int e1 = l1s[it + 1];
     for (int e = l1s[it]; e < e1; e += 64) {
         ws.load(t, l1l, e, e1);
