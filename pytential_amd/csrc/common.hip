@@ -24,21 +24,6 @@ void set_error(const char *fmt, ...)
     va_end(ap);
 }
 
-int side_streams(int device, hipStream_t out[3])
-{
-    static std::mutex mu;
-    static std::map<int, std::array<hipStream_t, 3>> pool;
-    std::lock_guard<std::mutex> lock(mu);
-    auto it = pool.find(device);
-    if (it == pool.end()) {
-        std::array<hipStream_t, 3> s{};
-        for (hipStream_t &x : s) QBX_HIP(hipStreamCreateWithFlags(&x, hipStreamNonBlocking));
-        it = pool.emplace(device, s).first;
-    }
-    for (int i = 0; i < 3; ++i) out[i] = it->second[i];
-    return QBX_OK;
-}
-
 int note_capture(qbx_ctx *ctx, hipStream_t st)
 {
     hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;

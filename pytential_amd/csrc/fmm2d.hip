@@ -3679,7 +3679,8 @@ static int p2m_multistream(qbx_ctx *ctx, hipStream_t *sts, int nst, hipEvent_t *
     const TD td = make_td(T);
     QBX_TRY(zero_fill(mpole, (exp_bytes(kd)) / 8, sts[0]));
     QBX_HIP(hipEventRecord(evs[0], sts[0]));
-    for (int k = 1; k < nst; ++k) QBX_HIP(hipStreamWaitEvent(sts[k], evs[0], 0));
+    fork_join fj(sts[0], evs[0]);
+    for (int k = 1; k < nst; ++k) QBX_TRY(fj.fork(sts[k], evs[0]));
     // the busiest levels first, each to the stream with the least work so far
     // (boxes x coefficients): a small level queued behind a big one would
     // start only when the near field, issued meanwhile on the other streams,
@@ -3701,6 +3702,7 @@ static int p2m_multistream(qbx_ctx *ctx, hipStream_t *sts, int nst, hipEvent_t *
         QBX_HIP(hipEventRecord(evs[k], sts[k]));
         QBX_HIP(hipStreamWaitEvent(sts[0], evs[k], 0));
     }
+    fj.done();
     *done = true;
     return QBX_OK;
 }
@@ -4851,10 +4853,8 @@ static int drive_impl(qbx_ctx *ctx, void *stream, const qbx_tree *T, const qbx_t
         QBX_TRY(qbx_finalize_potentials(ctx, stream, T, G, nr, P, out_user));
         return QBX_OK;
     }
-    if (!ctx->side[0]) {
-        QBX_TRY(side_streams(ctx->device, ctx->side));
-        for (hipEvent_t &e : ctx->ev) QBX_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
-    }
+    if (!ctx->side[0]) QBX_TRY(side_streams(ctx->device, ctx->side));
+    QBX_TRY(ctx_events(ctx));
     // The stage DAG on four streams (the stage order of drive_fmm is kept
     // within each stream; every array has one writer stream at a time):
     //   main: zero P, M; P2M levels -(join)-> M2M -> M2L -[eM]-> (wait eP) L += L4
@@ -4890,11 +4890,11 @@ static int drive_impl(qbx_ctx *ctx, void *stream, const qbx_tree *T, const qbx_t
     // after the multistream P2M each side stream has already waited for the
     // zero fills and runs its near-field stage (which reads no multipole)
     // right after its own P2M levels; only M2M waits for the join
-    if (!done) {
-        QBX_HIP(hipEventRecord(e0, st));
-        QBX_HIP(hipStreamWaitEvent(s1, e0, 0));
-        QBX_HIP(hipStreamWaitEvent(s2, e0, 0));
-        QBX_HIP(hipStreamWaitEvent(s3, e0, 0));
+    fork_join fj(st, e0);
+    if (!done) QBX_HIP(hipEventRecord(e0, st));
+    for (hipStream_t x : {s1, s2, s3}) {
+        if (!done) QBX_HIP(hipStreamWaitEvent(x, e0, 0));
+        fj.s[fj.n++] = x;
     }
     QBX_TRY(qbx_eval_direct(ctx, s1, T, R, G, d, str, nrm, P, 1));
     if (tsq)
@@ -4926,6 +4926,7 @@ static int drive_impl(qbx_ctx *ctx, void *stream, const qbx_tree *T, const qbx_t
                            d->source_kind == QBX_SOURCE_D ? QBX_TSQBX_D : QBX_TSQBX_S,
                            d->qbx_order, nr, str, nrm, INV4PI_3D, P, 1));
     QBX_HIP(hipStreamWaitEvent(st, e1, 0));
+    fj.done();
     QBX_TRY(qbx_finalize_potentials(ctx, stream, T, G, nr, P, out_user));
     return QBX_OK;
 }

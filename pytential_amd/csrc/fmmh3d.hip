@@ -3670,6 +3670,8 @@ int h3_drive_fmm_adjoint(qbx_ctx *ctx, hipStream_t st, const qbx_tree *T, const 
     QBX_TRY(ws_reserve(ctx, st, ctx->ws_adj_p, np, "adjoint potential workspace"));
     double *Ma = ctx->ws_adj_m.p, *La = ctx->ws_adj_l.p, *Qa = ctx->ws_adj_q.p,
            *Pa = ctx->ws_adj_p.p;
+    // M2L^T's items, which synchronise and allocate, before anything is launched
+    if (R->n2 > 0) QBX_TRY(h3_m2l_groups(T, R, hd));
     QBX_TRY(zero_fill(Ma, nm, st));
     QBX_TRY(zero_fill(La, nm, st));
     QBX_TRY(zero_fill(Pa, np, st));

@@ -225,6 +225,32 @@ int scratch_reserve(qbx_ctx *ctx, hipStream_t st, size_t bytes, void **p);
 // with many contexts (one per captured operator) does not spread its
 // streams over the hardware queues the main stream uses
 int side_streams(int device, hipStream_t out[3]);
+// creates this context's fork/join events that are not there yet
+int ctx_events(qbx_ctx *ctx);
+// Streams forked off st.  What done() has not taken back by the end of the scope
+// is joined there, so that an error return leaves nothing running that a later
+// call on st, or a release of the caller's arrays, is not ordered after.
+struct fork_join {
+    hipStream_t st;
+    hipEvent_t ev;  // for those joins
+    hipStream_t s[3] = {nullptr, nullptr, nullptr};
+    int n = 0;
+    fork_join(hipStream_t st_, hipEvent_t ev_) : st(st_), ev(ev_) {}
+    fork_join(const fork_join &) = delete;
+    fork_join &operator=(const fork_join &) = delete;
+    ~fork_join()
+    {
+        for (int i = 0; i < n; ++i)
+            if (hipEventRecord(ev, s[i]) == hipSuccess) (void)hipStreamWaitEvent(st, ev, 0);
+    }
+    int fork(hipStream_t x, hipEvent_t e)
+    {
+        QBX_HIP(hipStreamWaitEvent(x, e, 0));
+        s[n++] = x;
+        return QBX_OK;
+    }
+    void done() { n = 0; }
+};
 // the device address of this device's allocation-free scratch array (looked
 // up once per device, with the device current)
 int noalloc_scratch_address(int device, double **out);
@@ -290,16 +316,15 @@ int adjoint_dag(qbx_ctx *ctx, hipStream_t st, Run run, const double *Pa, double 
     // The level-by-level translations leave most of the chip idle: in 2D the
     // stages one after another take 1.25 ms, the longest of these chains 0.55
     // (65536 sources, 327680 grid targets, k = 20).
-    if (!ctx->side[0]) {
-        QBX_TRY(side_streams(ctx->device, ctx->side));
-        for (hipEvent_t &e : ctx->ev) QBX_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
-    }
+    if (!ctx->side[0]) QBX_TRY(side_streams(ctx->device, ctx->side));
+    QBX_TRY(ctx_events(ctx));
     hipStream_t s1 = ctx->side[0], s2 = ctx->side[1];
     hipEvent_t e0 = ctx->ev[0], eQ = ctx->ev[1], eL = ctx->ev[2], e1 = ctx->ev[3],
                e2 = ctx->ev[4];
+    fork_join fj(st, e0);
     QBX_HIP(hipEventRecord(e0, st));
-    QBX_HIP(hipStreamWaitEvent(s1, e0, 0));
-    QBX_HIP(hipStreamWaitEvent(s2, e0, 0));
+    QBX_TRY(fj.fork(s1, e0));
+    QBX_TRY(fj.fork(s2, e0));
     QBX_TRY(run(st, QBX_ADJ_QBXL2P, Pa, Qa));
     QBX_HIP(hipEventRecord(eQ, st));
     QBX_TRY(run(s1, QBX_ADJ_M2P, Pa, Ma));
@@ -320,6 +345,7 @@ int adjoint_dag(qbx_ctx *ctx, hipStream_t st, Run run, const double *Pa, double 
     QBX_HIP(hipStreamWaitEvent(st, e1, 0));
     QBX_TRY(run(st, QBX_ADJ_M2M, Ma, nullptr));
     QBX_HIP(hipStreamWaitEvent(st, e2, 0));
+    fj.done();
     QBX_TRY(run(st, QBX_ADJ_P2M, Ma, str_adj));
     return QBX_OK;
 }

@@ -1,0 +1,129 @@
+// The adjoint driver's stage DAG and the side streams on a HIP of bookkeeping:
+// every launch keeps the set of launches that are ordered before it.  Built and
+// run by test_streams_host.py.
+#include "../pytential_amd/csrc/qbx_internal.h"
+
+#include <cstdarg>
+#include <cstdlib>
+#include <map>
+#include <set>
+
+using std::set;
+
+struct Launch {
+    hipStream_t s;
+    int stage;
+    set<int> before;
+};
+static std::vector<Launch> launches;
+static std::map<void *, set<int>> known;                    // stream or event
+static std::map<void *, unsigned long long> capture;        // stream -> capture id
+static std::map<void *, bool> made;
+static long handles = 1000;
+
+static hipStream_t stream() { return (hipStream_t)(handles += 8); }
+
+extern "C" {
+hipError_t hipStreamCreateWithFlags(hipStream_t *s, unsigned) { *s = stream(); return hipSuccess; }
+hipError_t hipEventCreateWithFlags(hipEvent_t *e, unsigned)
+{
+    *e = (hipEvent_t)(handles += 8);
+    return hipSuccess;
+}
+hipError_t hipEventRecord(hipEvent_t e, hipStream_t s) { known[e] = known[s]; return hipSuccess; }
+hipError_t hipStreamWaitEvent(hipStream_t s, hipEvent_t e, unsigned)
+{
+    known[s].insert(known[e].begin(), known[e].end());
+    return hipSuccess;
+}
+hipError_t hipStreamIsCapturing(hipStream_t s, hipStreamCaptureStatus *c)
+{
+    *c = capture.count(s) ? hipStreamCaptureStatusActive : hipStreamCaptureStatusNone;
+    return hipSuccess;
+}
+hipError_t hipStreamGetCaptureInfo(hipStream_t s, hipStreamCaptureStatus *c,
+                                   unsigned long long *id)
+{
+    *id = capture.count(s) ? capture[s] : 0;
+    return hipStreamIsCapturing(s, c);
+}
+hipError_t hipFree(void *) { return hipSuccess; }
+const char *hipGetErrorString(hipError_t) { return ""; }
+}
+
+namespace qbx {
+void set_error(const char *, ...) {}
+}
+using namespace qbx;
+
+#define REQUIRE(c)                                                          \
+    do {                                                                    \
+        if (!(c)) {                                                         \
+            printf("line %d: %s\n", __LINE__, #c);                          \
+            exit(1);                                                        \
+        }                                                                   \
+    } while (0)
+
+// arrays: 0 Pa 1 Qa 2 La 3 Ma 4 str_adj; r reads, a adds by atomics, w anything else
+struct Use {
+    int stage;
+    const char *how[5];
+};
+static const Use USES[] = {
+    {QBX_ADJ_QBXL2P, {"r", "w", "", "", ""}}, {QBX_ADJ_L2QBXL, {"", "r", "w", "", ""}},
+    {QBX_ADJ_L2P, {"r", "", "w", "", ""}},    {QBX_ADJ_L2L, {"", "", "w", "", ""}},
+    {QBX_ADJ_M2L, {"", "", "r", "a", ""}},    {QBX_ADJ_M2QBXL, {"", "r", "", "a", ""}},
+    {QBX_ADJ_M2P, {"r", "", "", "a", ""}},    {QBX_ADJ_P2L, {"", "", "r", "", "a"}},
+    {QBX_ADJ_P2QBXL, {"", "r", "", "", "a"}}, {QBX_ADJ_P2P, {"r", "", "", "", "a"}},
+    {QBX_ADJ_M2M, {"", "", "", "w", ""}},     {QBX_ADJ_P2M, {"", "", "", "r", "w"}},
+};
+
+static const Use &use_of(int stage)
+{
+    for (const Use &u : USES)
+        if (u.stage == stage) return u;
+    abort();
+}
+
+static int dag(qbx_ctx *ctx, hipStream_t st, int fail, set<hipStream_t> *used = nullptr)
+{
+    launches.clear();
+    known.clear();
+    return adjoint_dag(
+        ctx, st,
+        [&](hipStream_t s, int stage, const double *, double *) {
+            if (stage == fail) return (int)QBX_ERR_INVALID;
+            if (used) used->insert(s);
+            launches.push_back({s, stage, known[s]});
+            known[s].insert((int)launches.size() - 1);
+            return (int)QBX_OK;
+        },
+        nullptr, nullptr, nullptr, nullptr, nullptr);
+}
+
+int main()
+{
+    qbx_ctx ctx;
+    hipStream_t st = stream();
+    // every pair of stages that share an array is ordered, but for readers
+    // together and atomic additions together
+    for (int tune : {4, 1}) {
+        ctx.tune[QBX_TUNE_DRIVE_STREAMS] = tune;
+        REQUIRE(dag(&ctx, st, -1) == QBX_OK && launches.size() == 12);
+        for (size_t j = 0; j < launches.size(); ++j)
+            for (size_t i = 0; i < j; ++i)
+                for (int a = 0; a < 5; ++a) {
+                    const std::string x = use_of(launches[i].stage).how[a],
+                                      y = use_of(launches[j].stage).how[a];
+                    if (x.empty() || y.empty() || (x == y && x != "w")) continue;
+                    REQUIRE(launches[j].before.count((int)i));
+                }
+        // whatever stage fails, all that was launched is before what st does next
+        for (const Use &u : USES) {
+            REQUIRE(dag(&ctx, st, u.stage) == QBX_ERR_INVALID);
+            REQUIRE(known[st].size() == launches.size());
+        }
+    }
+    printf("ok\n");
+    return 0;
+}
