@@ -318,12 +318,14 @@ enum {
     QBX_TUNE_M2QBXL_UNIT_ITER = 3,  /* M2QBXL: list-3 boxes per lane (1..64) */
     QBX_TUNE_L2QBXL_LANES = 4,      /* 2D Helmholtz one-density L2QBXL: lanes per
                                        center (1, 2, 4, 8) */
-    QBX_TUNE_DRIVE_STREAMS = 5,     /* qbx_drive_fmm and qbx_drive_fmm_adjoint: 4 =
-                                       their stage DAG on the caller's stream and up to
-                                       three side streams (default); 1 = every
-                                       stage on the caller's stream, so that many contexts
-                                       can run side by side on streams of their own (one
-                                       graph holding several evaluations) */
+    QBX_TUNE_DRIVE_STREAMS = 5,     /* 4 (default) = qbx_drive_fmm's stage DAG on the
+                                       caller's stream and three side streams that all
+                                       contexts share, qbx_drive_fmm_adjoint's on the
+                                       caller's and two that are this call's (in a capture,
+                                       that capture's) alone; 1 = every stage on the
+                                       caller's stream, so that many contexts can run side
+                                       by side on streams of their own (one graph holding
+                                       several evaluations) */
     QBX_TUNE_COUNT = 6
 };
 int qbx_ctx_set_tuning(qbx_ctx *ctx, int param, int value);

@@ -124,6 +124,45 @@ int main()
             REQUIRE(known[st].size() == launches.size());
         }
     }
+    ctx.tune[QBX_TUNE_DRIVE_STREAMS] = 4;
+    // calls one after another, also after an error, take the same two streams
+    set<hipStream_t> a, b;
+    dag(&ctx, st, -1, &a);
+    dag(&ctx, st, -1, &b);
+    REQUIRE(a == b && a.size() == 3);
+    // a call while another has them takes others
+    side_pair *p = nullptr, *q = nullptr;
+    REQUIRE(side_pair_hold(0, st, &p) == QBX_OK && p && a.count(p->s[0]) && a.count(p->s[1]));
+    b.clear();
+    dag(&ctx, st, -1, &b);
+    REQUIRE(b.size() == 3 && !b.count(p->s[0]) && !b.count(p->s[1]));
+    side_pair_release(p);
+    // a capture keeps its pair until it ends: not for eager calls, nor for
+    // another capture, but for the same one
+    hipStream_t c1 = stream(), c2 = stream();
+    capture[c1] = 7;
+    capture[c2] = 8;
+    REQUIRE(side_pair_hold(0, c1, &p) == QBX_OK && p);
+    side_pair_release(p);
+    capture[p->s[0]] = capture[p->s[1]] = 7;
+    for (hipStream_t s : {st, c2}) {
+        REQUIRE(side_pair_hold(0, s, &q) == QBX_OK && q && q != p);
+        side_pair_release(q);
+    }
+    REQUIRE(side_pair_hold(0, c1, &q) == QBX_OK && q == p);
+    // the pool is bounded; with all pairs taken a call runs on its own stream
+    std::vector<side_pair *> held{q};
+    while (true) {
+        REQUIRE(side_pair_hold(0, st, &q) == QBX_OK);
+        if (!q) break;
+        held.push_back(q);
+    }
+    REQUIRE(held.size() == SIDE_PAIRS);
+    b.clear();
+    REQUIRE(dag(&ctx, st, -1, &b) == QBX_OK && b == set<hipStream_t>{st});
+    // another device has its own
+    REQUIRE(side_pair_hold(1, st, &q) == QBX_OK && q);
+    for (side_pair *x : held) REQUIRE(x != q);
     printf("ok\n");
     return 0;
 }

@@ -1,8 +1,9 @@
-"""CPU: the stage order of the adjoint driver (csrc/qbx_internal.h adjoint_dag,
-csrc/streams.hip), compiled by the host compiler against a HIP that only keeps
-book of what is ordered before what (streams_host.cpp): stages that share an
-array are ordered, and an error at any stage leaves nothing unordered with the
-caller's stream."""
+"""CPU: the stage order of the adjoint driver and its side streams
+(csrc/qbx_internal.h adjoint_dag, csrc/streams.hip), compiled by the host
+compiler against a HIP that only keeps book of what is ordered before what
+(streams_host.cpp): stages that share an array are ordered, an error at any
+stage leaves nothing unordered with the caller's stream, calls at the same time
+and captures do not share streams, and the pool of streams is bounded."""
 import os
 import shutil
 import subprocess
