@@ -830,8 +830,10 @@ __global__ void __launch_bounds__(256) kh_p2qbxl_reg(HD hd, TD t, const int *ubo
 //
 // FP64 VALU bound.  14.3e6 (box, source) pairs at order 10: 8.5 ms with waves
 // of 8 sources at a time in LDS, their radial sequences by 8 lanes and a thread
-// per coefficient; now 1.5
-// (1.65 with 8 roles at this order, for more wavefronts in flight).
+// per coefficient; now 1.0.  Two wavefronts a SIMD at every order: order 10, the
+// only one that has to spill for them (22 registers too many, 88 bytes), takes
+// 1.45 ms with one wavefront and none spilled (1.65 with 8 roles); on 1024 boxes'
+// lists 298 us (407 with one), on the shortest, 11520 sources, 91 (84).
 constexpr int P2L_PMAX = 12;
 constexpr int p2l_roles(int P) { return P <= 4 ? 1 : P <= 6 ? 2 : P <= 10 ? 4 : 8; }
 constexpr int p2l_threads(int P) { return 64 * (p2l_roles(P) > 4 ? p2l_roles(P) : 4); }
@@ -979,10 +981,9 @@ __device__ __forceinline__ double reduce_scatter64(double *v, int lane)
 }
 
 template <int P>
-__global__ void __launch_bounds__(p2l_threads(P), P == 10 ? 1 : 2) kh_p2l_reg(HD hd, TD t, const int *boxes,
-                                                  const int *starts, const int *lists,
-                                                  const double *src, int ns,
-                                                  const double *str, double *local)
+__global__ void __launch_bounds__(p2l_threads(P), 2)
+kh_p2l_reg(HD hd, TD t, const int *boxes, const int *starts, const int *lists, const double *src,
+           int ns, const double *str, double *local)
 {
     constexpr P2LCols<P> C{};
     constexpr int CH = p2l_threads(P);
