@@ -832,8 +832,8 @@ __global__ void __launch_bounds__(256) kh_p2qbxl_reg(HD hd, TD t, const int *ubo
 // of 8 sources at a time in LDS, their radial sequences by 8 lanes and a thread
 // per coefficient; now 1.0.  Two wavefronts a SIMD at every order: order 10, the
 // only one that has to spill for them (22 registers too many, 88 bytes), takes
-// 1.45 ms with one wavefront and none spilled (1.65 with 8 roles); on 1024 boxes'
-// lists 298 us (407 with one), on the shortest, 11520 sources, 91 (84).
+// 1.45 ms with one wavefront and none spilled (1.65 with 8 roles); 184320 sources
+// and 500 loose points 298 us (407 with one), 11520 sources 91 (84).
 constexpr int P2L_PMAX = 12;
 constexpr int p2l_roles(int P) { return P <= 4 ? 1 : P <= 6 ? 2 : P <= 10 ? 4 : 8; }
 constexpr int p2l_threads(int P) { return 64 * (p2l_roles(P) > 4 ? p2l_roles(P) : 4); }
