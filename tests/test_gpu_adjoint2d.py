@@ -103,6 +103,7 @@ def test_transposed_stages_dot_identity(kernel, k, kind):
         lhs = _dot(ya, y).real
         rhs = _dot(xa, x).real
         scale = float(torch.linalg.norm(ya) * torch.linalg.norm(y)) + 1e-300
+        assert float(torch.linalg.norm(y)) > 0, stage
         err = abs(lhs - rhs) / scale
         print(f"[adjoint] {kernel}-{kind} {stage}: Re<y',Ax> {lhs:+.6e} Re<A^H y',x> "
               f"{rhs:+.6e} rel {err:.1e}", flush=True)

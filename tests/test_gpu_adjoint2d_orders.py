@@ -59,6 +59,7 @@ def test_stages_at_order(order, kind):
         y = f(x).reshape(-1)
         xa = F.adjoint_stage(w, stage, ya.clone(), normals=nrm).reshape(-1)
         scale = float(torch.linalg.norm(ya) * torch.linalg.norm(y)) + 1e-300
+        assert float(torch.linalg.norm(y)) > 0, stage
         err = abs(_dot(ya, y).real - _dot(xa, x).real) / scale
         print(f"[adjoint] order {order} {kind} {stage}: {err:.1e}", flush=True)
         assert err < 1e-12, (stage, err)
