@@ -15,10 +15,13 @@ __global__ void __launch_bounds__(256) k_ceil_mfma(int iters, double *out)
     ceil_d4 acc[8];
     for (int i = 0; i < 8; ++i) acc[i] = ceil_d4{0, 0, 0, 0};
     const double a = 1.0 + threadIdx.x * 1e-9, b = 1.0 - threadIdx.x * 1e-9;
-    for (int it = 0; it < iters; ++it) {
+    // 32 rounds an iteration: the compiler keeps the accumulators in VGPRs across
+    // the loop's edge and moves all 64 to AGPRs and back each time (with one
+    // round an iteration the probe read 46.9 TFLOP/s, with 32 71.5)
+    for (int it = 0; it < iters; it += 32) {
 #pragma unroll
-        for (int i = 0; i < 8; ++i)
-            acc[i] = __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, acc[i], 0, 0, 0);
+        for (int i = 0; i < 8 * 32; ++i)
+            acc[i % 8] = __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, acc[i % 8], 0, 0, 0);
     }
     double s = 0;
     for (int i = 0; i < 8; ++i) s += acc[i][0] + acc[i][1] + acc[i][2] + acc[i][3];
@@ -56,8 +59,8 @@ int main()
     CK(hipEventCreate(&e0));
     CK(hipEventCreate(&e1));
     float ms_mfma = 0.f, ms_fma = 0.f;
-    const int it_mfma = 2000, it_fma = 20000;
-    hipLaunchKernelGGL(k_ceil_mfma, dim3(blocks), dim3(256), 0, 0, 10, out);
+    const int it_mfma = 2048, it_fma = 20000;
+    hipLaunchKernelGGL(k_ceil_mfma, dim3(blocks), dim3(256), 0, 0, 32, out);
     CK(hipEventRecord(e0, 0));
     hipLaunchKernelGGL(k_ceil_mfma, dim3(blocks), dim3(256), 0, 0, it_mfma, out);
     CK(hipEventRecord(e1, 0));
