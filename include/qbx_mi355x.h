@@ -321,8 +321,8 @@ enum {
     QBX_TUNE_DRIVE_STREAMS = 5,     /* 4 (default) = qbx_drive_fmm's stage DAG on the
                                        caller's stream and three side streams that all
                                        contexts share, qbx_drive_fmm_adjoint's on the
-                                       caller's and two that are this call's (in a capture,
-                                       that capture's) alone; 1 = every stage on the
+                                       caller's and two that no other adjoint or capture
+                                       has meanwhile; 1 = every stage on the
                                        caller's stream, so that many contexts can run side
                                        by side on streams of their own (one graph holding
                                        several evaluations) */

@@ -4855,6 +4855,8 @@ static int drive_impl(qbx_ctx *ctx, void *stream, const qbx_tree *T, const qbx_t
     }
     if (!ctx->side[0]) QBX_TRY(side_streams(ctx->device, ctx->side));
     QBX_TRY(ctx_events(ctx));
+    side_holder hold;
+    QBX_TRY(side_streams_capture(ctx->device, st, &hold.p));
     // The stage DAG on four streams (the stage order of drive_fmm is kept
     // within each stream; every array has one writer stream at a time):
     //   main: zero P, M; P2M levels -(join)-> M2M -> M2L -[eM]-> (wait eP) L += L4

@@ -227,19 +227,30 @@ int scratch_reserve(qbx_ctx *ctx, hipStream_t st, size_t bytes, void **p);
 int side_streams(int device, hipStream_t out[3]);
 // creates this context's fork/join events that are not there yet
 int ctx_events(qbx_ctx *ctx);
-// Two side streams for one adjoint call.  A pair is one call's at a time, and
-// one capture's until that capture ends (streams forked into it belong to it),
-// so that adjoints captured side by side, or run while another thread captures,
-// never meet: on the streams of side_streams, which every forward shares, they
-// would.  At most SIDE_PAIRS to a device, kept until the process ends; with
-// all of them taken *out is null and the call runs on its own stream.
+// Two side streams for one adjoint call, so that adjoints captured side by side,
+// or run while another thread captures, never meet.  An eager call has two of
+// side_streams unless another adjoint or a capture has them (more streams would
+// share the process's four hardware queues with the caller's: the adjoint of
+// 65536 sources 1.84 -> 1.98 ms with an unlucky one), else, and always in a
+// capture, a pair of its own: one call's at a time, and one capture's until
+// that capture ends (streams forked into it belong to it).  At most SIDE_PAIRS
+// such pairs to a device, kept until the process ends; with all of them taken
+// *out is null and the call runs on its own stream.
 constexpr int SIDE_PAIRS = 4;
 struct side_pair {
     hipStream_t s[2] = {nullptr, nullptr};
     bool held = false;
 };
 int side_pair_hold(int device, hipStream_t st, side_pair **out);
+// for a forward, which forks side_streams into st's capture if there is one: an
+// adjoint that another thread is launching on them comes to its end first, and
+// none begins until release.  *out null: no capture.
+int side_streams_capture(int device, hipStream_t st, side_pair **out);
 void side_pair_release(side_pair *p);
+struct side_holder {
+    side_pair *p = nullptr;
+    ~side_holder() { side_pair_release(p); }
+};
 // Streams forked off st.  What done() has not taken back by the end of the scope
 // is joined there, so that an error return leaves nothing running that a later
 // call on st, or a release of the caller's arrays, is not ordered after.
@@ -301,10 +312,10 @@ template <typename Run>
 int adjoint_dag(qbx_ctx *ctx, hipStream_t st, Run run, const double *Pa, double *Qa, double *La,
                 double *Ma, double *str_adj)
 {
-    side_pair *pair = nullptr;
+    side_holder hold;
     if (ctx->tune[QBX_TUNE_DRIVE_STREAMS] > 1)
-        QBX_TRY(side_pair_hold(ctx->device, st, &pair));
-    if (!pair) {
+        QBX_TRY(side_pair_hold(ctx->device, st, &hold.p));
+    if (!hold.p) {
         QBX_TRY(run(st, QBX_ADJ_QBXL2P, Pa, Qa));
         QBX_TRY(run(st, QBX_ADJ_L2QBXL, Qa, La));
         QBX_TRY(run(st, QBX_ADJ_L2P, Pa, La));
@@ -332,12 +343,8 @@ int adjoint_dag(qbx_ctx *ctx, hipStream_t st, Run run, const double *Pa, double 
     // The level-by-level translations leave most of the chip idle: in 2D the
     // stages one after another take 1.25 ms, the longest of these chains 0.55
     // (65536 sources, 327680 grid targets, k = 20).
-    struct holder {
-        side_pair *p;
-        ~holder() { side_pair_release(p); }
-    } hold{pair};
     QBX_TRY(ctx_events(ctx));
-    hipStream_t s1 = pair->s[0], s2 = pair->s[1];
+    hipStream_t s1 = hold.p->s[0], s2 = hold.p->s[1];
     hipEvent_t e0 = ctx->ev[0], eQ = ctx->ev[1], eL = ctx->ev[2], e1 = ctx->ev[3],
                e2 = ctx->ev[4];
     fork_join fj(st, e0);

@@ -3,10 +3,13 @@
 // run by test_streams_host.py.
 #include "../pytential_amd/csrc/qbx_internal.h"
 
+#include <atomic>
+#include <chrono>
 #include <cstdarg>
 #include <cstdlib>
 #include <map>
 #include <set>
+#include <thread>
 
 using std::set;
 
@@ -125,39 +128,70 @@ int main()
         }
     }
     ctx.tune[QBX_TUNE_DRIVE_STREAMS] = 4;
-    // calls one after another, also after an error, take the same two streams
+    // calls one after another, also after an error, take the same two streams,
+    // those of the forward
+    hipStream_t fwd[3];
+    REQUIRE(side_streams(0, fwd) == QBX_OK);
     set<hipStream_t> a, b;
     dag(&ctx, st, -1, &a);
     dag(&ctx, st, -1, &b);
-    REQUIRE(a == b && a.size() == 3);
+    REQUIRE(a == b && (a == set<hipStream_t>{st, fwd[0], fwd[1]}));
+    auto apart = [](const side_pair *x, const hipStream_t *y) {
+        for (int i = 0; i < 3; ++i)
+            if (x->s[0] == y[i] || x->s[1] == y[i]) return false;
+        return true;
+    };
     // a call while another has them takes others
     side_pair *p = nullptr, *q = nullptr;
-    REQUIRE(side_pair_hold(0, st, &p) == QBX_OK && p && a.count(p->s[0]) && a.count(p->s[1]));
+    REQUIRE(side_pair_hold(0, st, &p) == QBX_OK && p && p->s[0] == fwd[0]);
     b.clear();
     dag(&ctx, st, -1, &b);
     REQUIRE(b.size() == 3 && !b.count(p->s[0]) && !b.count(p->s[1]));
-    side_pair_release(p);
-    // a capture keeps its pair until it ends: not for eager calls, nor for
-    // another capture, but for the same one
+    // a forward's capture waits for the one that has them
     hipStream_t c1 = stream(), c2 = stream();
     capture[c1] = 7;
     capture[c2] = 8;
-    REQUIRE(side_pair_hold(0, c1, &p) == QBX_OK && p);
+    std::atomic<bool> in{false};
+    std::thread th([&] {
+        side_pair *f = nullptr;
+        REQUIRE(side_streams_capture(0, c1, &f) == QBX_OK && f == p);
+        in = true;
+    });
+    std::this_thread::sleep_for(std::chrono::milliseconds(50));
+    REQUIRE(!in);
+    side_pair_release(p);
+    th.join();
+    // and no adjoint begins on them until it is through, nor, forked into its
+    // capture, until that ends
+    for (int forked = 0; forked < 2; ++forked) {
+        REQUIRE(side_pair_hold(0, st, &q) == QBX_OK && q && apart(q, fwd));
+        side_pair_release(q);
+        if (forked) break;
+        capture[fwd[0]] = capture[fwd[1]] = capture[fwd[2]] = 7;
+        side_pair_release(p);
+    }
+    for (hipStream_t x : fwd) capture.erase(x);
+    REQUIRE(side_streams_capture(0, st, &q) == QBX_OK && !q);
+    // an adjoint in a capture has its own pair, and keeps it until the capture
+    // ends: not for eager calls, nor for another capture, but for the same one
+    REQUIRE(side_pair_hold(0, c1, &p) == QBX_OK && p && apart(p, fwd));
     side_pair_release(p);
     capture[p->s[0]] = capture[p->s[1]] = 7;
-    for (hipStream_t s : {st, c2}) {
-        REQUIRE(side_pair_hold(0, s, &q) == QBX_OK && q && q != p);
-        side_pair_release(q);
-    }
+    REQUIRE(side_pair_hold(0, c2, &q) == QBX_OK && q && q != p && apart(q, fwd));
+    side_pair_release(q);
+    side_pair *first = nullptr;
+    REQUIRE(side_pair_hold(0, st, &first) == QBX_OK && first->s[0] == fwd[0]);
+    REQUIRE(side_pair_hold(0, st, &q) == QBX_OK && q && q != p);
+    side_pair_release(q);
     REQUIRE(side_pair_hold(0, c1, &q) == QBX_OK && q == p);
     // the pool is bounded; with all pairs taken a call runs on its own stream
-    std::vector<side_pair *> held{q};
+    std::vector<side_pair *> held{first, q};
     while (true) {
         REQUIRE(side_pair_hold(0, st, &q) == QBX_OK);
         if (!q) break;
         held.push_back(q);
     }
-    REQUIRE(held.size() == SIDE_PAIRS);
+    REQUIRE(held.size() == 1 + SIDE_PAIRS);
     b.clear();
     REQUIRE(dag(&ctx, st, -1, &b) == QBX_OK && b == set<hipStream_t>{st});
     // another device has its own

@@ -19,7 +19,7 @@ ROCM = os.environ.get("ROCM_PATH", "/opt/rocm")
                     reason="needs g++ and the HIP headers")
 def test_adjoint_stages_and_side_streams(tmp_path):
     exe = str(tmp_path / "streams_host")
-    subprocess.run(["g++", "-std=c++17", "-O1", "-D__HIP_PLATFORM_AMD__", "-I" + ROCM + "/include",
+    subprocess.run(["g++", "-std=c++17", "-O1", "-pthread", "-D__HIP_PLATFORM_AMD__", "-I" + ROCM + "/include",
                     "-x", "c++", os.path.join(HERE, "streams_host.cpp"),
                     os.path.join(CSRC, "streams.hip"), "-o", exe], check=True)
     r = subprocess.run([exe], capture_output=True, text=True, timeout=60)
