@@ -2,11 +2,8 @@
 // small elementwise kernels at the boundary (source reorder, upsampling).
 #include <hipcub/hipcub.hpp>
 
-#include <array>
 #include <cstdarg>
 #include <cstring>
-#include <map>
-#include <mutex>
 
 #include "qbx_internal.h"
 
